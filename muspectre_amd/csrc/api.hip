@@ -952,7 +952,7 @@ extern "C" int mugpu_cell_create(int dim, const int* res, const double* lengths,
   c->prec = precision;
   c->allow_even = allow_even;
   c->nc = dim * dim;
-  int rc = plan_init(c->plan, dim, res, c->nc, MUGPU_FP64);
+  int rc = plan_init(c->plan, dim, res, c->nc, MUGPU_FP64, precision == MUGPU_FP64);
   if (rc) {
     plan_free(c->plan);
     delete c;

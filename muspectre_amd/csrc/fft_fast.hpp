@@ -153,18 +153,6 @@ __device__ __forceinline__ c_t<T> czero() {
   return z;
 }
 
-// Workgroups are dispatched to the 8 XCDs round robin (workgroup b runs on
-// XCD b mod 8), each XCD with its own L2.  Tiles next to each other in HBM
-// share cache lines at their edges, so the tile of workgroup b is chosen to
-// give every XCD one contiguous range of tiles: neighbours then meet in the
-// same L2.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t total) {
-  const int64_t q = total / kXcds, r = total - q * kXcds;
-  const int64_t x = b % kXcds, local = b / kXcds;
-  return x * q + (x < r ? x : r) + local;
-}
-
 // ---- shapes of the workgroups -----------------------------------------------
 // last-axis passes: rows per workgroup (even: two rows share a complex
 // line); 288 threads in 3D, 256 in 2D; h = 1: half the rows (half the LDS,

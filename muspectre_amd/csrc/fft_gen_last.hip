@@ -1,0 +1,303 @@
+// Last-axis passes of FP64 grids whose last axis has a run-time length: r2c
+// with the CG direction update and K : p in front, c2r with the p . Ap partial
+// sums behind.
+//
+// Two rows share a complex line (row 2q in the real part, 2q + 1 in the
+// imaginary part), separated after the forward transform and combined before
+// the backward one by Hermitian symmetry, as in fft_fast.hpp.  Rows are
+// contiguous in HBM: every global access is an element-wise sweep of a row by
+// consecutive lanes.
+#include "fft_gen.hpp"
+
+namespace mugpu {
+
+namespace {
+
+struct GLast {
+  const double* in;
+  const double* rvec;
+  double* pout;
+  const double* scal;
+  const double* tan;
+  int tan_kind;
+  double2* spec;
+  double* out;
+  const double* dotv;
+  double* partials;
+  int64_t rows;
+  int RB, L, P, LS;  // rows and lines per workgroup, threads per line, LDS line stride
+  GenAxis ax;
+  const double2* tw;
+  const int* active;  // FftPlan::active
+};
+
+// LDS: [lines: n * LS complex][twiddles: n complex][staging: 2 rows of NC
+// values per point].  The updated p of two rows is staged as it lies in memory
+// and read back a voxel per thread (a lane stride of NC doubles, odd in 3D: no
+// bank conflict), so that r, p are read and p is written in full cache lines.
+template <int CLS, int DIM, int IN>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
+  if (a.active && !a.active[0]) return;
+  constexpr int NC = DIM * DIM;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x;
+  double2* s = reinterpret_cast<double2*>(smem);
+  double* sr = reinterpret_cast<double*>(smem);
+  double2* tw = s + n * LS;
+  double* sp = reinterpret_cast<double*>(tw + n);
+  gen_twiddles<double>(tw, a.tw, n);
+  const int64_t row0 = (int64_t)blockIdx.x * a.RB;
+  const double beta = IN == IN_TAN_PUPDATE ? a.scal[SC_BETA] : 0.0;
+  for (int r0 = 0; r0 < a.RB; r0 += 2) {
+    const int64_t base = (row0 + r0) * n * NC, lim = a.rows * n * NC;
+    const int tot = 2 * n * NC;
+    constexpr int KB = 4;
+    if (r0) __syncthreads();  // the staged rows before have been read
+    for (int e0 = 0; e0 < tot; e0 += KB * NT) {
+      double pv[KB], rv[KB];
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        const int64_t g = e < tot && base + e < lim ? base + e : lim - 1;
+        pv[i] = a.in[g];
+        if (IN == IN_TAN_PUPDATE) rv[i] = a.rvec[g];
+      }
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        if (e < tot) {
+          double x = 0.0;
+          if (base + e < lim) {
+            x = pv[i];
+            if (IN == IN_TAN_PUPDATE) {
+              x = -rv[i] + beta * x;
+              a.pout[base + e] = x;
+            }
+          }
+          sp[e] = x;
+        }
+      }
+    }
+    __syncthreads();
+    // rows beyond the last one hold zeros, for which K : p is not evaluated
+    auto voxels = [&](auto kind_c) {
+      constexpr int KIND = decltype(kind_c)::value;
+      for (int e = threadIdx.x; e < 2 * n; e += NT) {
+        const int r = e >= n, m = e - r * n;
+        double p[NC], dp[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) p[c] = sp[e * NC + c];
+        if (KIND >= 0 && row0 + r0 + r < a.rows) {
+          tangent_product<double, DIM>(KIND, a.tan, (row0 + r0 + r) * n + m, p, dp);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) dp[c] = p[c];
+        }
+        double* o = sr + 2 * (m * LS + (r0 >> 1) * NC) + r;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) o[2 * c] = dp[c];
+      }
+    };
+    if constexpr (IN == IN_PLAIN) {
+      voxels(std::integral_constant<int, -1>{});
+    } else {
+      switch (a.tan_kind) {
+        case TAN_SYM: voxels(std::integral_constant<int, TAN_SYM>{}); break;
+        case TAN_HEP: voxels(std::integral_constant<int, TAN_HEP>{}); break;
+        case TAN_ISO: voxels(std::integral_constant<int, TAN_ISO>{}); break;
+        default: voxels(std::integral_constant<int, TAN_FULL>{}); break;
+      }
+    }
+  }
+  __syncthreads();
+  const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
+  auto none_ld = [](int) { return double2{}; };
+  auto none_st = [](int, double2) {};
+  gen_fft<double, CLS, -1, false, false>(a.ax, a.P, p, p < a.P, s + l, LS, tw, none_ld, none_st);
+  for (int r = 0; r < a.RB; ++r) {
+    if (row0 + r >= a.rows) break;
+    double2* o = a.spec + (row0 + r) * nh * NC;
+    const double2* sl = s + (r >> 1) * NC;
+    for (int e = threadIdx.x; e < nh * NC; e += NT) {
+      const int k = e / NC, c = e - k * NC;
+      const double2 z = sl[k * LS + c], zc = sl[(k == 0 ? 0 : n - k) * LS + c];
+      double2 X;
+      if (!(r & 1)) {
+        X.x = 0.5 * (z.x + zc.x);
+        X.y = 0.5 * (z.y - zc.y);
+      } else {
+        X.x = 0.5 * (z.y + zc.y);
+        X.y = -0.5 * (z.x - zc.x);
+      }
+      o[e] = X;
+    }
+  }
+}
+
+// LDS: [lines][twiddles]; the half lines of a workgroup are staged over the
+// lines, combined through registers (kGenVals values per thread at most, which
+// P guarantees) and transformed in place.
+template <int CLS, int DIM, int OUT>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
+  if (a.active && !a.active[0]) return;
+  constexpr int NC = DIM * DIM;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[kGenMaxNT / 64];
+  const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x, RB = a.RB;
+  double2* s = reinterpret_cast<double2*>(smem);
+  const int stage = RB * nh * NC;  // staged values; the twiddles follow the larger of the two
+  double2* tw = s + (n * LS > stage ? n * LS : stage);
+  gen_twiddles<double>(tw, a.tw, n);
+  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  {
+    const int64_t base = row0 * nh * NC, lim = a.rows * nh * NC;
+    constexpr int KB = 4;
+    for (int e0 = 0; e0 < stage; e0 += KB * NT) {
+      double2 t[KB];
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        t[i] = a.spec[e < stage && base + e < lim ? base + e : lim - 1];
+      }
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        if (e < stage) s[e] = base + e < lim ? t[i] : double2{};
+      }
+    }
+  }
+  __syncthreads();
+  const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
+  const bool act = p < a.P;
+  {
+    const int rp = l / NC, c = l - rp * NC;
+    const double2* A0 = s + (2 * rp) * nh * NC + c;
+    const double2* B0 = A0 + nh * NC;
+    double2 v[kGenVals];
+#pragma unroll
+    for (int i = 0; i < kGenVals; ++i) {
+      const int m = p + i * a.P;
+      if (act && m < n) {
+        const int kk = m < nh ? m : n - m;
+        double2 A = A0[kk * NC], B = B0[kk * NC];
+        if (kk == 0 || 2 * kk == n) A.y = B.y = 0.0;
+        if (m >= nh) {
+          A.y = -A.y;
+          B.y = -B.y;
+        }
+        v[i].x = A.x - B.y;
+        v[i].y = A.y + B.x;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kGenVals; ++i) {
+      const int m = p + i * a.P;
+      if (act && m < n) s[m * LS + l] = v[i];
+    }
+    __syncthreads();
+  }
+  auto none_ld = [](int) { return double2{}; };
+  auto none_st = [](int, double2) {};
+  gen_fft<double, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
+  const double* sr = reinterpret_cast<const double*>(smem);
+  double acc = 0.0;
+  for (int r = 0; r < RB; ++r) {
+    if (row0 + r >= a.rows) break;
+    const int64_t base = (row0 + r) * n * NC;
+    const double* sl = sr + 2 * ((r >> 1) * NC) + (r & 1);
+    const int tot = n * NC;
+    constexpr int KB = 4;
+    for (int e0 = 0; e0 < tot; e0 += KB * NT) {
+      double dv[KB];
+      if (OUT == OUT_DOT) {
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+          const int e = e0 + i * NT + threadIdx.x;
+          dv[i] = a.dotv[base + (e < tot ? e : tot - 1)];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        if (e < tot) {
+          const int m = e / NC, c = e - m * NC;
+          const double val = sl[2 * (m * LS + c)];
+          a.out[base + e] = val;
+          if (OUT == OUT_DOT) acc += val * dv[i];
+        }
+      }
+    }
+  }
+  if (OUT == OUT_DOT) {
+    const double t = block_sum_waves(acc, red);
+    if (threadIdx.x == 0) a.partials[blockIdx.x] = t;
+  }
+}
+
+void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a) {
+  const int d = p.dim - 1;
+  a.in = static_cast<const double*>(op.in);
+  a.rvec = static_cast<const double*>(op.rvec);
+  a.pout = static_cast<double*>(op.pout);
+  a.scal = op.scal;
+  a.tan = static_cast<const double*>(op.tangent);
+  a.tan_kind = op.tan_kind;
+  a.spec = static_cast<double2*>(spec);
+  a.out = static_cast<double*>(op.out);
+  a.dotv = static_cast<const double*>(op.dotv);
+  a.partials = static_cast<double*>(p.partials);
+  a.rows = p.N / p.res[d];
+  a.RB = g.mult * 2;
+  a.L = g.L;
+  a.P = g.P;
+  a.LS = g.L | 1;
+  a.ax = p.gen[d];
+  a.tw = static_cast<const double2*>(p.tw64[d]);
+  a.active = p.active;
+}
+
+template <int CLS, int DIM>
+int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
+  const GenShape& g = p.gen_last;
+  GLast a{};
+  fill(p, op, spec, g, a);
+  const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  switch (op.in_mode) {
+    case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN>), grid, block, g.lds, stream(), a); break;
+    case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN>), grid, block, g.lds, stream(), a); break;
+    default: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE>), grid, block, g.lds, stream(), a); break;
+  }
+  MUGPU_HIP(hipGetLastError());
+  return MUGPU_OK;
+}
+
+template <int CLS, int DIM>
+int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
+  const GenShape& g = p.gen_last;
+  GLast a{};
+  fill(p, op, spec, g, a);
+  const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  if (op.out_mode == OUT_DOT)
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT>), grid, block, g.lds, stream(), a);
+  else
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN>), grid, block, g.lds, stream(), a);
+  MUGPU_HIP(hipGetLastError());
+  return MUGPU_OK;
+}
+
+}  // namespace
+
+int gen_r2c(FftPlan& p, const OpSpec& op, void* spec) {
+  const bool c1 = p.gen[p.dim - 1].cls != 0;
+  if (p.dim == 3) return c1 ? r2c_launch<1, 3>(p, op, spec) : r2c_launch<0, 3>(p, op, spec);
+  return c1 ? r2c_launch<1, 2>(p, op, spec) : r2c_launch<0, 2>(p, op, spec);
+}
+
+int gen_c2r(FftPlan& p, const OpSpec& op, void* spec) {
+  const bool c1 = p.gen[p.dim - 1].cls != 0;
+  if (p.dim == 3) return c1 ? c2r_launch<1, 3>(p, op, spec) : c2r_launch<0, 3>(p, op, spec);
+  return c1 ? c2r_launch<1, 2>(p, op, spec) : c2r_launch<0, 2>(p, op, spec);
+}
+
+}  // namespace mugpu

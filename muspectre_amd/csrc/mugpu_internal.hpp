@@ -110,6 +110,51 @@ __host__ __device__ constexpr int sym_index(int r, int c, int n) {
 enum Scalar { SC_RDR = 0, SC_PAP, SC_ALPHA, SC_NEWRDR, SC_BETA, SC_TMP0, SC_TMP1, SC_TOL2,
               SC_XALPHA, SC_COUNT };
 
+// ---- passes of run-time length (FP64; fft_gen.hpp) -------------------------------
+constexpr int kGenMaxPass = 12;
+constexpr int kGenQ = 4;          // output pairs of a prime radix formed at once
+constexpr int kGenTB = 2;         // such tasks held per thread
+constexpr int kGenMaxNT = 512;    // threads per workgroup
+constexpr int kGenThreads = 256;  // aimed at, where the passes can use them
+constexpr int kGenVals = 18;      // complex values of a line held per thread
+constexpr size_t kGenMaxLds = 150 * 1024;
+constexpr size_t kGenLds = 40 * 1024;  // four workgroups per CU
+// radices with a compiled butterfly, and how many of them a thread holds
+__host__ __device__ constexpr bool gen_compiled(int R) {
+  return R <= 5 || R == 7 || R == 8 || R == 9 || R == 11 || R == 13 || R == 17;
+}
+__host__ __device__ constexpr int gen_held(int R) { return R >= 16 ? 1 : 16 / R; }
+struct GenPass {
+  int R, NS, nb, step;  // radix, span before it, n / R, n / (NS R)
+  unsigned magic;       // j / NS = (j magic) >> 32
+};
+struct GenAxis {
+  int n, np, cls;  // cls 1: a radix above 9
+  GenPass ps[kGenMaxPass];
+};
+// shape of a workgroup: `mult` row pairs or k-points, L lines, P threads per
+// line; NT = 0: the axis does not fit
+struct GenShape {
+  int mult = 0, L = 0, P = 0, NT = 0;
+  size_t lds = 0;
+};
+bool gen_radices(int n, GenAxis& ax);
+GenShape gen_last_shape(const GenAxis& ax, int nc, int64_t rows);
+GenShape gen_axis0_shape(const GenAxis& ax, int nc, int64_t plane);
+GenShape gen_strided_shape(const GenAxis& ax, int64_t inner, int64_t outer);
+
+// Workgroups are dispatched to the 8 XCDs round robin (workgroup b runs on
+// XCD b mod 8), each XCD with its own L2.  Tiles next to each other in HBM
+// share cache lines at their edges, so the tile of workgroup b is chosen to
+// give every XCD one contiguous range of tiles: neighbours then meet in the
+// same L2.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int64_t xcd_tile(int64_t b, int64_t total) {
+  const int64_t q = total / kXcds, r = total - q * kXcds;
+  const int64_t x = b % kXcds, local = b / kXcds;
+  return x * q + (x < r ? x : r) + local;
+}
+
 // ---- FFT plan -----------------------------------------------------------------
 struct FftPlan {
   int dim = 0, nc = 0, prec = MUGPU_FP64;
@@ -128,6 +173,10 @@ struct FftPlan {
   int64_t nzblocks = 0;      // z-pass workgroups, the largest of nzb
   int64_t nzb[2] = {0, 0};   // c2r workgroups (p.Ap partials) per precision (0 FP64, 1 FP32)
   bool fastax[3] = {false, false, false};  // compile-time-length passes (fft_fast.hip)
+  // run-time-length passes of FP64 grids, per axis (genax: the axis has them)
+  GenAxis gen[3];
+  bool genax[3] = {false, false, false};
+  GenShape gen_last, gen_axis0, gen_str[3];
   // variant of each compile-time-length pass (bit 0: 8 values per thread
   // instead of 16 or 12; bit 1: half the rows or k-points per workgroup, for
   // the last-axis and first-axis projection passes), per precision (0 FP64,
@@ -150,7 +199,11 @@ void force_variant(int pass, int prec, int variant);
 // this length, dimension and precision
 bool fast_variant_valid(int pass, int n, int dim, int prec, int variant);
 
-int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec);
+// general: FP64 passes of run-time length where they fit.  Cells of the
+// FP32-refined solve go without: their x carries the FP32 rounding of its
+// inner solves (1.5e-6 relative), so a last-bit change of the FP64 residuals
+// would move their results by that much
+int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool general = true);
 void plan_free(FftPlan& p);
 
 // projection parameters handed to the fused axis-0 kernel
@@ -202,6 +255,11 @@ int fast_r2c(FftPlan& p, int prec, const OpSpec& op, void* spec);
 int fast_c2r(FftPlan& p, int prec, const OpSpec& op, void* spec);
 int fast_strided(FftPlan& p, int prec, int ax, void* spec, int sign);
 int fast_axis0_project(FftPlan& p, int prec, const ProjParams& pj, void* spec);
+// FP64 passes along axes of run-time length (fft_gen_last.hip, fft_gen_axis.hip)
+int gen_r2c(FftPlan& p, const OpSpec& op, void* spec);
+int gen_c2r(FftPlan& p, const OpSpec& op, void* spec);
+int gen_strided(FftPlan& p, int ax, void* spec, int sign);
+int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec);
 // the HBM pattern of the first-axis pass alone (n rows of plane k-points of nc
 // complex components, tiles of kp k-points), in place (fft_fast.hip)
 int line_pattern(void* data, int prec, int n, int64_t plane, int nc, int kp);
