@@ -264,7 +264,10 @@ int mugpu_scale_copy(double a, const void *d_x, void *d_y, int64_t n);
  * scalars carry the solve's r.r and beta from call to call.
  * mugpu_cg_start: x = 0; r = A x - b (= 0 - b: the operator of a zero
  *   field is zero exactly, so it is not applied; Ap is left unset);
- *   p = -r; returns rdr = r.r and rhs_norm2 = b.b.
+ *   p = -r; returns rdr = r.r and rhs_norm2 = b.b.  It also finds out
+ *   whether b = G b (as for every right-hand side of the Newton drivers):
+ *   the solve's p then stays in the range of the projector G, p.Ap =
+ *   p.(K:p), and the operator's last pass updates r itself.
  * mugpu_cg_step: [if update_p: p = -r + beta p with beta from the previous
  *   step] Ap = A p; alpha = rdr/(p.Ap); x += alpha p; r += alpha Ap;
  *   new_rdr = r.r; beta = new_rdr/rdr.  Returns new_rdr.
@@ -275,7 +278,8 @@ int mugpu_scale_copy(double a, const void *d_x, void *d_y, int64_t n);
  *   new_rdr > tol2 (the first always runs).  *steps returns the iterations
  *   run (one whose r.r is NaN counts and stops the loop), *new_rdr the r.r
  *   of the last.  The host reads back once per call instead of once per
- *   iteration; the arithmetic is that of mugpu_cg_step.  Where the last
+ *   iteration; the arithmetic is that of mugpu_cg_step.  Ap is work space
+ *   of this call (A p is not stored where the last pass updates r).  Where the last
  *   axis has compiled passes (lengths 16, 32, 48, 64, 96, 128, 256, 512),
  *   the x update of an iteration is applied by the next iteration's first
  *   pass (which reads p anyway), so the x update of the last iteration of a call is left

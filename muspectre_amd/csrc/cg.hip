@@ -4,6 +4,7 @@
 // workgroup adds them in a fixed order, so a result does not depend on
 // what else runs on the device.
 #include "mugpu_internal.hpp"
+#include "op_stages.hpp"
 
 namespace mugpu {
 
@@ -105,15 +106,43 @@ __global__ __launch_bounds__(kRT) void k_axpy_alpha(T* __restrict__ x, const T* 
   for (int64_t i = (int64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += stride) x[i] += al * p[i];
 }
 
-// r = Ax - b ; p = -r (Ax == nullptr: x = 0, where A x is zero exactly)
-template <typename T>
-__global__ __launch_bounds__(kRT) void k_cg_init(const T* __restrict__ Ax, const T* __restrict__ b,
-                                                 T* __restrict__ r, T* __restrict__ p, int64_t n) {
+// x = 0, r = -b, p = b and the partials of b.b and, kRedGrid further on, of
+// |b - g|^2 (g = G b tells whether b is in the range of G)
+__global__ __launch_bounds__(kRT) void k_cg_start(const double* __restrict__ b,
+                                                  const double* __restrict__ g, double* __restrict__ x,
+                                                  double* __restrict__ r, double* __restrict__ p,
+                                                  int64_t n, double* partials) {
+  __shared__ double red[16];
+  double bb = 0.0, dd = 0.0;
   const int64_t stride = (int64_t)gridDim.x * kRT;
   for (int64_t i = (int64_t)blockIdx.x * kRT + threadIdx.x; i < n; i += stride) {
-    const T rv = (Ax ? Ax[i] : T(0)) - b[i];
+    const double v = b[i], d = v - g[i], rv = 0.0 - v;
+    x[i] = 0.0;
     r[i] = rv;
     p[i] = -rv;
+    bb += v * v;
+    dd += d * d;
+  }
+  const double t = block_sum_waves(bb, red, kRT);
+  __syncthreads();
+  const double u = block_sum_waves(dd, red, kRT);
+  if (threadIdx.x == 0) {
+    partials[blockIdx.x] = t;
+    partials[kRedGrid + blockIdx.x] = u;
+  }
+}
+
+__global__ __launch_bounds__(1024) void k_cg_start_final(const double* __restrict__ partials, int count,
+                                                         double* scal) {
+  __shared__ double red[16];
+  const bool on = (int)threadIdx.x < count;
+  const double t = block_sum_waves(on ? partials[threadIdx.x] : 0.0, red, 1024);
+  __syncthreads();
+  const double u = block_sum_waves(on ? partials[kRedGrid + threadIdx.x] : 0.0, red, 1024);
+  if (threadIdx.x == 0) {
+    scal[SC_RDR] = t;
+    scal[SC_TMP0] = t;
+    scal[SC_TMP1] = u;
   }
 }
 
@@ -478,14 +507,12 @@ int scal_copy(double* d_scal, int from, int to) {
   return MUGPU_OK;
 }
 
-int cg_init_vectors(int prec, const void* Ax, const void* b, void* r, void* p, int64_t n) {
-  const unsigned g = grid_for(n);
-  if (prec == MUGPU_FP64)
-    hipLaunchKernelGGL((k_cg_init<double>), dim3(g), dim3(kRT), 0, stream(), (const double*)Ax,
-                       (const double*)b, (double*)r, (double*)p, n);
-  else
-    hipLaunchKernelGGL((k_cg_init<float>), dim3(g), dim3(kRT), 0, stream(), (const float*)Ax,
-                       (const float*)b, (float*)r, (float*)p, n);
+int cg_start_vectors(const double* b, const double* g, double* x, double* r, double* p, int64_t n,
+                     double* d_partials, double* d_scal) {
+  static_assert(kRedGrid <= 1024 && 2 * kRedGrid <= kRedBlocks, "one partial per thread, two halves");
+  const unsigned grid = grid_for(n);
+  hipLaunchKernelGGL(k_cg_start, dim3(grid), dim3(kRT), 0, stream(), b, g, x, r, p, n, d_partials);
+  hipLaunchKernelGGL(k_cg_start_final, dim3(1), dim3(1024), 0, stream(), d_partials, (int)grid, d_scal);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }

@@ -421,6 +421,7 @@ struct LArgs {
   const c_t<T>* tw;
   const int* active;  // FftPlan::active (single-cell kernels only)
   T* x;               // OpSpec::xvec (IN_TAN_PUPDATE_X kernels only)
+  T* ap;              // OpSpec::ap_out (OUT_RUPD kernels only)
 };
 
 // ISO: the tangent is known to be isotropic (TAN_ISO), which the compiler
@@ -432,6 +433,7 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   T* sr = reinterpret_cast<T*>(smem);
   const int64_t row0 = bx * RB;
+  double acc = 0.0;  // p . K p of this workgroup (FP64)
   if constexpr (IN == IN_PLAIN) {
     const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
     for (int e = threadIdx.x; e < RB * N * NC; e += NT) {
@@ -500,6 +502,10 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
 #pragma unroll
           for (int c = 0; c < NC; ++c) pv[c] = sr[2 * (m * LS + (r >> 1) * NC + c) + (r & 1)];
           tangent_product<T, DIM>(KIND, a.tan, row * N + m, pv, dp);
+          if constexpr (sizeof(T) == 8) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc += pv[c] * dp[c];
+          }
 #pragma unroll
           for (int c = 0; c < NC; ++c) sr[2 * (m * LS + (r >> 1) * NC + c) + (r & 1)] = dp[c];
         }
@@ -542,6 +548,13 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
       X.y = T(-0.5) * (z.x - zc.x);
     }
     a.spec[obase + e] = X;
+  }
+  if constexpr (sizeof(T) == 8 && IN != IN_PLAIN) {
+    if (a.partials) {
+      __syncthreads();
+      const double t = block_sum_waves(acc, reinterpret_cast<double*>(smem), NT);
+      if (threadIdx.x == 0) a.partials[bx] = t;
+    }
   }
 }
 
@@ -649,16 +662,18 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   const T* sr = reinterpret_cast<const T*>(smem);
   const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
   double acc = 0.0;
+  const T al = OUT == OUT_RUPD ? (T)a.scal[SC_ALPHA] : T(0);
   {
     constexpr int TOT = RB * N * NC, kBatch = 8;
     for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
       T dv[kBatch];
-      if (OUT == OUT_DOT) {
+      if (OUT != OUT_PLAIN) {
+        const T* __restrict__ dsrc = OUT == OUT_RUPD ? a.out : a.dotv;
 #pragma unroll
         for (int i = 0; i < kBatch; ++i) {
           const int e = e0 + i * NT + threadIdx.x;
           const int64_t g = base + e < lim ? base + e : lim - 1;
-          dv[i] = a.dotv[g];
+          dv[i] = dsrc[g];
         }
       }
 #pragma unroll
@@ -668,13 +683,24 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
           const int r = e / (N * NC), rem = e - r * (N * NC);
           const int m = rem / NC, c = rem - m * NC;
           const T val = sr[2 * (m * LS + (r >> 1) * NC + c) + (r & 1)];
-          a.out[base + e] = val;
-          if (OUT == OUT_DOT) acc += (double)val * (double)dv[i];
+          if constexpr (OUT == OUT_RUPD) {
+            const T rv = dv[i] + al * val;
+            a.out[base + e] = rv;
+            if (a.ap) a.ap[base + e] = val;
+            acc += (double)rv * (double)rv;
+          } else {
+            a.out[base + e] = val;
+            if (OUT == OUT_DOT) acc += (double)val * (double)dv[i];
+          }
         }
       }
     }
   }
-  if (OUT == OUT_DOT) {
+  if constexpr (OUT == OUT_RUPD) {
+    __syncthreads();
+    const double t = block_sum_waves(acc, reinterpret_cast<double*>(smem), NT);
+    if (threadIdx.x == 0) a.partials[bx] = t;
+  } else if (OUT == OUT_DOT) {
     __syncthreads();
     const double t = block_sum_any<NT>(acc, reinterpret_cast<double*>(smem));
     if (threadIdx.x == 0) a.partials[bx] = t;

@@ -20,6 +20,15 @@ int c2r_n(FftPlan& p, const OpSpec& op, void* spec) {
   constexpr int NT = RB / 2 * NC * (N / E);
   constexpr size_t lds = TwLds<T, N>::total(lds_c2r<T, N, E, DIM, H>());
   const dim3 grid((unsigned)((a.rows + RB - 1) / RB));
+  if constexpr (sizeof(T) == 8) {
+    a.scal = op.scal;
+    a.ap = reinterpret_cast<T*>(op.ap_out);
+    if (op.out_mode == OUT_RUPD) {
+      hipLaunchKernelGGL((k_c2r_fast<T, N, E, DIM, OUT_RUPD, H>), grid, dim3(NT), lds, stream(), a);
+      MUGPU_HIP(hipGetLastError());
+      return MUGPU_OK;
+    }
+  }
   if (op.out_mode == OUT_DOT)
     hipLaunchKernelGGL((k_c2r_fast<T, N, E, DIM, OUT_DOT, H>), grid, dim3(NT), lds, stream(), a);
   else

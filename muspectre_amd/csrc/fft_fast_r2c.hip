@@ -20,6 +20,7 @@ int r2c_n(FftPlan& p, const OpSpec& op, void* spec) {
   a.tw = tw_of<T>(p, DIM - 1);
   a.active = p.active;
   a.x = reinterpret_cast<T*>(op.xvec);
+  a.partials = op.fin_alpha ? reinterpret_cast<double*>(p.partials) : nullptr;
   constexpr int RB = z_rows(N, DIM, H);
   constexpr int NT = RB / 2 * DIM * DIM * (N / E);
   constexpr size_t lds = TwLds<T, N>::total(lds_lines<T, N, DIM, H>());

@@ -362,18 +362,5 @@ __device__ __forceinline__ void gen_twiddles(c_t<T>* dst, const c_t<T>* __restri
   for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = tw[i];
 }
 
-// sum over a workgroup of whole wavefronts (fixed order): in each wavefront by
-// lane halving, then over the wavefronts; the result is valid in thread 0
-__device__ __forceinline__ double block_sum_waves(double v, double* red) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) v += __shfl_down(v, s, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double t = 0.0;
-  if (threadIdx.x == 0)
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-  return t;
-}
-
 }  // namespace
 }  // namespace mugpu

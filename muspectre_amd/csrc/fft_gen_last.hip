@@ -22,6 +22,8 @@ struct GLast {
   int tan_kind;
   double2* spec;
   double* out;
+  double* x;
+  double* ap;
   const double* dotv;
   double* partials;
   int64_t rows;
@@ -43,24 +45,29 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x;
   double2* s = reinterpret_cast<double2*>(smem);
   double* sr = reinterpret_cast<double*>(smem);
+  __shared__ double red[16];
   double2* tw = s + n * LS;
   double* sp = reinterpret_cast<double*>(tw + n);
   gen_twiddles<double>(tw, a.tw, n);
   const int64_t row0 = (int64_t)blockIdx.x * a.RB;
-  const double beta = IN == IN_TAN_PUPDATE ? a.scal[SC_BETA] : 0.0;
+  constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
+  const double beta = PU ? a.scal[SC_BETA] : 0.0;
+  const double al = XU ? a.scal[SC_ALPHA] : 0.0;
+  double acc = 0.0;  // p . K p
   for (int r0 = 0; r0 < a.RB; r0 += 2) {
     const int64_t base = (row0 + r0) * n * NC, lim = a.rows * n * NC;
     const int tot = 2 * n * NC;
     constexpr int KB = 4;
     if (r0) __syncthreads();  // the staged rows before have been read
     for (int e0 = 0; e0 < tot; e0 += KB * NT) {
-      double pv[KB], rv[KB];
+      double pv[KB], rv[KB], xv[KB];
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
         const int e = e0 + i * NT + threadIdx.x;
         const int64_t g = e < tot && base + e < lim ? base + e : lim - 1;
         pv[i] = a.in[g];
-        if (IN == IN_TAN_PUPDATE) rv[i] = a.rvec[g];
+        if (PU) rv[i] = a.rvec[g];
+        if (XU) xv[i] = a.x[g];
       }
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
@@ -69,7 +76,8 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
           double x = 0.0;
           if (base + e < lim) {
             x = pv[i];
-            if (IN == IN_TAN_PUPDATE) {
+            if (XU) a.x[base + e] = xv[i] + al * x;
+            if (PU) {
               x = -rv[i] + beta * x;
               a.pout[base + e] = x;
             }
@@ -89,6 +97,8 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
         for (int c = 0; c < NC; ++c) p[c] = sp[e * NC + c];
         if (KIND >= 0 && row0 + r0 + r < a.rows) {
           tangent_product<double, DIM>(KIND, a.tan, (row0 + r0 + r) * n + m, p, dp);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc += p[c] * dp[c];
         } else {
 #pragma unroll
           for (int c = 0; c < NC; ++c) dp[c] = p[c];
@@ -132,6 +142,10 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
       o[e] = X;
     }
   }
+  if (IN != IN_PLAIN && a.partials) {
+    const double t = block_sum_waves(acc, red, NT);
+    if (threadIdx.x == 0) a.partials[blockIdx.x] = t;
+  }
 }
 
 // LDS: [lines][twiddles]; the half lines of a workgroup are staged over the
@@ -142,7 +156,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   if (a.active && !a.active[0]) return;
   constexpr int NC = DIM * DIM;
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ double red[kGenMaxNT / 64];
+  __shared__ double red[16];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x, RB = a.RB;
   double2* s = reinterpret_cast<double2*>(smem);
   const int stage = RB * nh * NC;  // staged values; the twiddles follow the larger of the two
@@ -201,6 +215,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   auto none_st = [](int, double2) {};
   gen_fft<double, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
   const double* sr = reinterpret_cast<const double*>(smem);
+  const double al = OUT == OUT_RUPD ? a.scal[SC_ALPHA] : 0.0;
   double acc = 0.0;
   for (int r = 0; r < RB; ++r) {
     if (row0 + r >= a.rows) break;
@@ -210,11 +225,12 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
     constexpr int KB = 4;
     for (int e0 = 0; e0 < tot; e0 += KB * NT) {
       double dv[KB];
-      if (OUT == OUT_DOT) {
+      if (OUT != OUT_PLAIN) {
+        const double* __restrict__ dsrc = OUT == OUT_RUPD ? a.out : a.dotv;
 #pragma unroll
         for (int i = 0; i < KB; ++i) {
           const int e = e0 + i * NT + threadIdx.x;
-          dv[i] = a.dotv[base + (e < tot ? e : tot - 1)];
+          dv[i] = dsrc[base + (e < tot ? e : tot - 1)];
         }
       }
 #pragma unroll
@@ -223,14 +239,21 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
         if (e < tot) {
           const int m = e / NC, c = e - m * NC;
           const double val = sl[2 * (m * LS + c)];
-          a.out[base + e] = val;
-          if (OUT == OUT_DOT) acc += val * dv[i];
+          if (OUT == OUT_RUPD) {
+            const double rv = dv[i] + al * val;
+            a.out[base + e] = rv;
+            if (a.ap) a.ap[base + e] = val;
+            acc += rv * rv;
+          } else {
+            a.out[base + e] = val;
+            if (OUT == OUT_DOT) acc += val * dv[i];
+          }
         }
       }
     }
   }
-  if (OUT == OUT_DOT) {
-    const double t = block_sum_waves(acc, red);
+  if (OUT != OUT_PLAIN) {
+    const double t = block_sum_waves(acc, red, NT);
     if (threadIdx.x == 0) a.partials[blockIdx.x] = t;
   }
 }
@@ -246,6 +269,8 @@ void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a)
   a.spec = static_cast<double2*>(spec);
   a.out = static_cast<double*>(op.out);
   a.dotv = static_cast<const double*>(op.dotv);
+  a.x = static_cast<double*>(op.xvec);
+  a.ap = static_cast<double*>(op.ap_out);
   a.partials = static_cast<double*>(p.partials);
   a.rows = p.N / p.res[d];
   a.RB = g.mult * 2;
@@ -262,11 +287,16 @@ int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
   const GenShape& g = p.gen_last;
   GLast a{};
   fill(p, op, spec, g, a);
+  if (!op.fin_alpha) a.partials = nullptr;
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
   switch (op.in_mode) {
     case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN>), grid, block, g.lds, stream(), a); break;
     case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN>), grid, block, g.lds, stream(), a); break;
-    default: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE>), grid, block, g.lds, stream(), a); break;
+    default:
+      if (op.xvec) hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE_X>), grid, block, g.lds, stream(), a);
+      else hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE>), grid, block, g.lds, stream(), a);
+      break;
   }
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
@@ -278,7 +308,9 @@ int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
   GLast a{};
   fill(p, op, spec, g, a);
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
-  if (op.out_mode == OUT_DOT)
+  if (op.out_mode == OUT_RUPD)
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD>), grid, block, g.lds, stream(), a);
+  else if (op.out_mode == OUT_DOT)
     hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT>), grid, block, g.lds, stream(), a);
   else
     hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN>), grid, block, g.lds, stream(), a);

@@ -525,6 +525,10 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
       p.nzb[pr] = (rows + rb - 1) / rb;
     }
     p.zrb = fast_rows_per_block(n, dim, 0);
+    for (int iso = 0; iso < 2; ++iso) {
+      const int rb = fast_rows_per_block(n, dim, p.fvar[0][FV_R2C][iso]);
+      p.nzr[iso] = (rows + rb - 1) / rb;
+    }
   } else {
     if (!fits((nc + 1) / 2, n, kNT)) {
       set_error("last axis of %d points exceeds the supported line length", n);
@@ -543,7 +547,7 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
   if (!p.fastax[dim - 1]) p.nzb[0] = p.nzb[1] = (rows + p.zrb - 1) / p.zrb;
   if (p.genax[dim - 1]) {
     const int rb = 2 * p.gen_last.mult;
-    p.nzb[0] = (rows + rb - 1) / rb;
+    p.nzb[0] = p.nzr[0] = p.nzr[1] = (rows + rb - 1) / rb;
   }
   p.nzblocks = p.nzb[0] > p.nzb[1] ? p.nzb[0] : p.nzb[1];
   // strided middle axis: up to 16 lines (256 B rows in FP64)
@@ -790,9 +794,15 @@ int launch_project(FftPlan& p, const ProjParams& pj, c_t<T>* spec) {
 template <typename T, int DIM>
 int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spectrum) {
   c_t<T>* spec = reinterpret_cast<c_t<T>*>(spectrum);
-  // the fused x update is carried by the compiled last-axis r2c only
-  if (op.xvec && !p.fastax[DIM - 1]) return MUGPU_EARG;
+  // the fused x update and the early alpha are not carried by the passes of
+  // this file
+  const bool carried = p.fastax[DIM - 1] || (sizeof(T) == 8 && p.genax[DIM - 1]);
+  if (op.xvec && !carried) return MUGPU_EARG;
+  if ((op.fin_alpha || op.out_mode == OUT_RUPD) && (sizeof(T) != 8 || !carried)) return MUGPU_EARG;
   MUGPU_TRY((launch_r2c<T, DIM>(p, op, spec)));
+  if (op.fin_alpha)
+    MUGPU_TRY(finalize((const double*)p.partials, p.nzr[op.tan_kind == TAN_ISO ? 1 : 0], op.fin_alpha,
+                       FIN_ALPHA, const_cast<int*>(p.active)));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, -1));
   if (pj.kind >= 0) {
     MUGPU_TRY((launch_project<T, DIM>(p, pj, spec)));

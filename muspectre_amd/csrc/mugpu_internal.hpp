@@ -170,6 +170,7 @@ struct FftPlan {
   int xWk = 1;     // fused axis-0 projection pass: k-points per workgroup
   int xNT = 256;   // threads of the fused pass
   void* partials = nullptr;  // double per z-pass workgroup
+  int64_t nzr[2] = {0, 0};   // r2c workgroups of FP64 (p.Kp partials): full, isotropic tangent
   int64_t nzblocks = 0;      // z-pass workgroups, the largest of nzb
   int64_t nzb[2] = {0, 0};   // c2r workgroups (p.Ap partials) per precision (0 FP64, 1 FP32)
   bool fastax[3] = {false, false, false};  // compile-time-length passes (fft_fast.hip)
@@ -219,7 +220,9 @@ struct ProjParams {
 // alpha p_old (chosen by the launcher when OpSpec::xvec is set)
 enum InMode { IN_PLAIN = 0, IN_TAN = 1, IN_TAN_PUPDATE = 2, IN_TAN_PUPDATE_X = 3 };
 // output stage of the last-axis c2r pass
-enum OutMode { OUT_PLAIN = 0, OUT_DOT = 1 };
+// OUT_RUPD: r += alpha A p with the partials of r . r, for solves whose alpha is
+// known before the inverse transform (OpSpec::fin_alpha)
+enum OutMode { OUT_PLAIN = 0, OUT_DOT = 1, OUT_RUPD = 2 };
 
 struct OpSpec {
   int in_mode = IN_PLAIN;
@@ -234,8 +237,14 @@ struct OpSpec {
   int tan_kind = TAN_FULL;
   const void* tangent = nullptr; // plan precision
   int out_mode = OUT_PLAIN;
-  void* out = nullptr;           // real field (plan precision)
+  void* out = nullptr;           // real field (plan precision); OUT_RUPD: r
   const void* dotv = nullptr;    // vector dotted with the output for OUT_DOT
+  // FP64, IN_TAN*: alpha = r . r / (p . K p) is formed in fin_alpha (the scalar
+  // block) right after the first pass, from that pass's partials of p . K p.
+  // It equals r . r / (p . G K p) for p in the range of G, the orthogonal
+  // projector, so OUT_RUPD can use it and A p need not be stored
+  double* fin_alpha = nullptr;
+  void* ap_out = nullptr;        // OUT_RUPD: also store A p here (optional)
 };
 
 // full operator: r2c (with input stage) -> [axis passes] -> projection ->
@@ -319,7 +328,10 @@ int axpy_alpha(int prec, void* x, const void* p, const double* d_scal, int64_t n
                int slot = SC_ALPHA);
 // scal[to] = scal[from] on the device
 int scal_copy(double* d_scal, int from, int to);
-int cg_init_vectors(int prec, const void* Ax, const void* b, void* r, void* p, int64_t n);
+// start of an FP64 solve: x = 0, r = -b, p = b; b.b into scal[SC_RDR] and
+// scal[SC_TMP0], |b - g|^2 into scal[SC_TMP1]
+int cg_start_vectors(const double* b, const double* g, double* x, double* r, double* p, int64_t n,
+                     double* d_partials, double* d_scal);
 int axpby(int prec, double a, const void* x, double b, void* y, int64_t n);
 int convert(int from_prec, const void* src, int to_prec, void* dst, int64_t n, double scale);
 // x64 += scale d32; with p32: scale (d32 + scal[SC_ALPHA] p32)

@@ -191,4 +191,23 @@ __device__ double block_sum_any(double v, double* red) {
   return red[0];
 }
 
+// the same for a workgroup of NT threads (any NT <= 1024) by lane halving in
+// each wavefront, then over the wavefronts, in a fixed order; red holds 16
+// doubles; the result is valid in thread 0.  Every thread must call it.
+__device__ __forceinline__ double block_sum_waves(double v, double* red, int NT) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lanes = NT - 64 * wave < 64 ? NT - 64 * wave : 64;
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const double o = __shfl_down(v, s, 64);
+    if (lane + s < lanes) v += o;
+  }
+  if (lane == 0) red[wave] = v;
+  __syncthreads();
+  double t = 0.0;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < (NT + 63) / 64; ++w) t += red[w];
+  return t;
+}
+
 }  // namespace mugpu
