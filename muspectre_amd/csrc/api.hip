@@ -661,6 +661,8 @@ extern "C" int mugpu_fft_tune_pass(int dim, const int* res, int precision, int p
   for (int i = 0; i < 2; ++i) plan.fvar[pr][pass][i] = (unsigned char)variant;
   // (the plan's partials buffer holds the c2r partials of every variant)
   const size_t s = precision == MUGPU_FP64 ? 8 : 4;
+  // (the FP64 isotropic r2c runs with packed lines, as in a CG iteration)
+  plan.packed = pass == FV_R2C && precision == MUGPU_FP64 && iso != 0;
   const int tk = iso ? TAN_ISO : (dim == 3 ? TAN_SYM : TAN_FULL);
   const size_t nd = (size_t)plan.N * nc;
   void *spec = nullptr, *a = nullptr, *b = nullptr, *c = nullptr, *tan = nullptr;
@@ -1518,14 +1520,14 @@ extern "C" int mugpu_cg_step(mugpu_cell c, int update_p, void* d_x, void* d_r, v
     op.out = d_r;
     op.ap_out = d_Ap;
     MUGPU_TRY(run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum));
-    MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.nzb[0], c->scal, FIN_BETA));
+    MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA));
     MUGPU_TRY(axpy_alpha(MUGPU_FP64, d_x, d_p, c->scal, n));
   } else {
     op.out_mode = OUT_DOT;
     op.out = d_Ap;
     op.dotv = d_p;
     MUGPU_TRY(run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum));
-    MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.nzb[0], c->scal, FIN_ALPHA));
+    MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_ALPHA));
     MUGPU_TRY(cg_update(MUGPU_FP64, d_x, d_r, d_p, d_Ap, c->scal, n, c->partials));
   }
   MUGPU_TRY(sync_scalars(c->scal));
@@ -1578,10 +1580,10 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
     int e = run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum);
     if (early)
       return e != MUGPU_OK ? e
-                           : finalize((const double*)c->plan.partials, c->plan.nzb[0], c->scal, FIN_BETA,
+                           : finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA,
                                       c->ctl);
     if (e == MUGPU_OK)
-      e = finalize((const double*)c->plan.partials, c->plan.nzb[0], c->scal, FIN_ALPHA, c->ctl);
+      e = finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_ALPHA, c->ctl);
     if (e == MUGPU_OK)
       e = cg_update(MUGPU_FP64, fuse ? nullptr : d_x, d_r, d_p, d_Ap, c->scal, n, c->partials,
                     c->ctl);

@@ -187,24 +187,29 @@ constexpr int s_lines() {
 }
 
 // ---- LDS per workgroup and occupancy ----------------------------------------
-template <typename T, int N, int DIM, int H>
+// (PK: packed symmetric lines, op_stages.hpp)
+template <typename T, int N, int DIM, int H, bool PK>
 constexpr size_t lds_lines() {
-  return (size_t)N * lstride(z_rows(N, DIM, H) / 2 * DIM * DIM) * sizeof(c_t<T>);
+  constexpr size_t lines = (size_t)N * lstride(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK)) * sizeof(c_t<T>);
+  // the packed r2c pass stages all components of its rows first
+  constexpr size_t stage = PK ? (size_t)z_rows(N, DIM, H) * N * DIM * DIM * sizeof(T) : 0;
+  return lines > stage ? lines : stage;
 }
-template <typename T, int N, int E, int DIM, int H>
+template <typename T, int N, int E, int DIM, int H, bool PK>
 constexpr size_t lds_c2r() {
-  constexpr size_t lines = lds_lines<T, N, DIM, H>();
-  constexpr size_t tile = (size_t)z_rows(N, DIM, H) * (N / 2 + 1) * DIM * DIM * sizeof(c_t<T>);
-  constexpr size_t red = (size_t)z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E) * sizeof(double);
+  constexpr int NL = nb_lines(DIM, PK);
+  constexpr size_t lines = (size_t)N * lstride(z_rows(N, DIM, H) / 2 * NL) * sizeof(c_t<T>);
+  constexpr size_t tile = (size_t)z_rows(N, DIM, H) * (N / 2 + 1) * NL * sizeof(c_t<T>);
+  constexpr size_t red = (size_t)z_rows(N, DIM, H) / 2 * NL * (N / E) * sizeof(double);
   return lines > tile ? (lines > red ? lines : red) : (tile > red ? tile : red);
 }
 template <typename T, int N, int E>
 constexpr size_t lds_strided() {
   return (size_t)N * lstride(s_lines<T, N, E>()) * sizeof(c_t<T>);
 }
-template <typename T, int N, int E, int DIM, int H>
+template <typename T, int N, int E, int DIM, int H, bool PK>
 constexpr size_t lds_axis0() {
-  return (size_t)N * lstride(x_kpts(N, DIM, sizeof(T) == 4, E, H) * DIM * DIM) * sizeof(c_t<T>);
+  return (size_t)N * lstride(x_kpts(N, DIM, sizeof(T) == 4, E, H) * nb_lines(DIM, PK)) * sizeof(c_t<T>);
 }
 // Twiddle table W_N^m, m < N, in LDS: a workgroup copies the table after its
 // B bytes of lines, and the passes read it there (LDS reads, mostly
@@ -302,10 +307,10 @@ struct XArgs {
   const int* active;  // FftPlan::active (single-cell kernels only)
 };
 
-template <typename T, int N, int E, int DIM, int H>
+template <typename T, int N, int E, int DIM, int H, bool PK>
 __device__ __forceinline__ void axis0_body(const XArgs<T>& a, unsigned char* smem, int64_t bx,
                                            int64_t gx) {
-  constexpr int NC = DIM * DIM, KP = x_kpts(N, DIM, sizeof(T) == 4, E, H), L = KP * NC, LS = lstride(L),
+  constexpr int NC = nb_lines(DIM, PK), KP = x_kpts(N, DIM, sizeof(T) == 4, E, H), L = KP * NC, LS = lstride(L),
                 NT = L * (N / E);
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   const int l = threadIdx.x % L, p = threadIdx.x / L;
@@ -341,7 +346,8 @@ __device__ __forceinline__ void axis0_body(const XArgs<T>& a, unsigned char* sme
       for (int r = 0; r < NC; ++r) f[r] = czero<T>();
       continue;
     }
-    project_point<T, DIM>(f, 1, xi, a.kind, a.norm);
+    if constexpr (PK) project_point_sym<T, DIM>(f, xi, a.norm);
+    else project_point<T, DIM>(f, 1, xi, a.kind, a.norm);
   }
   __syncthreads();
   load_first<T, N, E>(v, p, [&](int m) { return at(m); });
@@ -350,21 +356,21 @@ __device__ __forceinline__ void axis0_body(const XArgs<T>& a, unsigned char* sme
   if (valid) store_last<T, N, E>(v, p, [&](int m, c_t<T> x) { base[m * inner] = x; });
 }
 
-template <typename T, int N, int E, int DIM, int H>
+template <typename T, int N, int E, int DIM, int H, bool PK>
 __device__ __forceinline__ void axis0_entry(const XArgs<T>& a, unsigned char* smem) {
   if (a.active && !a.active[0]) return;
   XArgs<T> b = a;
-  b.tw = twiddles_for<T, N, x_kpts(N, DIM, sizeof(T) == 4, E, H) * DIM * DIM * (N / E),
-                      lds_axis0<T, N, E, DIM, H>()>(a.tw, smem);
-  axis0_body<T, N, E, DIM, H>(b, smem, blockIdx.x, gridDim.x);
+  b.tw = twiddles_for<T, N, x_kpts(N, DIM, sizeof(T) == 4, E, H) * nb_lines(DIM, PK) * (N / E),
+                      lds_axis0<T, N, E, DIM, H, PK>()>(a.tw, smem);
+  axis0_body<T, N, E, DIM, H, PK>(b, smem, blockIdx.x, gridDim.x);
 }
 
-template <typename T, int N, int E, int DIM, int H>
+template <typename T, int N, int E, int DIM, int H, bool PK>
 // (no register bound: the projection stage needs its registers, and spilling
 // them costs more than the second workgroup per CU gains)
-__global__ __launch_bounds__(x_kpts(N, DIM, sizeof(T) == 4, E, H) * DIM * DIM * (N / E)) void k_axis0_fast(XArgs<T> a) {
+__global__ __launch_bounds__(x_kpts(N, DIM, sizeof(T) == 4, E, H) * nb_lines(DIM, PK) * (N / E)) void k_axis0_fast(XArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  axis0_entry<T, N, E, DIM, H>(a, smem);
+  axis0_entry<T, N, E, DIM, H, PK>(a, smem);
 }
 
 // The same pass with the register allocation told to leave room for
@@ -377,11 +383,11 @@ template <typename T>
 __host__ __device__ constexpr int axis0_hint() {
   return sizeof(T) == 8 ? 4 : 6;
 }
-template <typename T, int N, int E, int DIM, int H>
-__global__ __launch_bounds__(x_kpts(N, DIM, sizeof(T) == 4, E, H) * DIM * DIM * (N / E))
+template <typename T, int N, int E, int DIM, int H, bool PK>
+__global__ __launch_bounds__(x_kpts(N, DIM, sizeof(T) == 4, E, H) * nb_lines(DIM, PK) * (N / E))
 __attribute__((amdgpu_waves_per_eu(axis0_hint<T>()))) void k_axis0_bounded(XArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  axis0_entry<T, N, E, DIM, H>(a, smem);
+  axis0_entry<T, N, E, DIM, H, PK>(a, smem);
 }
 
 template <int N, int E, int DIM, int H>
@@ -397,8 +403,8 @@ __global__ __launch_bounds__(x_kpts(N, DIM, true, E, H) * DIM * DIM * (N / E)) v
   a.norm = (float)sl.norm;
   extern __shared__ __align__(16) unsigned char smem[];
   a.tw = twiddles_for<float, N, x_kpts(N, DIM, true, E, H) * DIM * DIM * (N / E),
-                      lds_axis0<float, N, E, DIM, H>()>(shape.tw, smem);
-  axis0_body<float, N, E, DIM, H>(a, smem, blockIdx.x, gridDim.x);
+                      lds_axis0<float, N, E, DIM, H, false>()>(shape.tw, smem);
+  axis0_body<float, N, E, DIM, H, false>(a, smem, blockIdx.x, gridDim.x);
 }
 
 // ---- last axis: input stage, r2c ---------------------------------------------
@@ -426,15 +432,85 @@ struct LArgs {
 
 // ISO: the tangent is known to be isotropic (TAN_ISO), which the compiler
 // folds in; otherwise a.tan_kind selects it at run time
-template <typename T, int N, int E, int DIM, int IN, bool ISO, int H>
+template <typename T, int N, int E, int DIM, int IN, bool ISO, int H, bool PK>
 __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem, int64_t bx) {
-  constexpr int NC = DIM * DIM, RB = z_rows(N, DIM, H), L = RB / 2 * NC, LS = lstride(L);
+  constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK), RB = z_rows(N, DIM, H), L = RB / 2 * NL, LS = lstride(L);
   constexpr int NT = L * (N / E), NH = N / 2 + 1;
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   T* sr = reinterpret_cast<T*>(smem);
   const int64_t row0 = bx * RB;
   double acc = 0.0;  // p . K p of this workgroup (FP64)
-  if constexpr (IN == IN_PLAIN) {
+  if constexpr (PK) {
+    // the rows are staged as they lie in memory; each thread then forms the
+    // packed K : p (or the symmetric part of the field) of its voxels in
+    // registers, and the lines take the place of the staged rows
+    static_assert(IN == IN_PLAIN || ISO, "packed lines need a symmetric K : p");
+    constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
+    const T beta = PU ? (T)a.scal[SC_BETA] : T(0);
+    const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
+    constexpr int TOT = RB * N * NC, kBatch = 8;
+    const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
+    for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
+      T pv[kBatch], rv[kBatch], xv[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        const int64_t g = base + e < lim ? base + e : lim - 1;
+        pv[i] = a.in[g];
+        if (PU) rv[i] = a.rvec[g];
+        if (XU) xv[i] = a.x[g];
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int e = e0 + i * NT + threadIdx.x;
+        if (e < TOT) {
+          T x = T(0);
+          if (base + e < lim) {
+            x = pv[i];
+            if (XU) a.x[base + e] = xv[i] + al * x;
+            if (PU) {
+              x = -rv[i] + beta * x;
+              a.pout[base + e] = x;
+            }
+          }
+          sr[e] = x;
+        }
+      }
+    }
+    __syncthreads();
+    constexpr int V = (RB * N + NT - 1) / NT;
+    T q[V][NL];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int e = threadIdx.x + i * NT;
+      if (e < RB * N) {
+        T pv[NC], dp[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) pv[c] = sr[e * NC + c];
+        if (IN != IN_PLAIN) {
+          // (rows beyond the last one: p is zero and the tangent read is the
+          // last voxel's, so K : p is zero)
+          const int64_t vox = row0 * N + e, last = a.rows * N - 1;
+          tangent_product<T, DIM>(TAN_ISO, a.tan, vox < last ? vox : last, pv, dp);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc += pv[c] * dp[c];
+          pack_lines<T, DIM, true>(dp, q[i]);
+        } else {
+          pack_lines<T, DIM, true>(pv, q[i]);
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int e = threadIdx.x + i * NT;
+      if (e < RB * N) {
+        const int r = e / N, m = e - (e / N) * N;
+#pragma unroll
+        for (int c = 0; c < NL; ++c) sr[2 * (m * LS + (r >> 1) * NL + c) + (r & 1)] = q[i][c];
+      }
+    }
+  } else if constexpr (IN == IN_PLAIN) {
     const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
     for (int e = threadIdx.x; e < RB * N * NC; e += NT) {
       const int r = e / (N * NC), rem = e - r * (N * NC);
@@ -531,12 +607,12 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
   Passes<T, N, E, -1, 0, 1>::run(v, p, a.tw, at);
   store_last<T, N, E>(v, p, [&](int m, c_t<T> x) { at(m) = x; });
   __syncthreads();
-  const int64_t obase = row0 * NH * NC, olim = a.rows * NH * NC;
-  for (int e = threadIdx.x; e < RB * NH * NC; e += NT) {
+  const int64_t obase = row0 * NH * NL, olim = a.rows * NH * NL;
+  for (int e = threadIdx.x; e < RB * NH * NL; e += NT) {
     if (obase + e >= olim) break;
-    const int r = e / (NH * NC), rem = e - r * (NH * NC);
-    const int k = rem / NC, c = rem - k * NC;
-    const int ln = (r >> 1) * NC + c;
+    const int r = e / (NH * NL), rem = e - r * (NH * NL);
+    const int k = rem / NL, c = rem - k * NL;
+    const int ln = (r >> 1) * NL + c;
     const c_t<T> z = s[k * LS + ln];
     const c_t<T> zc = s[(k == 0 ? 0 : N - k) * LS + ln];
     c_t<T> X;
@@ -558,14 +634,14 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
   }
 }
 
-template <typename T, int N, int E, int DIM, int IN, bool ISO, int H>
-__global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E))
-MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<T, N, DIM, H>())) void k_r2c_fast(LArgs<T> a) {
+template <typename T, int N, int E, int DIM, int IN, bool ISO, int H, bool PK>
+__global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E))
+MUGPU_WPE(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), (lds_lines<T, N, DIM, H, PK>())) void k_r2c_fast(LArgs<T> a) {
   if (a.active && !a.active[0]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   LArgs<T> b = a;
-  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_lines<T, N, DIM, H>()>(a.tw, smem);
-  r2c_body<T, N, E, DIM, IN, ISO, H>(b, smem, blockIdx.x);
+  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), lds_lines<T, N, DIM, H, PK>()>(a.tw, smem);
+  r2c_body<T, N, E, DIM, IN, ISO, H, PK>(b, smem, blockIdx.x);
 }
 
 // batched: the first iteration of a solve takes p as it is, later ones
@@ -574,7 +650,7 @@ MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<T, N, DIM, H>(
 // the served material is isotropic (TAN_ISO tangents)
 template <int N, int E, int DIM, int H>
 __global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E))
-MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<float, N, DIM, H>())) void k_r2c_batch(
+MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<float, N, DIM, H, false>())) void k_r2c_batch(
     const BatchSlot* __restrict__ slots, int64_t rows, const float2* __restrict__ tw) {
   const BatchSlot& sl = slots[blockIdx.z];
   if (!sl.ctl[CTL_ACTIVE]) return;
@@ -589,9 +665,9 @@ MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<float, N, DIM,
   a.rows = rows;
   a.x = sl.x;
   extern __shared__ __align__(16) unsigned char smem[];
-  a.tw = twiddles_for<float, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_lines<float, N, DIM, H>()>(tw, smem);
-  if (sl.ctl[CTL_ITER] == 0) r2c_body<float, N, E, DIM, IN_TAN, true, H>(a, smem, blockIdx.x);
-  else r2c_body<float, N, E, DIM, IN_TAN_PUPDATE_X, true, H>(a, smem, blockIdx.x);
+  a.tw = twiddles_for<float, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_lines<float, N, DIM, H, false>()>(tw, smem);
+  if (sl.ctl[CTL_ITER] == 0) r2c_body<float, N, E, DIM, IN_TAN, true, H, false>(a, smem, blockIdx.x);
+  else r2c_body<float, N, E, DIM, IN_TAN_PUPDATE_X, true, H, false>(a, smem, blockIdx.x);
 }
 
 // ---- last axis: c2r, output stage ---------------------------------------------
@@ -599,17 +675,17 @@ MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_lines<float, N, DIM,
 // symmetry (imaginary parts of k = 0 and k = n/2 discarded) and combined into
 // Z = A + i B, whose backward transform holds row 2 rp in its real and row
 // 2 rp + 1 in its imaginary part.
-template <typename T, int N, int E, int DIM, int OUT, int H>
+template <typename T, int N, int E, int DIM, int OUT, int H, bool PK>
 __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem, int64_t bx) {
-  constexpr int NC = DIM * DIM, RB = z_rows(N, DIM, H), L = RB / 2 * NC, LS = lstride(L);
+  constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK), RB = z_rows(N, DIM, H), L = RB / 2 * NL, LS = lstride(L);
   constexpr int NT = L * (N / E), NH = N / 2 + 1;
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   const int64_t row0 = bx * RB;
   {
     // loads issued in batches of kBatch before their LDS stores, so that each
     // thread keeps several HBM requests in flight
-    constexpr int TOT = RB * NH * NC, kBatch = 8;
-    const int64_t base = row0 * NH * NC, lim = a.rows * NH * NC;
+    constexpr int TOT = RB * NH * NL, kBatch = 8;
+    const int64_t base = row0 * NH * NL, lim = a.rows * NH * NL;
     for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
       c_t<T> t[kBatch];
       // clamped, unconditional loads (a predicated load per element would be
@@ -635,12 +711,12 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   }
   __syncthreads();
   const int l = threadIdx.x % L, p = threadIdx.x / L;
-  const int rp = l / NC, cc = l - rp * NC;
+  const int rp = l / NL, cc = l - rp * NL;
   c_t<T> v[E];
   load_first<T, N, E>(v, p, [&](int i) {
     const int kk = i <= N / 2 ? i : N - i;
-    c_t<T> A = s[((2 * rp) * NH + kk) * NC + cc];
-    c_t<T> B = s[((2 * rp + 1) * NH + kk) * NC + cc];
+    c_t<T> A = s[((2 * rp) * NH + kk) * NL + cc];
+    c_t<T> B = s[((2 * rp + 1) * NH + kk) * NL + cc];
     if (kk == 0 || 2 * kk == N) {
       A.y = T(0);
       B.y = T(0);
@@ -682,7 +758,7 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
         if (e < TOT && base + e < lim) {
           const int r = e / (N * NC), rem = e - r * (N * NC);
           const int m = rem / NC, c = rem - m * NC;
-          const T val = sr[2 * (m * LS + (r >> 1) * NC + c) + (r & 1)];
+          const T val = sr[2 * (m * LS + (r >> 1) * NL + line_of<DIM, PK>(c)) + (r & 1)];
           if constexpr (OUT == OUT_RUPD) {
             const T rv = dv[i] + al * val;
             a.out[base + e] = rv;
@@ -707,19 +783,19 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   }
 }
 
-template <typename T, int N, int E, int DIM, int OUT, int H>
-__global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E))
-MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_c2r<T, N, E, DIM, H>())) void k_c2r_fast(LArgs<T> a) {
+template <typename T, int N, int E, int DIM, int OUT, int H, bool PK>
+__global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E))
+MUGPU_WPE(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), (lds_c2r<T, N, E, DIM, H, PK>())) void k_c2r_fast(LArgs<T> a) {
   if (a.active && !a.active[0]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   LArgs<T> b = a;
-  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_c2r<T, N, E, DIM, H>()>(a.tw, smem);
-  c2r_body<T, N, E, DIM, OUT, H>(b, smem, blockIdx.x);
+  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), lds_c2r<T, N, E, DIM, H, PK>()>(a.tw, smem);
+  c2r_body<T, N, E, DIM, OUT, H, PK>(b, smem, blockIdx.x);
 }
 
 template <int N, int E, int DIM, int H>
 __global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E))
-MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_c2r<float, N, E, DIM, H>())) void k_c2r_batch(
+MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_c2r<float, N, E, DIM, H, false>())) void k_c2r_batch(
     const BatchSlot* __restrict__ slots, int64_t rows, const float2* __restrict__ tw) {
   const BatchSlot& sl = slots[blockIdx.z];
   if (!sl.ctl[CTL_ACTIVE]) return;
@@ -730,8 +806,8 @@ MUGPU_WPE(z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), (lds_c2r<float, N, E, DIM
   a.partials = sl.zpart;
   a.rows = rows;
   extern __shared__ __align__(16) unsigned char smem[];
-  a.tw = twiddles_for<float, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_c2r<float, N, E, DIM, H>()>(tw, smem);
-  c2r_body<float, N, E, DIM, OUT_DOT, H>(a, smem, blockIdx.x);
+  a.tw = twiddles_for<float, N, z_rows(N, DIM, H) / 2 * DIM * DIM * (N / E), lds_c2r<float, N, E, DIM, H, false>()>(tw, smem);
+  c2r_body<float, N, E, DIM, OUT_DOT, H, false>(a, smem, blockIdx.x);
 }
 
 // ---- launchers ----------------------------------------------------------------

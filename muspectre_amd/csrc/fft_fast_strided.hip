@@ -8,7 +8,7 @@ namespace {
 
 template <typename T, int N, int E>
 int strided_n(FftPlan& p, int ax, void* spec, int sign) {
-  int64_t inner = p.nc;
+  int64_t inner = p.lines();
   for (int d = ax + 1; d < p.dim; ++d) inner *= p.hres[d];
   int64_t outer = 1;
   for (int d = 0; d < ax; ++d) outer *= p.hres[d];

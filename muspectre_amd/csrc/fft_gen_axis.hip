@@ -82,18 +82,18 @@ bool gen_radices(int n, GenAxis& ax) {
   return true;
 }
 
-GenShape gen_last_shape(const GenAxis& ax, int nc, int64_t rows) {
+GenShape gen_last_shape(const GenAxis& ax, int nc, int nl, int64_t rows) {
   // pairs of rows per workgroup: more while the grid keeps 1024 workgroups
   // and the LDS leaves room for four of them per CU
   GenShape best{};
   const int n = ax.n;
   for (int mult = 1; mult <= 8; ++mult) {
     GenShape g{};
-    const int L = mult * nc;
+    const int L = mult * nl;
     if (!threads_for(ax, L, g)) break;
     const size_t lines = (size_t)n * (L | 1) * 16, tw = (size_t)n * 16;
     const size_t fwd = lines + tw + (size_t)2 * n * nc * 8;
-    const size_t half = (size_t)2 * mult * (n / 2 + 1) * nc * 16;
+    const size_t half = (size_t)2 * mult * (n / 2 + 1) * nl * 16;
     const size_t bwd = (lines > half ? lines : half) + tw;
     g.mult = mult;
     g.lds = fwd > bwd ? fwd : bwd;
@@ -104,11 +104,11 @@ GenShape gen_last_shape(const GenAxis& ax, int nc, int64_t rows) {
   return best;
 }
 
-GenShape gen_axis0_shape(const GenAxis& ax, int nc, int64_t plane) {
+GenShape gen_axis0_shape(const GenAxis& ax, int nl, int64_t plane) {
   GenShape best{};
   for (int mult = 1; mult <= 4; mult *= 2) {
     GenShape g{};
-    const int L = mult * nc;
+    const int L = mult * nl;
     if (!threads_for(ax, L, g)) break;
     g.mult = mult;
     g.lds = (size_t)ax.n * ((L | 1) + 1) * 16;
@@ -178,10 +178,10 @@ struct GAxis0 {
   const int* active;  // FftPlan::active
 };
 
-template <int CLS, int DIM>
+template <int CLS, int DIM, bool PK>
 __global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0 a) {
   if (a.active && !a.active[0]) return;
-  constexpr int NC = DIM * DIM;
+  constexpr int NC = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS, KP = a.KP;
   double2* s = reinterpret_cast<double2*>(smem);
@@ -219,7 +219,8 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0 a) {
       for (int r = 0; r < NC; ++r) f[r] = double2{};
       continue;
     }
-    project_point<double, DIM>(f, 1, xi, a.kind, a.norm);
+    if constexpr (PK) project_point_sym<double, DIM>(f, xi, a.norm);
+    else project_point<double, DIM>(f, 1, xi, a.kind, a.norm);
   }
   __syncthreads();
   gen_fft<double, CLS, +1, false, true>(a.ax, a.P, p, act, s + l, LS, tw, ld, st);
@@ -230,11 +231,11 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0 a) {
 int gen_strided(FftPlan& p, int ax, void* spec, int sign) {
   GStr a{};
   a.data = static_cast<double2*>(spec);
-  a.inner = p.nc;
+  a.inner = p.lines();
   for (int d = ax + 1; d < p.dim; ++d) a.inner *= p.hres[d];
   int64_t outer = 1;
   for (int d = 0; d < ax; ++d) outer *= p.hres[d];
-  const GenShape& g = p.gen_str[ax];
+  const GenShape& g = p.gen_str[ax][p.packed ? 1 : 0];
   a.L = g.L;
   a.P = g.P;
   a.LS = g.L | 1;
@@ -257,7 +258,7 @@ int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec) {
   GAxis0 a{};
   a.data = static_cast<double2*>(spec);
   a.plane = p.kpts / p.res[0];
-  const GenShape& g = p.gen_axis0;
+  const GenShape& g = p.gen_axis0[p.packed ? 1 : 0];
   a.KP = g.mult;
   a.L = g.L;
   a.P = g.P;
@@ -274,13 +275,18 @@ int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec) {
   a.norm = pj.norm;
   a.active = p.active;
   const dim3 grid((unsigned)((a.plane + a.KP - 1) / a.KP)), block((unsigned)g.NT);
-  if (p.dim == 3) {
-    if (a.ax.cls == 0) hipLaunchKernelGGL((k_gen_axis0<0, 3>), grid, block, g.lds, stream(), a);
-    else hipLaunchKernelGGL((k_gen_axis0<1, 3>), grid, block, g.lds, stream(), a);
-  } else {
-    if (a.ax.cls == 0) hipLaunchKernelGGL((k_gen_axis0<0, 2>), grid, block, g.lds, stream(), a);
-    else hipLaunchKernelGGL((k_gen_axis0<1, 2>), grid, block, g.lds, stream(), a);
-  }
+  auto go = [&](auto dim, auto pk) {
+    constexpr int D = decltype(dim)::value;
+    constexpr bool K = decltype(pk)::value;
+    if (a.ax.cls == 0) hipLaunchKernelGGL((k_gen_axis0<0, D, K>), grid, block, g.lds, stream(), a);
+    else hipLaunchKernelGGL((k_gen_axis0<1, D, K>), grid, block, g.lds, stream(), a);
+  };
+  using D2 = std::integral_constant<int, 2>;
+  using D3 = std::integral_constant<int, 3>;
+  if (p.dim == 3 && p.packed) go(D3{}, std::true_type{});
+  else if (p.dim == 3) go(D3{}, std::false_type{});
+  else if (p.packed) go(D2{}, std::true_type{});
+  else go(D2{}, std::false_type{});
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }

@@ -37,10 +37,10 @@ struct GLast {
 // values per point].  The updated p of two rows is staged as it lies in memory
 // and read back a voxel per thread (a lane stride of NC doubles, odd in 3D: no
 // bank conflict), so that r, p are read and p is written in full cache lines.
-template <int CLS, int DIM, int IN>
+template <int CLS, int DIM, int IN, bool PK>
 __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
   if (a.active && !a.active[0]) return;
-  constexpr int NC = DIM * DIM;
+  constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x;
   double2* s = reinterpret_cast<double2*>(smem);
@@ -103,13 +103,17 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
 #pragma unroll
           for (int c = 0; c < NC; ++c) dp[c] = p[c];
         }
-        double* o = sr + 2 * (m * LS + (r0 >> 1) * NC) + r;
+        double q[NL];
+        pack_lines<double, DIM, PK>(dp, q);
+        double* o = sr + 2 * (m * LS + (r0 >> 1) * NL) + r;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) o[2 * c] = dp[c];
+        for (int c = 0; c < NL; ++c) o[2 * c] = q[c];
       }
     };
     if constexpr (IN == IN_PLAIN) {
       voxels(std::integral_constant<int, -1>{});
+    } else if constexpr (PK) {
+      voxels(std::integral_constant<int, TAN_ISO>{});
     } else {
       switch (a.tan_kind) {
         case TAN_SYM: voxels(std::integral_constant<int, TAN_SYM>{}); break;
@@ -126,10 +130,10 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
   gen_fft<double, CLS, -1, false, false>(a.ax, a.P, p, p < a.P, s + l, LS, tw, none_ld, none_st);
   for (int r = 0; r < a.RB; ++r) {
     if (row0 + r >= a.rows) break;
-    double2* o = a.spec + (row0 + r) * nh * NC;
-    const double2* sl = s + (r >> 1) * NC;
-    for (int e = threadIdx.x; e < nh * NC; e += NT) {
-      const int k = e / NC, c = e - k * NC;
+    double2* o = a.spec + (row0 + r) * nh * NL;
+    const double2* sl = s + (r >> 1) * NL;
+    for (int e = threadIdx.x; e < nh * NL; e += NT) {
+      const int k = e / NL, c = e - k * NL;
       const double2 z = sl[k * LS + c], zc = sl[(k == 0 ? 0 : n - k) * LS + c];
       double2 X;
       if (!(r & 1)) {
@@ -151,20 +155,20 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
 // LDS: [lines][twiddles]; the half lines of a workgroup are staged over the
 // lines, combined through registers (kGenVals values per thread at most, which
 // P guarantees) and transformed in place.
-template <int CLS, int DIM, int OUT>
+template <int CLS, int DIM, int OUT, bool PK>
 __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   if (a.active && !a.active[0]) return;
-  constexpr int NC = DIM * DIM;
+  constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[16];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x, RB = a.RB;
   double2* s = reinterpret_cast<double2*>(smem);
-  const int stage = RB * nh * NC;  // staged values; the twiddles follow the larger of the two
+  const int stage = RB * nh * NL;  // staged values; the twiddles follow the larger of the two
   double2* tw = s + (n * LS > stage ? n * LS : stage);
   gen_twiddles<double>(tw, a.tw, n);
   const int64_t row0 = (int64_t)blockIdx.x * RB;
   {
-    const int64_t base = row0 * nh * NC, lim = a.rows * nh * NC;
+    const int64_t base = row0 * nh * NL, lim = a.rows * nh * NL;
     constexpr int KB = 4;
     for (int e0 = 0; e0 < stage; e0 += KB * NT) {
       double2 t[KB];
@@ -184,16 +188,16 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
   const bool act = p < a.P;
   {
-    const int rp = l / NC, c = l - rp * NC;
-    const double2* A0 = s + (2 * rp) * nh * NC + c;
-    const double2* B0 = A0 + nh * NC;
+    const int rp = l / NL, c = l - rp * NL;
+    const double2* A0 = s + (2 * rp) * nh * NL + c;
+    const double2* B0 = A0 + nh * NL;
     double2 v[kGenVals];
 #pragma unroll
     for (int i = 0; i < kGenVals; ++i) {
       const int m = p + i * a.P;
       if (act && m < n) {
         const int kk = m < nh ? m : n - m;
-        double2 A = A0[kk * NC], B = B0[kk * NC];
+        double2 A = A0[kk * NL], B = B0[kk * NL];
         if (kk == 0 || 2 * kk == n) A.y = B.y = 0.0;
         if (m >= nh) {
           A.y = -A.y;
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   for (int r = 0; r < RB; ++r) {
     if (row0 + r >= a.rows) break;
     const int64_t base = (row0 + r) * n * NC;
-    const double* sl = sr + 2 * ((r >> 1) * NC) + (r & 1);
+    const double* sl = sr + 2 * ((r >> 1) * NL) + (r & 1);
     const int tot = n * NC;
     constexpr int KB = 4;
     for (int e0 = 0; e0 < tot; e0 += KB * NT) {
@@ -238,7 +242,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
         const int e = e0 + i * NT + threadIdx.x;
         if (e < tot) {
           const int m = e / NC, c = e - m * NC;
-          const double val = sl[2 * (m * LS + c)];
+          const double val = sl[2 * (m * LS + line_of<DIM, PK>(c))];
           if (OUT == OUT_RUPD) {
             const double rv = dv[i] + al * val;
             a.out[base + e] = rv;
@@ -282,54 +286,63 @@ void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a)
   a.active = p.active;
 }
 
-template <int CLS, int DIM>
+template <int CLS, int DIM, bool PK>
 int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
-  const GenShape& g = p.gen_last;
+  const GenShape& g = p.gen_last[PK ? 1 : 0];
   GLast a{};
   fill(p, op, spec, g, a);
   if (!op.fin_alpha) a.partials = nullptr;
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  p.wg_r2c = grid.x;
   if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
   switch (op.in_mode) {
-    case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN>), grid, block, g.lds, stream(), a); break;
-    case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN>), grid, block, g.lds, stream(), a); break;
+    case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a); break;
+    case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN, PK>), grid, block, g.lds, stream(), a); break;
     default:
-      if (op.xvec) hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE_X>), grid, block, g.lds, stream(), a);
-      else hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE>), grid, block, g.lds, stream(), a);
+      if (op.xvec) hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE_X, PK>), grid, block, g.lds, stream(), a);
+      else hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE, PK>), grid, block, g.lds, stream(), a);
       break;
   }
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }
 
-template <int CLS, int DIM>
+template <int CLS, int DIM, bool PK>
 int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
-  const GenShape& g = p.gen_last;
+  const GenShape& g = p.gen_last[PK ? 1 : 0];
   GLast a{};
   fill(p, op, spec, g, a);
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  p.wg_c2r = grid.x;
   if (op.out_mode == OUT_RUPD)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds, stream(), a);
   else if (op.out_mode == OUT_DOT)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT, PK>), grid, block, g.lds, stream(), a);
   else
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds, stream(), a);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
+}
+
+template <int DIM, bool PK>
+int r2c_cls(FftPlan& p, const OpSpec& op, void* spec) {
+  return p.gen[DIM - 1].cls ? r2c_launch<1, DIM, PK>(p, op, spec) : r2c_launch<0, DIM, PK>(p, op, spec);
+}
+template <int DIM, bool PK>
+int c2r_cls(FftPlan& p, const OpSpec& op, void* spec) {
+  return p.gen[DIM - 1].cls ? c2r_launch<1, DIM, PK>(p, op, spec) : c2r_launch<0, DIM, PK>(p, op, spec);
 }
 
 }  // namespace
 
 int gen_r2c(FftPlan& p, const OpSpec& op, void* spec) {
-  const bool c1 = p.gen[p.dim - 1].cls != 0;
-  if (p.dim == 3) return c1 ? r2c_launch<1, 3>(p, op, spec) : r2c_launch<0, 3>(p, op, spec);
-  return c1 ? r2c_launch<1, 2>(p, op, spec) : r2c_launch<0, 2>(p, op, spec);
+  if (p.packed) return p.dim == 3 ? r2c_cls<3, true>(p, op, spec) : r2c_cls<2, true>(p, op, spec);
+  return p.dim == 3 ? r2c_cls<3, false>(p, op, spec) : r2c_cls<2, false>(p, op, spec);
 }
 
 int gen_c2r(FftPlan& p, const OpSpec& op, void* spec) {
-  const bool c1 = p.gen[p.dim - 1].cls != 0;
-  if (p.dim == 3) return c1 ? c2r_launch<1, 3>(p, op, spec) : c2r_launch<0, 3>(p, op, spec);
-  return c1 ? c2r_launch<1, 2>(p, op, spec) : c2r_launch<0, 2>(p, op, spec);
+  if (p.packed) return p.dim == 3 ? c2r_cls<3, true>(p, op, spec) : c2r_cls<2, true>(p, op, spec);
+  return p.dim == 3 ? c2r_cls<3, false>(p, op, spec) : c2r_cls<2, false>(p, op, spec);
 }
 
 }  // namespace mugpu

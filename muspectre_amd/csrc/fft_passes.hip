@@ -508,27 +508,29 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
   // solve, single points and the longest axes
   for (int d = 0; d < dim; ++d) {
     if (!general || p.fastax[d] || !gen_radices(res[d], p.gen[d])) continue;
-    int64_t inner = nc, outer = 1;
+    int64_t inner = 1, outer = 1;
     for (int k = d + 1; k < dim; ++k) inner *= p.hres[k];
     for (int k = 0; k < d; ++k) outer *= p.hres[k];
-    if (d == dim - 1) p.gen_last = gen_last_shape(p.gen[d], nc, rows);
-    else p.gen_str[d] = gen_strided_shape(p.gen[d], inner, outer);
-    p.genax[d] = d == dim - 1 ? p.gen_last.NT > 0 : p.gen_str[d].NT > 0;
-    if (d == 0) {
-      p.gen_axis0 = gen_axis0_shape(p.gen[d], nc, p.kpts / res[0]);
-      p.genax[d] = p.genax[d] && p.gen_axis0.NT > 0;
+    p.genax[d] = true;
+    for (int pk = 0; pk < 2; ++pk) {
+      const int nl = pk ? dim * (dim + 1) / 2 : nc;
+      if (d == dim - 1) p.gen_last[pk] = gen_last_shape(p.gen[d], nc, nl, rows);
+      else p.gen_str[d][pk] = gen_strided_shape(p.gen[d], inner * nl, outer);
+      if (d == 0) p.gen_axis0[pk] = gen_axis0_shape(p.gen[d], nl, p.kpts / res[0]);
+      p.genax[d] = p.genax[d] && (d == dim - 1 || p.gen_str[d][pk].NT > 0) &&
+                   (d < dim - 1 || p.gen_last[pk].NT > 0) && (d > 0 || p.gen_axis0[pk].NT > 0);
     }
   }
+  p.general = general;
+  p.can_pack = true;
+  for (int d = 0; d < dim; ++d)
+    p.can_pack = p.can_pack && (p.fastax[d] || p.genax[d] || (d > 0 && d < dim - 1 && res[d] == 1));
   if (p.fastax[dim - 1]) {
     for (int pr = 0; pr < 2; ++pr) {
       const int rb = fast_rows_per_block(n, dim, p.fvar[pr][FV_C2R][0]);
       p.nzb[pr] = (rows + rb - 1) / rb;
     }
     p.zrb = fast_rows_per_block(n, dim, 0);
-    for (int iso = 0; iso < 2; ++iso) {
-      const int rb = fast_rows_per_block(n, dim, p.fvar[0][FV_R2C][iso]);
-      p.nzr[iso] = (rows + rb - 1) / rb;
-    }
   } else {
     if (!fits((nc + 1) / 2, n, kNT)) {
       set_error("last axis of %d points exceeds the supported line length", n);
@@ -545,10 +547,7 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
     p.zrb = rb;
   }
   if (!p.fastax[dim - 1]) p.nzb[0] = p.nzb[1] = (rows + p.zrb - 1) / p.zrb;
-  if (p.genax[dim - 1]) {
-    const int rb = 2 * p.gen_last.mult;
-    p.nzb[0] = p.nzr[0] = p.nzr[1] = (rows + rb - 1) / rb;
-  }
+  if (p.genax[dim - 1]) p.nzb[0] = (rows + 1) / 2;  // at most: a pair of rows per workgroup
   p.nzblocks = p.nzb[0] > p.nzb[1] ? p.nzb[0] : p.nzb[1];
   // strided middle axis: up to 16 lines (256 B rows in FP64)
   if (dim == 3 && !p.fastax[1]) {
@@ -687,6 +686,7 @@ int launch_c2r(FftPlan& p, const OpSpec& op, c_t<T>* spec) {
   a.rows = p.N / n;
   a.active = p.active;
   a.rb = p.zrb;
+  p.wg_c2r = (a.rows + a.rb - 1) / a.rb;
   a.ls = odd_stride(n);
   a.ap = p.ax[DIM - 1];
   a.tw = tw_of<T>(p, DIM - 1);
@@ -710,7 +710,7 @@ template <typename T>
 int launch_strided(FftPlan& p, int ax, int W, c_t<T>* spec, int sign) {
   SArgs<T> a{};
   a.data = spec;
-  int64_t inner = p.nc;
+  int64_t inner = p.lines();
   for (int d = ax + 1; d < p.dim; ++d) inner *= p.hres[d];
   int64_t outer = 1;
   for (int d = 0; d < ax; ++d) outer *= p.hres[d];
@@ -799,10 +799,13 @@ int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spec
   const bool carried = p.fastax[DIM - 1] || (sizeof(T) == 8 && p.genax[DIM - 1]);
   if (op.xvec && !carried) return MUGPU_EARG;
   if ((op.fin_alpha || op.out_mode == OUT_RUPD) && (sizeof(T) != 8 || !carried)) return MUGPU_EARG;
+  p.packed = sizeof(T) == 8 && p.can_pack && pj.kind == MUGPU_PROJ_SMALL_STRAIN &&
+             (op.in_mode == IN_PLAIN || op.tan_kind == TAN_ISO) &&
+             (p.general || op.out_mode != OUT_PLAIN);
   MUGPU_TRY((launch_r2c<T, DIM>(p, op, spec)));
   if (op.fin_alpha)
-    MUGPU_TRY(finalize((const double*)p.partials, p.nzr[op.tan_kind == TAN_ISO ? 1 : 0], op.fin_alpha,
-                       FIN_ALPHA, const_cast<int*>(p.active)));
+    MUGPU_TRY(finalize((const double*)p.partials, p.wg_r2c, op.fin_alpha, FIN_ALPHA,
+                       const_cast<int*>(p.active)));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, -1));
   if (pj.kind >= 0) {
     MUGPU_TRY((launch_project<T, DIM>(p, pj, spec)));
@@ -820,6 +823,7 @@ int r2c_impl(FftPlan& p, const void* in, void* spectrum) {
   OpSpec op;
   op.in_mode = IN_PLAIN;
   op.in = in;
+  p.packed = false;
   MUGPU_TRY((launch_r2c<T, DIM>(p, op, spec)));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, -1));
   return launch_strided<T>(p, 0, p.xW, spec, -1);
@@ -828,6 +832,7 @@ int r2c_impl(FftPlan& p, const void* in, void* spectrum) {
 template <typename T, int DIM>
 int c2r_impl(FftPlan& p, void* spectrum, void* out) {
   c_t<T>* spec = reinterpret_cast<c_t<T>*>(spectrum);
+  p.packed = false;
   MUGPU_TRY(launch_strided<T>(p, 0, p.xW, spec, +1));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, +1));
   OpSpec op;

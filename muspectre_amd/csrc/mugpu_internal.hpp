@@ -139,8 +139,9 @@ struct GenShape {
   size_t lds = 0;
 };
 bool gen_radices(int n, GenAxis& ax);
-GenShape gen_last_shape(const GenAxis& ax, int nc, int64_t rows);
-GenShape gen_axis0_shape(const GenAxis& ax, int nc, int64_t plane);
+// (nc components per point, nl lines per row or k-point)
+GenShape gen_last_shape(const GenAxis& ax, int nc, int nl, int64_t rows);
+GenShape gen_axis0_shape(const GenAxis& ax, int nl, int64_t plane);
 GenShape gen_strided_shape(const GenAxis& ax, int64_t inner, int64_t outer);
 
 // Workgroups are dispatched to the 8 XCDs round robin (workgroup b runs on
@@ -170,14 +171,20 @@ struct FftPlan {
   int xWk = 1;     // fused axis-0 projection pass: k-points per workgroup
   int xNT = 256;   // threads of the fused pass
   void* partials = nullptr;  // double per z-pass workgroup
-  int64_t nzr[2] = {0, 0};   // r2c workgroups of FP64 (p.Kp partials): full, isotropic tangent
+  int64_t wg_r2c = 0, wg_c2r = 0;  // workgroups of the latest FP64 last-axis launches (their partials)
   int64_t nzblocks = 0;      // z-pass workgroups, the largest of nzb
   int64_t nzb[2] = {0, 0};   // c2r workgroups (p.Ap partials) per precision (0 FP64, 1 FP32)
   bool fastax[3] = {false, false, false};  // compile-time-length passes (fft_fast.hip)
   // run-time-length passes of FP64 grids, per axis (genax: the axis has them)
   GenAxis gen[3];
   bool genax[3] = {false, false, false};
-  GenShape gen_last, gen_axis0, gen_str[3];
+  GenShape gen_last[2], gen_axis0[2], gen_str[3][2];  // one line per component; packed
+  // packed symmetric lines (op_stages.hpp) of FP64 small-strain operators: every
+  // axis has a pass that takes them (can_pack), whether the plan's own operators
+  // use them too or only the CG iterations (general, plan_init), and whether
+  // the run in hand does (packed)
+  bool general = true, can_pack = false, packed = false;
+  int lines() const { return packed ? dim * (dim + 1) / 2 : nc; }
   // variant of each compile-time-length pass (bit 0: 8 values per thread
   // instead of 16 or 12; bit 1: half the rows or k-points per workgroup, for
   // the last-axis and first-axis projection passes), per precision (0 FP64,
@@ -200,7 +207,8 @@ void force_variant(int pass, int prec, int variant);
 // this length, dimension and precision
 bool fast_variant_valid(int pass, int n, int dim, int prec, int variant);
 
-// general: FP64 passes of run-time length where they fit.  Cells of the
+// general: FP64 passes of run-time length where they fit, packed symmetric
+// lines.  Cells of the
 // FP32-refined solve go without: their x carries the FP32 rounding of its
 // inner solves (1.5e-6 relative), so a last-bit change of the FP64 residuals
 // would move their results by that much

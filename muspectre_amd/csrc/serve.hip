@@ -421,7 +421,7 @@ int mugpu_server_s::class_of(Request* r) {
   c->dim = r->dim;
   for (int d = 0; d < 3; ++d) c->res[d] = r->res[d];
   c->N = r->N;
-  MUGPU_TRY(plan_init(c->plan, r->dim, r->res, r->nc, MUGPU_FP32));
+  MUGPU_TRY(plan_init(c->plan, r->dim, r->res, r->nc, MUGPU_FP32, false));
   const int cap = cfg.max_batch;
   MUGPU_TRY(dev_alloc(&c->d_slots, sizeof(BatchSlot) * cap, "the batch slots"));
   MUGPU_TRY(dev_alloc(&c->d_ctl, sizeof(int) * CTL_COUNT * cap, "the batch control words"));

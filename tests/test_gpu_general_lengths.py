@@ -75,10 +75,13 @@ def test_transforms_vs_numpy(capi, res):
 
 
 @pytest.mark.parametrize("form", [0, 1], ids=["finite", "small"])
-@pytest.mark.parametrize("res", [[51, 38], [23, 7], [15, 22, 9], [9, 26, 13], [19, 6, 17]],
+@pytest.mark.parametrize("res", [[51, 38], [23, 7], [15, 22, 9], [9, 26, 13], [19, 6, 17],
+                                 # compiled last axis under an odd number of rows
+                                 [5, 7, 16], [3, 5, 96], [9, 512], [7, 256]],
                          ids=lambda r: "x".join(map(str, r)))
 def test_operator_vs_oracle(capi, oracle, res, form):
-    """G:(K:dF) through every pass of a cell; the bound of the other operator
+    """G:(K:dF) through every pass of a cell (small strain: packed symmetric
+    lines, of a dF that is not symmetric); the bound of the other operator
     tests, 1e-12 of the largest value."""
     from test_gpu_abi_cell import GpuCell
     d, N = len(res), int(np.prod(res))
@@ -103,3 +106,7 @@ def test_operator_vs_oracle(capi, oracle, res, form):
     bi, bo = DeviceBuffer.from_array(dF), DeviceBuffer(dF.nbytes)
     capi.check(gc.lib.mugpu_cell_directional_stiffness(gc.h, bi.ptr, bo.ptr))
     assert np.abs(bo.download(dF.shape) - ref).max() <= 1e-12 * np.abs(ref).max()
+    # the projection alone
+    refG = oc.apply_projection(dF.copy())
+    capi.check(gc.lib.mugpu_cell_apply_projection(gc.h, bi.ptr))
+    assert np.abs(bi.download(dF.shape) - refG).max() <= 1e-12 * np.abs(refG).max()
