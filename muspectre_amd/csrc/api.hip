@@ -1519,8 +1519,12 @@ extern "C" int mugpu_cg_step(mugpu_cell c, int update_p, void* d_x, void* d_r, v
     op.out_mode = OUT_RUPD;
     op.out = d_r;
     op.ap_out = d_Ap;
+    if (c->plan.fold_ok) op.fold_pk = c->partials;
     MUGPU_TRY(run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum));
-    MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA));
+    if (op.fold_pk)
+      MUGPU_TRY(fold_beta((const double*)c->plan.partials, (int)c->plan.wg_c2r, c->scal, nullptr, 1));
+    else
+      MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA));
     MUGPU_TRY(axpy_alpha(MUGPU_FP64, d_x, d_p, c->scal, n));
   } else {
     op.out_mode = OUT_DOT;
@@ -1553,6 +1557,7 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
     op.fin_alpha = c->scal;
     op.out_mode = OUT_RUPD;
     op.out = d_r;
+    if (c->plan.fold_ok) op.fold_pk = c->partials;
   } else {
     op.out_mode = OUT_DOT;
     op.out = d_Ap;
@@ -1577,7 +1582,12 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
   auto queue = [&](int i) -> int {
     op.in_mode = (i > 0 || update_p) ? IN_TAN_PUPDATE : IN_TAN;
     op.xvec = fuse && (i > 0 || pend_here) ? d_x : nullptr;
+    op.fold_iter = i;
     int e = run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum);
+    if (op.fold_pk)
+      return e != MUGPU_OK || i + 1 < max_steps
+                 ? e
+                 : fold_beta((const double*)c->plan.partials, (int)c->plan.wg_c2r, c->scal, c->ctl, max_steps);
     if (early)
       return e != MUGPU_OK ? e
                            : finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA,

@@ -239,6 +239,27 @@ inline unsigned grid_for(int64_t n, int cap = kRedGrid) {
   return (unsigned)g;
 }
 
+__global__ __launch_bounds__(64) void k_fold_beta(const double* __restrict__ rr, int count, double* scal,
+                                                  int* ctl, int iters) {
+  __shared__ double red[1];
+  if (ctl && !ctl[CTL_ACTIVE]) {
+    // stopped by an earlier iteration's test
+    if (threadIdx.x == 0) scal[SC_RDR] = scal[SC_NEWRDR];
+    return;
+  }
+  const double s = fold_sum(rr, count, red);
+  if (threadIdx.x == 0) {
+    const double old = scal[(iters - 1) & 1 ? SC_RDR1 : SC_RDR];
+    scal[SC_NEWRDR] = s;
+    scal[SC_BETA] = s / old;
+    scal[SC_RDR] = s;
+    if (ctl) {
+      if (s == s) ctl[CTL_ITER] = iters;
+      ctl[CTL_ACTIVE] = 0;
+    }
+  }
+}
+
 __global__ void k_scal_copy(double* scal, int from, int to) {
   if (threadIdx.x == 0) scal[to] = scal[from];
 }
@@ -496,6 +517,13 @@ int axpy_alpha(int prec, void* x, const void* p, const double* d_scal, int64_t n
   else
     hipLaunchKernelGGL((k_axpy_alpha<float>), dim3(g), dim3(kRT), 0, stream(), (float*)x,
                        (const float*)p, d_scal, n, slot);
+  MUGPU_HIP(hipGetLastError());
+  return MUGPU_OK;
+}
+
+int fold_beta(const double* rr, int count, double* d_scal, int* ctl, int iters) {
+  if (count < 1 || count > kFoldMax) return MUGPU_EARG;
+  hipLaunchKernelGGL(k_fold_beta, dim3(1), dim3(64), 0, stream(), rr, count, d_scal, ctl, iters);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }

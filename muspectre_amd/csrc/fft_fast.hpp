@@ -428,6 +428,7 @@ struct LArgs {
   const int* active;  // FftPlan::active (single-cell kernels only)
   T* x;               // OpSpec::xvec (IN_TAN_PUPDATE_X kernels only)
   T* ap;              // OpSpec::ap_out (OUT_RUPD kernels only)
+  ScalarFold fold;    // (FP64)
 };
 
 // ISO: the tangent is known to be isotropic (TAN_ISO), which the compiler
@@ -446,7 +447,14 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
     // registers, and the lines take the place of the staged rows
     static_assert(IN == IN_PLAIN || ISO, "packed lines need a symmetric K : p");
     constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
-    const T beta = PU ? (T)a.scal[SC_BETA] : T(0);
+    T beta = PU ? (T)a.scal[SC_BETA] : T(0);
+    if constexpr (sizeof(T) == 8 && PU) {
+      if (a.fold.rr) {
+        const double rr = fold_sum(a.fold.rr, a.fold.nrr, reinterpret_cast<double*>(smem));
+        if (!fold_beta_test(a.fold, rr, beta)) return;
+        __syncthreads();
+      }
+    }
     const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
     constexpr int TOT = RB * N * NC, kBatch = 8;
     const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
@@ -525,7 +533,14 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
     constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X;
     // the previous iteration's x update, x += alpha p_old, when fused here
     constexpr bool XU = IN == IN_TAN_PUPDATE_X;
-    const T beta = PU ? (T)a.scal[SC_BETA] : T(0);
+    T beta = PU ? (T)a.scal[SC_BETA] : T(0);
+    if constexpr (sizeof(T) == 8 && PU) {
+      if (a.fold.rr) {
+        const double rr = fold_sum(a.fold.rr, a.fold.nrr, reinterpret_cast<double*>(smem));
+        if (!fold_beta_test(a.fold, rr, beta)) return;
+        __syncthreads();
+      }
+    }
     const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
     {
       constexpr int TOT = RB * N * NC, kBatch = 8;
@@ -681,6 +696,13 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   constexpr int NT = L * (N / E), NH = N / 2 + 1;
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   const int64_t row0 = bx * RB;
+  T alpha = T(0);
+  if constexpr (sizeof(T) == 8 && OUT == OUT_RUPD) {
+    if (a.fold.pk) {
+      alpha = fold_alpha(a.fold, fold_sum(a.fold.pk, a.fold.npk, reinterpret_cast<double*>(smem)));
+      __syncthreads();
+    }
+  }
   {
     // loads issued in batches of kBatch before their LDS stores, so that each
     // thread keeps several HBM requests in flight
@@ -738,7 +760,7 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   const T* sr = reinterpret_cast<const T*>(smem);
   const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
   double acc = 0.0;
-  const T al = OUT == OUT_RUPD ? (T)a.scal[SC_ALPHA] : T(0);
+  const T al = OUT != OUT_RUPD ? T(0) : a.fold.pk ? alpha : (T)a.scal[SC_ALPHA];
   {
     constexpr int TOT = RB * N * NC, kBatch = 8;
     for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {

@@ -30,6 +30,7 @@ int c2r_n(FftPlan& p, const OpSpec& op, void* spec) {
   if constexpr (sizeof(T) == 8) {
     a.scal = op.scal;
     a.ap = reinterpret_cast<T*>(op.ap_out);
+    a.fold = p.fold;
     if (p.packed) {
       if (op.out_mode == OUT_RUPD) c2r_go<T, N, E, DIM, OUT_RUPD, H, true>(p, a);
       else if (op.out_mode == OUT_DOT) c2r_go<T, N, E, DIM, OUT_DOT, H, true>(p, a);

@@ -32,6 +32,10 @@ int r2c_n(FftPlan& p, const OpSpec& op, void* spec) {
   a.active = p.active;
   a.x = reinterpret_cast<T*>(op.xvec);
   a.partials = op.fin_alpha ? reinterpret_cast<double*>(p.partials) : nullptr;
+  if (sizeof(T) == 8) {
+    a.fold = p.fold;
+    if (a.fold.pk) a.partials = a.fold.pk;
+  }
   const bool iso = op.tan_kind == TAN_ISO;
   // the fused x update goes with the p update only
   const bool xu = op.xvec != nullptr;

@@ -96,8 +96,20 @@ GenShape gen_last_shape(const GenAxis& ax, int nc, int nl, int64_t rows) {
     const size_t half = (size_t)2 * mult * (n / 2 + 1) * nl * 16;
     const size_t bwd = (lines > half ? lines : half) + tw;
     g.mult = mult;
-    g.lds = fwd > bwd ? fwd : bwd;
-    if (g.lds > kGenMaxLds) break;
+    // threads beyond the transforms' share the sweeps over the staged rows
+    // (four values each): up to 256 where the grid leaves the chip idle anyway
+    // (33x27x35: r2c 22.6 -> 16.0, c2r 10.6 -> 8.9 us), else only in the r2c
+    // pass, which stages most, and at most twice as many (125^3: 144 -> 128 us;
+    // four times as many cost 22.5 -> 26.0 us at 63^3)
+    const bool idle = rows / (2 * mult) < 1024;
+    int sweep = (2 * n * nc / 4 + 63) / 64 * 64;
+    if (sweep > kGenThreads) sweep = kGenThreads;
+    g.NT_bwd = idle && sweep > g.NT ? sweep : g.NT;
+    if (!idle && sweep > 2 * g.NT) sweep = 2 * g.NT;
+    if (sweep > g.NT) g.NT = sweep;
+    g.lds = fwd;
+    g.lds_bwd = bwd;
+    if (fwd > kGenMaxLds || bwd > kGenMaxLds) break;
     if (mult > 1 && (g.lds > kGenLds || L > 40 || rows / (2 * mult) < 1024)) break;
     best = g;
   }

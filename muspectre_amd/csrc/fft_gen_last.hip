@@ -31,6 +31,7 @@ struct GLast {
   GenAxis ax;
   const double2* tw;
   const int* active;  // FftPlan::active
+  ScalarFold fold;
 };
 
 // LDS: [lines: n * LS complex][twiddles: n complex][staging: 2 rows of NC
@@ -39,7 +40,6 @@ struct GLast {
 // bank conflict), so that r, p are read and p is written in full cache lines.
 template <int CLS, int DIM, int IN, bool PK>
 __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
-  if (a.active && !a.active[0]) return;
   constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x;
@@ -48,10 +48,13 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
   __shared__ double red[16];
   double2* tw = s + n * LS;
   double* sp = reinterpret_cast<double*>(tw + n);
-  gen_twiddles<double>(tw, a.tw, n);
+  // (the flag and the partial sums are read together)
+  const int on = a.active ? a.active[0] : 1;
   const int64_t row0 = (int64_t)blockIdx.x * a.RB;
   constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
-  const double beta = PU ? a.scal[SC_BETA] : 0.0;
+  double beta = PU ? a.scal[SC_BETA] : 0.0;
+  const double rr = PU && a.fold.rr ? fold_sum(a.fold.rr, a.fold.nrr, red) : 0.0;
+  if (!on || (PU && a.fold.rr && !fold_beta_test(a.fold, rr, beta))) return;
   const double al = XU ? a.scal[SC_ALPHA] : 0.0;
   double acc = 0.0;  // p . K p
   for (int r0 = 0; r0 < a.RB; r0 += 2) {
@@ -86,6 +89,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
         }
       }
     }
+    if (r0 == 0) gen_twiddles<double>(tw, a.tw, n);
     __syncthreads();
     // rows beyond the last one hold zeros, for which K : p is not evaluated
     auto voxels = [&](auto kind_c) {
@@ -157,7 +161,6 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
 // P guarantees) and transformed in place.
 template <int CLS, int DIM, int OUT, bool PK>
 __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
-  if (a.active && !a.active[0]) return;
   constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[16];
@@ -165,7 +168,11 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   double2* s = reinterpret_cast<double2*>(smem);
   const int stage = RB * nh * NL;  // staged values; the twiddles follow the larger of the two
   double2* tw = s + (n * LS > stage ? n * LS : stage);
-  gen_twiddles<double>(tw, a.tw, n);
+  const int on = a.active ? a.active[0] : 1;
+  const bool fold = OUT == OUT_RUPD && a.fold.pk;
+  const double pk = fold ? fold_sum(a.fold.pk, a.fold.npk, red) : 0.0;
+  if (!on) return;
+  const double alpha = fold ? fold_alpha(a.fold, pk) : 0.0;
   const int64_t row0 = (int64_t)blockIdx.x * RB;
   {
     const int64_t base = row0 * nh * NL, lim = a.rows * nh * NL;
@@ -184,6 +191,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
       }
     }
   }
+  gen_twiddles<double>(tw, a.tw, n);
   __syncthreads();
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
   const bool act = p < a.P;
@@ -219,7 +227,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   auto none_st = [](int, double2) {};
   gen_fft<double, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
   const double* sr = reinterpret_cast<const double*>(smem);
-  const double al = OUT == OUT_RUPD ? a.scal[SC_ALPHA] : 0.0;
+  const double al = OUT != OUT_RUPD ? 0.0 : fold ? alpha : a.scal[SC_ALPHA];
   double acc = 0.0;
   for (int r = 0; r < RB; ++r) {
     if (row0 + r >= a.rows) break;
@@ -284,6 +292,7 @@ void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a)
   a.ax = p.gen[d];
   a.tw = static_cast<const double2*>(p.tw64[d]);
   a.active = p.active;
+  a.fold = p.fold;
 }
 
 template <int CLS, int DIM, bool PK>
@@ -294,6 +303,7 @@ int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
   if (!op.fin_alpha) a.partials = nullptr;
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
   p.wg_r2c = grid.x;
+  if (a.fold.pk) a.partials = a.fold.pk;
   if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
   switch (op.in_mode) {
     case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a); break;
@@ -312,14 +322,14 @@ int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
   const GenShape& g = p.gen_last[PK ? 1 : 0];
   GLast a{};
   fill(p, op, spec, g, a);
-  const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
+  const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT_bwd);
   p.wg_c2r = grid.x;
   if (op.out_mode == OUT_RUPD)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds_bwd, stream(), a);
   else if (op.out_mode == OUT_DOT)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT, PK>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT, PK>), grid, block, g.lds_bwd, stream(), a);
   else
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds, stream(), a);
+    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds_bwd, stream(), a);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }

@@ -592,6 +592,7 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
     const int rbmin = fast_rows_per_block(res[dim - 1], dim, 2);
     nzmax = (p.N / res[dim - 1] + rbmin - 1) / rbmin;
   }
+  p.fold_ok = nzmax <= kFoldMax;
   MUGPU_TRY(dev_alloc(&p.partials, sizeof(double) * (size_t)(nzmax > kRedBlocks ? nzmax : kRedBlocks),
                       "the transform's partial sums"));
   return MUGPU_OK;
@@ -802,8 +803,21 @@ int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spec
   p.packed = sizeof(T) == 8 && p.can_pack && pj.kind == MUGPU_PROJ_SMALL_STRAIN &&
              (op.in_mode == IN_PLAIN || op.tan_kind == TAN_ISO) &&
              (p.general || op.out_mode != OUT_PLAIN);
+  p.fold = ScalarFold{};
+  if (op.fin_alpha && op.fold_pk) {
+    p.fold.pk = op.fold_pk;
+    p.fold.iter = op.fold_iter;
+    p.fold.ctl = const_cast<int*>(p.active);
+    p.fold.scal = op.fin_alpha;
+    if (op.fold_iter > 0) {
+      p.fold.rr = (const double*)p.partials;
+      p.fold.nrr = (int)p.wg_c2r;
+    }
+  }
   MUGPU_TRY((launch_r2c<T, DIM>(p, op, spec)));
-  if (op.fin_alpha)
+  p.fold.rr = nullptr;
+  p.fold.npk = (int)p.wg_r2c;
+  if (op.fin_alpha && !op.fold_pk)
     MUGPU_TRY(finalize((const double*)p.partials, p.wg_r2c, op.fin_alpha, FIN_ALPHA,
                        const_cast<int*>(p.active)));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, -1));

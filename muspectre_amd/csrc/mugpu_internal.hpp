@@ -107,8 +107,30 @@ __host__ __device__ constexpr int sym_index(int r, int c, int n) {
 // SC_TOL2: squared stopping threshold of a batched inner CG
 // SC_XALPHA: alpha of a pending x update (kept apart from SC_ALPHA, which
 // the next solve on the cell overwrites)
+// SC_RDR1: with SC_RDR, the r . r of alternate iterations of a chunk whose
+// scalars are folded into the passes (ScalarFold)
 enum Scalar { SC_RDR = 0, SC_PAP, SC_ALPHA, SC_NEWRDR, SC_BETA, SC_TMP0, SC_TMP1, SC_TOL2,
-              SC_XALPHA, SC_COUNT };
+              SC_XALPHA, SC_RDR1, SC_COUNT };
+
+// Scalars of an FP64 CG iteration without kernels of their own, for grids whose
+// passes have at most kFoldMax workgroups: every workgroup of the c2r pass sums
+// the first pass's partials of p . K p itself (alpha), and every workgroup of
+// the next r2c pass the c2r pass's partials of r . r (beta and the loop test);
+// workgroup 0 stores what the host and the later kernels read.  A pass that
+// waits for a chunk's previous kernel anyway then costs a few hundred ns more
+// instead of a launch of 4 to 5 us; with more partials than kFoldMax the
+// redundant reads cost more than that, and k_finalize runs.  All of them sum in
+// one order (fold_sum), so any mixture gives the same bits.
+struct ScalarFold {
+  double* pk = nullptr;  // partials of p . K p (r2c writes, c2r sums); null: not folded
+  const double* rr = nullptr;  // r2c: partials of r . r to sum; null: beta is in the scalar block
+  int nrr = 0;                 // their number
+  int npk = 0;                 // c2r: number of p . K p partials
+  int iter = 0;                // iterations of the chunk already run
+  int* ctl = nullptr;          // CTL_* words (r2c with rr)
+  double* scal = nullptr;
+};
+constexpr int kFoldMax = 1024;
 
 // ---- passes of run-time length (FP64; fft_gen.hpp) -------------------------------
 constexpr int kGenMaxPass = 12;
@@ -135,8 +157,8 @@ struct GenAxis {
 // shape of a workgroup: `mult` row pairs or k-points, L lines, P threads per
 // line; NT = 0: the axis does not fit
 struct GenShape {
-  int mult = 0, L = 0, P = 0, NT = 0;
-  size_t lds = 0;
+  int mult = 0, L = 0, P = 0, NT = 0, NT_bwd = 0;
+  size_t lds = 0, lds_bwd = 0;  // _bwd: of the c2r pass
 };
 bool gen_radices(int n, GenAxis& ax);
 // (nc components per point, nl lines per row or k-point)
@@ -191,6 +213,8 @@ struct FftPlan {
   // 1 FP32), per pass and, for the r2c pass, per tangent (0 full matrices,
   // 1 isotropic)
   unsigned char fvar[2][5][2] = {};
+  ScalarFold fold;  // of the run in hand (operator_impl)
+  bool fold_ok = false;  // no last-axis pass of this plan has more than kFoldMax workgroups
   // while set: every pass kernel returns at once when active[0] == 0 (CG
   // iterations launched ahead of the host's stopping test)
   const int* active = nullptr;
@@ -253,6 +277,10 @@ struct OpSpec {
   // projector, so OUT_RUPD can use it and A p need not be stored
   double* fin_alpha = nullptr;
   void* ap_out = nullptr;        // OUT_RUPD: also store A p here (optional)
+  // with fin_alpha: workgroups of the latest c2r pass and the buffer for the
+  // partials of p . K p, where the scalars may be folded into the passes
+  double* fold_pk = nullptr;
+  int fold_iter = 0;             // iterations of the chunk already run; > 0: beta is folded too
 };
 
 // full operator: r2c (with input stage) -> [axis passes] -> projection ->
@@ -336,6 +364,9 @@ int axpy_alpha(int prec, void* x, const void* p, const double* d_scal, int64_t n
                int slot = SC_ALPHA);
 // scal[to] = scal[from] on the device
 int scal_copy(double* d_scal, int from, int to);
+// beta after the last iteration of a folded chunk (ctl != null: where the chunk
+// still ran; `iters` iterations of it were queued) or after a single step
+int fold_beta(const double* rr, int count, double* d_scal, int* ctl, int iters);
 // start of an FP64 solve: x = 0, r = -b, p = b; b.b into scal[SC_RDR] and
 // scal[SC_TMP0], |b - g|^2 into scal[SC_TMP1]
 int cg_start_vectors(const double* b, const double* g, double* x, double* r, double* p, int64_t n,

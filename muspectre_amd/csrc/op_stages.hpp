@@ -279,4 +279,57 @@ __device__ __forceinline__ double block_sum_waves(double v, double* red, int NT)
   return t;
 }
 
+// sum of up to kFoldMax partials by the first wavefront, in an order that does
+// not depend on the workgroup: lane l adds l, l + 64, ..., then lane halving;
+// the result is in every thread.  Every thread must call it (a barrier inside);
+// red holds one double
+__device__ __forceinline__ double fold_sum(const double* __restrict__ part, int count, double* red) {
+  if (threadIdx.x < 64) {
+    double v = 0.0;
+    for (int i0 = 0; i0 < count; i0 += 64 * 4) {
+      double t[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = i0 + 64 * k + (int)threadIdx.x;
+        t[k] = part[i < count ? i : count - 1];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (i0 + 64 * k + (int)threadIdx.x < count) v += t[k];
+    }
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_down(v, s, 64);
+    if (threadIdx.x == 0) red[0] = v;
+  }
+  __syncthreads();
+  return red[0];
+}
+
+// r2c: beta and SolverCG's loop test after the previous iteration, from the sum s
+// of its r . r partials; false: the loop has stopped (workgroup 0 says so to the
+// later kernels)
+__device__ __forceinline__ bool fold_beta_test(const ScalarFold& f, double s, double& beta) {
+  const double old = f.scal[(f.iter - 1) & 1 ? SC_RDR1 : SC_RDR];
+  const bool go = s > f.scal[SC_TOL2];  // (false for NaN)
+  beta = s / old;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    f.scal[f.iter & 1 ? SC_RDR1 : SC_RDR] = s;
+    f.scal[SC_NEWRDR] = s;
+    f.scal[SC_BETA] = beta;
+    // an iteration whose r . r is NaN is not counted here (the host does)
+    if (s == s) f.ctl[CTL_ITER] = f.iter;
+    if (!go) f.ctl[CTL_ACTIVE] = 0;
+  }
+  return go;
+}
+// c2r: alpha from the sum s of the p . K p partials
+__device__ __forceinline__ double fold_alpha(const ScalarFold& f, double s) {
+  const double al = f.scal[f.iter & 1 ? SC_RDR1 : SC_RDR] / s;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    f.scal[SC_PAP] = s;
+    f.scal[SC_ALPHA] = al;
+  }
+  return al;
+}
+
 }  // namespace mugpu
