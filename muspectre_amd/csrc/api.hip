@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "mugpu_internal.hpp"
+#include "op_stages.hpp"
 
 namespace mugpu {
 
@@ -1151,14 +1152,22 @@ extern "C" int mugpu_cell_initialise(mugpu_cell c) {
   // tangent alone -> its dim^3 form; laws whose tangent is major-symmetric
   // (LE1-4 and a major-symmetric generic C pushed forward from PK2, the
   // consistent HEP1 tangent; 3D) -> upper triangle; otherwise the full matrix
+  // FP64 cells of LE1-4 alone, or in 3D of the consistent HEP1 alone, keep the
+  // factors of the tangent (the FP32-refined solve reads an FP32 copy of the
+  // matrix)
   bool all_hep = !c->mats.empty(), all_sym = c->dim == 3 && !c->mats.empty(), any_gen = false;
+  bool all_le = !c->mats.empty() && c->prec == MUGPU_FP64, all_ct = all_le && c->dim == 3;
   for (auto& m : c->mats) {
+    all_le = all_le && m.family >= MUGPU_LE1 && m.family <= MUGPU_LE4;
+    all_ct = all_ct && m.family == MUGPU_HEP1_CT;
     all_hep = all_hep && m.family == MUGPU_HEP1;
     all_sym = all_sym && m.family != MUGPU_HEP1 && (m.family != MUGPU_LEG || m.major_sym);
     any_gen = any_gen || m.family == MUGPU_LEG;
   }
   c->tan_kind = c->form == MUGPU_SMALL_STRAIN && !any_gen ? TAN_ISO
                 : all_hep                                 ? TAN_HEP
+                : all_le                                  ? TAN_LEF
+                : all_ct                                  ? TAN_HCT
                 : all_sym                                 ? TAN_SYM
                                                           : TAN_FULL;
   const size_t tn = (size_t)tangent_values(c->tan_kind, c->dim, c->N);
@@ -1271,6 +1280,16 @@ extern "C" int mugpu_cell_get_tangent(mugpu_cell c, double* h_K) {
     auto s = [&](int q) { return t[(size_t)tan_off(v, q, st)]; };
     if (c->tan_kind == TAN_FULL) {
       for (int q = 0; q < nc * nc; ++q) K[q] = s(q);
+    } else if (c->tan_kind == TAN_LEF || c->tan_kind == TAN_HCT) {
+      // column by column: K : e_q
+      double f[kHct], e[9];
+      for (int q = 0; q < st; ++q) f[q] = s(q);
+      for (int q = 0; q < nc; ++q) {
+        for (int r = 0; r < nc; ++r) e[r] = r == q ? 1.0 : 0.0;
+        if (c->tan_kind == TAN_HCT) hct_product<double>(f, e, K + nc * q);
+        else if (d == 3) lef_product<double, 3>(f, e, K + nc * q);
+        else lef_product<double, 2>(f, e, K + nc * q);
+      }
     } else if (c->tan_kind == TAN_SYM) {
       for (int col = 0; col < nc; ++col)
         for (int row = 0; row < nc; ++row)

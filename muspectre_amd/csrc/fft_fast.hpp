@@ -608,6 +608,12 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
       switch (a.tan_kind) {
         case TAN_SYM: kp_loop(std::integral_constant<int, TAN_SYM>{}); break;
         case TAN_HEP: kp_loop(std::integral_constant<int, TAN_HEP>{}); break;
+        case TAN_LEF:
+          if constexpr (sizeof(T) == 8) kp_loop(std::integral_constant<int, TAN_LEF>{});
+          break;
+        case TAN_HCT:
+          if constexpr (sizeof(T) == 8 && DIM == 3) kp_loop(std::integral_constant<int, TAN_HCT>{});
+          break;
         case TAN_ISO: kp_loop(std::integral_constant<int, TAN_ISO>{}); break;
         default: kp_loop(std::integral_constant<int, TAN_FULL>{}); break;
       }

@@ -122,6 +122,10 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
       switch (a.tan_kind) {
         case TAN_SYM: voxels(std::integral_constant<int, TAN_SYM>{}); break;
         case TAN_HEP: voxels(std::integral_constant<int, TAN_HEP>{}); break;
+        case TAN_LEF: voxels(std::integral_constant<int, TAN_LEF>{}); break;
+        case TAN_HCT:
+          if constexpr (DIM == 3) voxels(std::integral_constant<int, TAN_HCT>{});
+          break;
         case TAN_ISO: voxels(std::integral_constant<int, TAN_ISO>{}); break;
         default: voxels(std::integral_constant<int, TAN_FULL>{}); break;
       }

@@ -132,6 +132,8 @@ __global__ __launch_bounds__(NT) void k_last_r2c(ZArgs<T> a) {
     switch (a.tan_kind) {
       case TAN_SYM: voxels(std::integral_constant<int, TAN_SYM>{}); break;
       case TAN_HEP: voxels(std::integral_constant<int, TAN_HEP>{}); break;
+      case TAN_LEF: voxels(std::integral_constant<int, TAN_LEF>{}); break;
+      case TAN_HCT: voxels(std::integral_constant<int, TAN_HCT>{}); break;
       case TAN_ISO: voxels(std::integral_constant<int, TAN_ISO>{}); break;
       default: voxels(std::integral_constant<int, TAN_FULL>{}); break;
     }

@@ -13,10 +13,12 @@
 // The tangent is written in the representation the cell chose: ISO
 // (lambda, mu), HEP (dim^3, j-independent Kirchhoff->PK1 tangent), FULL
 // (the reference's nc x nc matrix) or SYM (its upper triangle), in the
-// voxel-blocked layout of tan_off().
+// voxel-blocked layout of tan_off().  FP64 finite-strain cells of one kind of
+// law keep the factors of the tangent instead (TAN_LEF, TAN_HCT).
 #include <cmath>
 
 #include "mugpu_internal.hpp"
+#include "op_stages.hpp"
 
 namespace mugpu {
 
@@ -370,6 +372,89 @@ __device__ void hep1_consistent_tangent(const MatArgs& a, int64_t v, const doubl
     }
 }
 
+// the same tangent as its factors in the eigenbasis of be* (hct_product): the
+// rotation V as a quaternion (the largest component first, so that nothing is
+// divided by a small one), H = V^T F^-T, g_mn b_n, the moduli, and the eigenvalues
+// of N and tau, which are coaxial with be*
+__device__ void hep1_tangent_factors(const MatArgs& a, int64_t v, const double* Fi, const double* bes,
+                                     double c1, double c2, double c3, const double* Ns,
+                                     const double* tau) {
+  double ev[3], V[9];
+  jacobi3(bes, ev, V);
+  double* o = a.tan + tan_off(v, 0, kHct);
+  auto put = [&](int i, double x) { o[i * kTanBlock] = x; };
+  // V(i, j) at i + 3 j
+  const double tr = V[0] + V[4] + V[8];
+  double w, x, y, z;
+  if (tr >= V[0] && tr >= V[4] && tr >= V[8]) {
+    w = 1 + tr;
+    x = V[5] - V[7];
+    y = V[6] - V[2];
+    z = V[1] - V[3];
+  } else if (V[0] >= V[4] && V[0] >= V[8]) {
+    w = V[5] - V[7];
+    x = 1 + V[0] - V[4] - V[8];
+    y = V[1] + V[3];
+    z = V[6] + V[2];
+  } else if (V[4] >= V[8]) {
+    w = V[6] - V[2];
+    x = V[1] + V[3];
+    y = 1 + V[4] - V[0] - V[8];
+    z = V[5] + V[7];
+  } else {
+    w = V[1] - V[3];
+    x = V[6] + V[2];
+    y = V[5] + V[7];
+    z = 1 + V[8] - V[0] - V[4];
+  }
+  const double inv = 1.0 / sqrt(w * w + x * x + y * y + z * z);
+  put(0, w * inv);
+  put(1, x * inv);
+  put(2, y * inv);
+  put(3, z * inv);
+  // H(m, j) = sum_q V(q, m) Finv(j, q)
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      put(4 + m + 3 * j, V[3 * m] * Fi[j] + V[1 + 3 * m] * Fi[j + 3] + V[2 + 3 * m] * Fi[j + 6]);
+  const int pm[3] = {0, 0, 1}, pn[3] = {1, 2, 2};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double bm = ev[pm[k]], bn = ev[pn[k]], h = bn - bm;
+    const double g = h == 0.0 ? 1.0 / bm : log1p(h / bm) / h;
+    put(13 + 2 * k, g * bn);
+    put(14 + 2 * k, g * bm);
+  }
+  // eigenvalues of N and tau
+  double n[3], t[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    double sn = 0, st = 0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double vv = V[i + 3 * m] * V[j + 3 * m];
+        sn += vv * Ns[i + 3 * j];
+        st += vv * tau[i + 3 * j];
+      }
+    n[m] = sn;
+    t[m] = st;
+  }
+  // tau = t0 I + t1 N (its deviator is along N): t1 from the widest pair of n
+  const double t0 = (t[0] + t[1] + t[2]) / 3.0;
+  const double nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+  const double t1 = ((t[0] - t0) * n[0] + (t[1] - t0) * n[1] + (t[2] - t0) * n[2]) / nn;
+  put(19, c1);
+  put(20, c2);
+  put(21, c3);
+  put(22, n[0]);
+  put(23, n[1]);
+  put(24, t0);
+  put(25, t1);
+}
+
 // write an isotropic tangent (lambda, mu) in the cell's representation
 template <int D>
 __device__ void store_iso(const MatArgs& a, int64_t v, double lam, double mu) {
@@ -445,6 +530,20 @@ __device__ void pk1_from_pk2_store(const MatArgs& a, int64_t v, const double* F,
 #pragma unroll
   for (int q = 0; q < NC; ++q) P[q] = Pl[q];
   if (!a.need_tangent) return;
+  if (a.tan_kind == TAN_LEF) {
+    constexpr int NL = sym_lines(D), ST = NC + NL + 2;
+    double* o = a.tan + tan_off(v, 0, ST);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) o[q * kTanBlock] = F[q];
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+#pragma unroll
+      for (int i = 0; i <= j; ++i)
+        o[(NC + sym_line<D>(i, j)) * kTanBlock] = 0.5 * (S[i + D * j] + S[j + D * i]);
+    o[(NC + NL) * kTanBlock] = lam;
+    o[(NC + NL + 1) * kTanBlock] = mu;
+    return;
+  }
   for (int n = 0; n < D; ++n)
     for (int j = 0; j < D; ++j)
       for (int m = 0; m < D; ++m)
@@ -590,6 +689,12 @@ __global__ __launch_bounds__(256) void k_hep1(MatArgs a) {
     const double c1 = plastic ? a.bulk / 2. - mu / 3 + a0 * mu : 0.5 * lam;
     const double c2 = plastic ? (1 - 3 * a0) * mu : mu;
     const double c3 = plastic ? 2 * mu * (a0 - a1) : 0.0;
+    if constexpr (D == 3) {
+      if (a.tan_kind == TAN_HCT) {
+        hep1_tangent_factors(a, v, Fi, bes, c1, c2, c3, Ns, tau);
+        return;
+      }
+    }
     double Pl[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) Pl[c] = a.P[v * NC + c];

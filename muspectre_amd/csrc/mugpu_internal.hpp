@@ -78,15 +78,26 @@ void timing_void(int64_t from);
 // SYM : the upper triangle r <= c of a major-symmetric K (finite-strain
 //       hyperelastic laws and the consistent elasto-plastic tangent),
 //       nc (nc + 1) / 2 entries, row by row
+// LEF : FP64 finite-strain cells of linear elastic laws (LE1-4): F, the PK2
+//       stress S (Voigt order) and (lambda, mu), from which dP = dF S +
+//       F (C : sym(F^T dF)) is formed; dim^2 + dim (dim + 1) / 2 + 2 numbers, 17
+//       in 3D where the matrix has 45
+// HCT : FP64 3D cells of HyperElastoPlastic1 with the consistent tangent alone:
+//       the 26 numbers of hct_product (op_stages.hpp)
+// A CG iteration reads the tangent once per voxel, so its size counts (256^3
+// HCT: r2c pass 2.57 -> 2.04 ms; 175x147x99 LEF: 340 -> 261 us).
 //
 // Storage is voxel-blocked: blocks of kTanBlock consecutive voxels, entry
 // major inside a block, so that lanes on consecutive voxels read one
 // contiguous run per entry (coalesced) while a voxel's entries stay in one
 // block.
-enum TangentKind { TAN_FULL = 0, TAN_ISO = 1, TAN_HEP = 2, TAN_SYM = 3 };
+enum TangentKind { TAN_FULL = 0, TAN_ISO = 1, TAN_HEP = 2, TAN_SYM = 3, TAN_LEF = 4, TAN_HCT = 5 };
+constexpr int kHct = 26;
 constexpr int kTanBlock = 64;
 __host__ __device__ inline int tangent_stride(int kind, int dim) {
   const int nc = dim * dim;
+  if (kind == TAN_LEF) return nc + dim * (dim + 1) / 2 + 2;
+  if (kind == TAN_HCT) return kHct;
   return kind == TAN_FULL ? nc * nc
                           : kind == TAN_ISO ? 2 : kind == TAN_HEP ? dim * dim * dim : nc * (nc + 1) / 2;
 }

@@ -7,6 +7,136 @@
 
 namespace mugpu {
 
+// ---- symmetric fields (small strain) ---------------------------------------------
+// The small-strain projection takes and gives symmetric tensors, and K : p of
+// an isotropic tangent is symmetric: the spectra between the passes then hold
+// the dim (dim + 1) / 2 independent components (Voigt order: the diagonal, then
+// yz, xz, xy) instead of dim^2, 2/3 (3D) or 3/4 (2D) of the bytes and of the
+// transforms.  The projection of a field is that of its symmetric part, which
+// is taken when a field enters.  Measured per launch at 128^3 FP64: middle axis
+// 56 + 46 -> 38 + 32 us, first axis 62 -> 53, c2r 98 -> 76.
+__host__ __device__ constexpr int sym_lines(int dim) { return dim * (dim + 1) / 2; }
+// lines per row or k-point: packed or one per component
+__host__ __device__ constexpr int nb_lines(int dim, bool packed) {
+  return packed ? sym_lines(dim) : dim * dim;
+}
+template <int DIM>
+__host__ __device__ constexpr int sym_line(int i, int j) {
+  return i == j ? i : DIM == 3 ? 6 - (i + j) : 2;
+}
+// line of component c = i + dim j
+template <int DIM, bool PK>
+__host__ __device__ constexpr int line_of(int c) {
+  return PK ? sym_line<DIM>(c % DIM, c / DIM) : c;
+}
+template <typename T, int DIM, bool PK>
+__device__ __forceinline__ void pack_lines(const T* f, T* q) {
+  if constexpr (PK) {
+#pragma unroll
+    for (int j = 0; j < DIM; ++j)
+#pragma unroll
+      for (int i = 0; i <= j; ++i)
+        q[sym_line<DIM>(i, j)] = i == j ? f[i + DIM * i] : T(0.5) * (f[i + DIM * j] + f[j + DIM * i]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < DIM * DIM; ++c) q[c] = f[c];
+  }
+}
+
+// ---- tangents kept as factors ------------------------------------------------------
+// LEF: q holds F, S and (lambda, mu); p, dp at i + DIM j
+template <typename T, int DIM>
+__host__ __device__ __forceinline__ void lef_product(const T* q, const T* p, T* dp) {
+  constexpr int NC = DIM * DIM, NL = sym_lines(DIM);
+  const T *F = q, *S = q + NC;
+  const T lam = q[NC + NL], mu = q[NC + NL + 1];
+  T e[NC], tr = 0;  // F^T dF
+#pragma unroll
+  for (int j = 0; j < DIM; ++j)
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) {
+      T s = 0;
+#pragma unroll
+      for (int k = 0; k < DIM; ++k) s += F[k + DIM * i] * p[k + DIM * j];
+      e[i + DIM * j] = s;
+      if (i == j) tr += s;
+    }
+#pragma unroll
+  for (int j = 0; j < DIM; ++j)
+#pragma unroll
+    for (int i = 0; i < DIM; ++i) {
+      T s = 0;
+#pragma unroll
+      for (int k = 0; k < DIM; ++k) {
+        const T t = (k == j ? lam * tr : T(0)) + mu * (e[k + DIM * j] + e[j + DIM * k]);
+        s += p[i + DIM * k] * S[sym_line<DIM>(k, j)] + F[i + DIM * k] * t;
+      }
+      dp[i + DIM * j] = s;
+    }
+}
+
+// HCT: the consistent HEP1 tangent (materials.hip) in the eigenbasis V of the
+// trial b_e.  With H = V^T F^-T, D = V^T dF, Q = D H^T and t, n the eigenvalues of
+// tau and N, b those of b_e and g the divided differences of ln:
+//   dP = V [C(M) - diag(t) Q^T] H,  M_mm = 2 Q_mm,
+//   M_mn = g_mn (b_n Q_mn + b_m Q_nm),
+//   C(M) = c1 tr(M) I + c2 M + c3 diag(n) (n . diag M),  t_m = t0 + t1 n_m
+// q: [0, 4) V as a unit quaternion, [4, 13) H, [13, 19) g_mn b_n for (m, n) =
+// 01, 10, 02, 20, 12, 21, [19] c1, [20] c2, [21] c3, [22] n_0, [23] n_1 (n is
+// traceless), [24] t0, [25] t1
+template <typename T>
+__host__ __device__ __forceinline__ void hct_product(const T* q, const T* p, T* dp) {
+  T V[9];
+  {
+    const T w = q[0], x = q[1], y = q[2], z = q[3];
+    V[0] = 1 - 2 * (y * y + z * z);
+    V[1] = 2 * (x * y + w * z);
+    V[2] = 2 * (x * z - w * y);
+    V[3] = 2 * (x * y - w * z);
+    V[4] = 1 - 2 * (x * x + z * z);
+    V[5] = 2 * (y * z + w * x);
+    V[6] = 2 * (x * z + w * y);
+    V[7] = 2 * (y * z - w * x);
+    V[8] = 1 - 2 * (x * x + y * y);
+  }
+  const T* H = q + 4;
+  T D[9], Q[9], A[9];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) D[m + 3 * j] = V[3 * m] * p[3 * j] + V[1 + 3 * m] * p[1 + 3 * j] + V[2 + 3 * m] * p[2 + 3 * j];
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) Q[m + 3 * n] = D[m] * H[n] + D[m + 3] * H[n + 3] + D[m + 6] * H[n + 6];
+  const T n0 = q[22], n1 = q[23], n2 = -n0 - n1;
+  const T m0 = 2 * Q[0], m1 = 2 * Q[4], m2 = 2 * Q[8];
+  const T ct = q[19] * (m0 + m1 + m2), c2 = q[20], nm = q[21] * (n0 * m0 + n1 * m1 + n2 * m2);
+  const T m01 = c2 * (q[13] * Q[3] + q[14] * Q[1]);
+  const T m02 = c2 * (q[15] * Q[6] + q[16] * Q[2]);
+  const T m12 = c2 * (q[17] * Q[7] + q[18] * Q[5]);
+  const T t0 = q[24] + q[25] * n0, t1 = q[24] + q[25] * n1, t2 = q[24] + q[25] * n2;
+  // A = C(M) - diag(t) Q^T
+  A[0] = ct + c2 * m0 + n0 * nm - t0 * Q[0];
+  A[4] = ct + c2 * m1 + n1 * nm - t1 * Q[4];
+  A[8] = ct + c2 * m2 + n2 * nm - t2 * Q[8];
+  A[3] = m01 - t0 * Q[1];
+  A[1] = m01 - t1 * Q[3];
+  A[6] = m02 - t0 * Q[2];
+  A[2] = m02 - t2 * Q[6];
+  A[7] = m12 - t1 * Q[5];
+  A[5] = m12 - t2 * Q[7];
+  // dP = V (A H)
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    T b[3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) b[m] = A[m] * H[3 * j] + A[m + 3] * H[1 + 3 * j] + A[m + 6] * H[2 + 3 * j];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) dp[i + 3 * j] = V[i] * b[0] + V[i + 3] * b[1] + V[i + 6] * b[2];
+  }
+}
+
 // dp = K : p for voxel v in the cell's tangent representation (blocked
 // layout of tan_off(); lanes on consecutive voxels read contiguous runs)
 template <typename T, int DIM>
@@ -23,6 +153,19 @@ __device__ __forceinline__ void tangent_product(int kind, const T* __restrict__ 
 #pragma unroll
       for (int i = 0; i < DIM; ++i)
         dp[i + DIM * j] = (i == j ? lam * tr : T(0)) + mu * (p[i + DIM * j] + p[j + DIM * i]);
+  } else if (sizeof(T) == 8 && kind == TAN_LEF) {
+    constexpr int S = NC + sym_lines(DIM) + 2;
+    const T* K = tan + tan_off(v, 0, S);
+    T q[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) q[i] = K[i * kTanBlock];
+    lef_product<T, DIM>(q, p, dp);
+  } else if (sizeof(T) == 8 && DIM == 3 && kind == TAN_HCT) {
+    const T* K = tan + tan_off(v, 0, kHct);
+    T q[kHct];
+#pragma unroll
+    for (int i = 0; i < kHct; ++i) q[i] = K[i * kTanBlock];
+    if constexpr (DIM == 3) hct_product<T>(q, p, dp);
   } else if (kind == TAN_HEP) {
     constexpr int S = DIM * DIM * DIM;
     const T* M = tan + tan_off(v, 0, S);
@@ -66,42 +209,6 @@ __device__ __forceinline__ void tangent_product(int kind, const T* __restrict__ 
       for (int c = 0; c < NC; ++c) a += K[(r + NC * c) * kTanBlock] * p[c];
       dp[r] = a;
     }
-  }
-}
-
-// ---- symmetric fields (small strain) ---------------------------------------------
-// The small-strain projection takes and gives symmetric tensors, and K : p of
-// an isotropic tangent is symmetric: the spectra between the passes then hold
-// the dim (dim + 1) / 2 independent components (Voigt order: the diagonal, then
-// yz, xz, xy) instead of dim^2, 2/3 (3D) or 3/4 (2D) of the bytes and of the
-// transforms.  The projection of a field is that of its symmetric part, which
-// is taken when a field enters.  Measured per launch at 128^3 FP64: middle axis
-// 56 + 46 -> 38 + 32 us, first axis 62 -> 53, c2r 98 -> 76.
-__host__ __device__ constexpr int sym_lines(int dim) { return dim * (dim + 1) / 2; }
-// lines per row or k-point: packed or one per component
-__host__ __device__ constexpr int nb_lines(int dim, bool packed) {
-  return packed ? sym_lines(dim) : dim * dim;
-}
-template <int DIM>
-__host__ __device__ constexpr int sym_line(int i, int j) {
-  return i == j ? i : DIM == 3 ? 6 - (i + j) : 2;
-}
-// line of component c = i + dim j
-template <int DIM, bool PK>
-__host__ __device__ constexpr int line_of(int c) {
-  return PK ? sym_line<DIM>(c % DIM, c / DIM) : c;
-}
-template <typename T, int DIM, bool PK>
-__device__ __forceinline__ void pack_lines(const T* f, T* q) {
-  if constexpr (PK) {
-#pragma unroll
-    for (int j = 0; j < DIM; ++j)
-#pragma unroll
-      for (int i = 0; i <= j; ++i)
-        q[sym_line<DIM>(i, j)] = i == j ? f[i + DIM * i] : T(0.5) * (f[i + DIM * j] + f[j + DIM * i]);
-  } else {
-#pragma unroll
-    for (int c = 0; c < DIM * DIM; ++c) q[c] = f[c];
   }
 }
 
