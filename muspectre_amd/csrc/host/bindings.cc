@@ -47,6 +47,13 @@ py::array field_to(const std::vector<Real>& v, int64_t rows, int64_t cols) {
   return std::move(out);
 }
 
+// a result field straight into the array it is read as
+py::array result_array(const ResultField& f) {
+  py::array_t<double, py::array::f_style> out({(py::ssize_t)f.size(), (py::ssize_t)1});
+  f.copy_to(out.mutable_data());
+  return std::move(out);
+}
+
 // a (dim x dim) numpy array -> column-major Matrix (Eigen::MatrixXd semantics)
 Matrix matrix_from(const rarr& a) {
   if (a.ndim() != 2) throw SolverError("load increments must be 2D arrays");
@@ -719,10 +726,10 @@ PYBIND11_MODULE(_muSpectre, mod) {
   py::class_<OptimizeResult>(mod, "OptimizeResult")
       .def(py::init<>())
       .def_property("grad",
-                    [](const OptimizeResult& r) { return field_to(r.grad.host(), r.grad.size(), 1); },
+                    [](const OptimizeResult& r) { return result_array(r.grad); },
                     [](OptimizeResult& r, farr a) { r.grad.assign(a.data(), (int64_t)a.size()); })
       .def_property("stress",
-                    [](const OptimizeResult& r) { return field_to(r.stress.host(), r.stress.size(), 1); },
+                    [](const OptimizeResult& r) { return result_array(r.stress); },
                     [](OptimizeResult& r, farr a) { r.stress.assign(a.data(), (int64_t)a.size()); })
       .def_readwrite("success", &OptimizeResult::success)
       .def_readwrite("status", &OptimizeResult::status)

@@ -72,6 +72,10 @@ const std::vector<Real>& ResultField::host() const {
   }
   return host_;
 }
+void ResultField::copy_to(Real* dst) const {
+  if (host_valid_) std::copy(host_.begin(), host_.end(), dst);
+  else if (dev_) dev_->download(dst);
+}
 void ResultField::assign(const Real* h, int64_t n) {
   dev_.reset();
   host_.assign(h, h + n);

@@ -100,6 +100,8 @@ class ResultField {
   void capture(const void* d_src, int64_t n);
   int64_t size() const { return host_valid_ ? (int64_t)host_.size() : (dev_ ? dev_->size() : 0); }
   const std::vector<Real>& host() const;
+  // the values into dst (size() of them)
+  void copy_to(Real* dst) const;
   void assign(const Real* h, int64_t n);
 
  private:
