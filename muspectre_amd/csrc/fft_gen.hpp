@@ -1,4 +1,4 @@
-// FP64 passes for axis lengths known at run time (any length without a
+// Passes for axis lengths known at run time (any length without a
 // compile-time instantiation; the odd lengths that the reference's
 // projections ask for are all of this kind): building blocks of the kernels in
 // fft_gen_last.hip and fft_gen_axis.hip.

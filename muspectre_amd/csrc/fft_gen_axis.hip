@@ -1,4 +1,4 @@
-// Strided passes of FP64 grids along an axis of run-time length: c2c along
+// Strided passes along an axis of run-time length: c2c along
 // the middle axis (or the first one, for the engine's transforms), and the
 // first axis with the projection between its two transforms.  The plans'
 // shapes are made here too.
@@ -147,69 +147,72 @@ GenShape gen_strided_shape(const GenAxis& ax, int64_t inner, int64_t outer) {
 
 namespace {
 
+template <typename T>
 struct GStr {
-  double2* data;
+  c_t<T>* data;
   int64_t inner;
   int L, P, LS;
   GenAxis ax;
-  const double2* tw;
+  const c_t<T>* tw;
   const int* active;  // FftPlan::active
 };
 
 // data[(o * n + m) * inner + w]: the workgroup transforms L consecutive lines w
 // of plane o; HBM is read by the first pass and written by the last
-template <int CLS, int SG>
-__global__ __launch_bounds__(kGenMaxNT) void k_gen_strided(GStr a) {
+template <typename T, int CLS, int SG>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_strided(GStr<T> a) {
   if (a.active && !a.active[0]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS;
-  double2* s = reinterpret_cast<double2*>(smem);
-  double2* tw = s + n * LS;
-  gen_twiddles<double>(tw, a.tw, n);
+  c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
+  c_t<T>* tw = s + n * LS;
+  gen_twiddles<T>(tw, a.tw, n);
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
   const int64_t gx = gridDim.x;
   const int64_t t = xcd_tile(blockIdx.y * gx + blockIdx.x, gx * gridDim.y);
   const int64_t o = t / gx;
   const int64_t w = (t - o * gx) * a.L + l;
   const bool act = p < a.P && w < a.inner;
-  double2* base = a.data + o * n * a.inner + (w < a.inner ? w : a.inner - 1);
+  c_t<T>* base = a.data + o * n * a.inner + (w < a.inner ? w : a.inner - 1);
   const int64_t inner = a.inner;
-  gen_fft<double, CLS, SG, true, true>(
+  gen_fft<T, CLS, SG, true, true>(
       a.ax, a.P, p, act, s + l, LS, tw, [&](int m) { return base[m * inner]; },
-      [&](int m, double2 x) { base[m * inner] = x; });
+      [&](int m, c_t<T> x) { base[m * inner] = x; });
 }
 
+template <typename T>
 struct GAxis0 {
-  double2* data;
+  c_t<T>* data;
   int64_t plane;  // k-points per first-axis index
   int KP, L, P, LS;
   GenAxis ax;
-  const double2* tw;
+  const c_t<T>* tw;
   int kind, allow_even, res[3], hlast;
-  double Lc[3], norm;
+  double Lc[3];
+  T norm;
   const int* active;  // FftPlan::active
 };
 
-template <int CLS, int DIM, bool PK>
-__global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0 a) {
+template <typename T, int CLS, int DIM, bool PK>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0<T> a) {
   if (a.active && !a.active[0]) return;
   constexpr int NC = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS, KP = a.KP;
-  double2* s = reinterpret_cast<double2*>(smem);
-  double2* tw = s + n * LS;
-  gen_twiddles<double>(tw, a.tw, n);
+  c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
+  c_t<T>* tw = s + n * LS;
+  gen_twiddles<T>(tw, a.tw, n);
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
   const int64_t q0 = xcd_tile(blockIdx.x, gridDim.x) * KP;
   const int64_t inner = a.plane * NC;
   const int64_t w = q0 * NC + l;
   const bool act = p < a.P, valid = w < inner;
-  double2* base = a.data + (valid ? w : inner - 1);
+  c_t<T>* base = a.data + (valid ? w : inner - 1);
   auto ld = [&](int m) { return base[m * inner]; };
-  auto st = [&](int m, double2 x) {
+  auto st = [&](int m, c_t<T> x) {
     if (valid) base[m * inner] = x;
   };
-  gen_fft<double, CLS, -1, true, false>(a.ax, a.P, p, act, s + l, LS, tw, ld, st);
+  gen_fft<T, CLS, -1, true, false>(a.ax, a.P, p, act, s + l, LS, tw, ld, st);
   // projection per wave vector (k0, q0 + kp); KP is 1, 2 or 4 and divides the
   // thread count, so a thread keeps one kp
   const int sh = KP >> 1;  // log2 of KP
@@ -224,25 +227,24 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_axis0(GAxis0 a) {
   }
   for (int k0 = threadIdx.x >> sh; k0 < n && q < a.plane; k0 += blockDim.x >> sh) {
     c[0] = k0;
-    double xi[DIM];
-    double2* f = s + k0 * LS + kp * NC;
-    if (!unit_wave_vector<double, DIM>(c, a.res, a.Lc, a.allow_even, xi)) {
+    T xi[DIM];
+    c_t<T>* f = s + k0 * LS + kp * NC;
+    if (!unit_wave_vector<T, DIM>(c, a.res, a.Lc, a.allow_even, xi)) {
 #pragma unroll
-      for (int r = 0; r < NC; ++r) f[r] = double2{};
+      for (int r = 0; r < NC; ++r) f[r] = c_t<T>{};
       continue;
     }
-    if constexpr (PK) project_point_sym<double, DIM>(f, xi, a.norm);
-    else project_point<double, DIM>(f, 1, xi, a.kind, a.norm);
+    if constexpr (PK) project_point_sym<T, DIM>(f, xi, a.norm);
+    else project_point<T, DIM>(f, 1, xi, a.kind, a.norm);
   }
   __syncthreads();
-  gen_fft<double, CLS, +1, false, true>(a.ax, a.P, p, act, s + l, LS, tw, ld, st);
+  gen_fft<T, CLS, +1, false, true>(a.ax, a.P, p, act, s + l, LS, tw, ld, st);
 }
 
-}  // namespace
-
-int gen_strided(FftPlan& p, int ax, void* spec, int sign) {
-  GStr a{};
-  a.data = static_cast<double2*>(spec);
+template <typename T>
+int strided_t(FftPlan& p, int ax, void* spec, int sign) {
+  GStr<T> a{};
+  a.data = static_cast<c_t<T>*>(spec);
   a.inner = p.lines();
   for (int d = ax + 1; d < p.dim; ++d) a.inner *= p.hres[d];
   int64_t outer = 1;
@@ -252,31 +254,32 @@ int gen_strided(FftPlan& p, int ax, void* spec, int sign) {
   a.P = g.P;
   a.LS = g.L | 1;
   a.ax = p.gen[ax];
-  a.tw = static_cast<const double2*>(p.tw64[ax]);
+  a.tw = static_cast<const c_t<T>*>(sizeof(T) == 8 ? p.tw64[ax] : p.tw32[ax]);
   a.active = p.active;
   const dim3 grid((unsigned)((a.inner + a.L - 1) / a.L), (unsigned)outer), block((unsigned)g.NT);
   if (a.ax.cls == 0) {
-    if (sign < 0) hipLaunchKernelGGL((k_gen_strided<0, -1>), grid, block, g.lds, stream(), a);
-    else hipLaunchKernelGGL((k_gen_strided<0, +1>), grid, block, g.lds, stream(), a);
+    if (sign < 0) hipLaunchKernelGGL((k_gen_strided<T, 0, -1>), grid, block, g.lds, stream(), a);
+    else hipLaunchKernelGGL((k_gen_strided<T, 0, +1>), grid, block, g.lds, stream(), a);
   } else {
-    if (sign < 0) hipLaunchKernelGGL((k_gen_strided<1, -1>), grid, block, g.lds, stream(), a);
-    else hipLaunchKernelGGL((k_gen_strided<1, +1>), grid, block, g.lds, stream(), a);
+    if (sign < 0) hipLaunchKernelGGL((k_gen_strided<T, 1, -1>), grid, block, g.lds, stream(), a);
+    else hipLaunchKernelGGL((k_gen_strided<T, 1, +1>), grid, block, g.lds, stream(), a);
   }
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }
 
-int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec) {
-  GAxis0 a{};
-  a.data = static_cast<double2*>(spec);
+template <typename T, int DIM, bool PK>
+int axis0_t(FftPlan& p, const ProjParams& pj, void* spec) {
+  GAxis0<T> a{};
+  a.data = static_cast<c_t<T>*>(spec);
   a.plane = p.kpts / p.res[0];
-  const GenShape& g = p.gen_axis0[p.packed ? 1 : 0];
+  const GenShape& g = p.gen_axis0[PK ? 1 : 0];
   a.KP = g.mult;
   a.L = g.L;
   a.P = g.P;
   a.LS = g.L | 1;
   a.ax = p.gen[0];
-  a.tw = static_cast<const double2*>(p.tw64[0]);
+  a.tw = static_cast<const c_t<T>*>(sizeof(T) == 8 ? p.tw64[0] : p.tw32[0]);
   a.kind = pj.kind;
   a.allow_even = pj.allow_even;
   for (int d = 0; d < 3; ++d) {
@@ -284,23 +287,26 @@ int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec) {
     a.Lc[d] = pj.L[d];
   }
   a.hlast = p.hres[p.dim - 1];
-  a.norm = pj.norm;
+  a.norm = (T)pj.norm;
   a.active = p.active;
   const dim3 grid((unsigned)((a.plane + a.KP - 1) / a.KP)), block((unsigned)g.NT);
-  auto go = [&](auto dim, auto pk) {
-    constexpr int D = decltype(dim)::value;
-    constexpr bool K = decltype(pk)::value;
-    if (a.ax.cls == 0) hipLaunchKernelGGL((k_gen_axis0<0, D, K>), grid, block, g.lds, stream(), a);
-    else hipLaunchKernelGGL((k_gen_axis0<1, D, K>), grid, block, g.lds, stream(), a);
-  };
-  using D2 = std::integral_constant<int, 2>;
-  using D3 = std::integral_constant<int, 3>;
-  if (p.dim == 3 && p.packed) go(D3{}, std::true_type{});
-  else if (p.dim == 3) go(D3{}, std::false_type{});
-  else if (p.packed) go(D2{}, std::true_type{});
-  else go(D2{}, std::false_type{});
+  if (a.ax.cls == 0) hipLaunchKernelGGL((k_gen_axis0<T, 0, DIM, PK>), grid, block, g.lds, stream(), a);
+  else hipLaunchKernelGGL((k_gen_axis0<T, 1, DIM, PK>), grid, block, g.lds, stream(), a);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
+}
+
+}  // namespace
+
+int gen_strided(FftPlan& p, int prec, int ax, void* spec, int sign) {
+  return prec == MUGPU_FP64 ? strided_t<double>(p, ax, spec, sign) : strided_t<float>(p, ax, spec, sign);
+}
+
+int gen_axis0_project(FftPlan& p, int prec, const ProjParams& pj, void* spec) {
+  if (prec != MUGPU_FP64)
+    return p.dim == 3 ? axis0_t<float, 3, false>(p, pj, spec) : axis0_t<float, 2, false>(p, pj, spec);
+  if (p.packed) return p.dim == 3 ? axis0_t<double, 3, true>(p, pj, spec) : axis0_t<double, 2, true>(p, pj, spec);
+  return p.dim == 3 ? axis0_t<double, 3, false>(p, pj, spec) : axis0_t<double, 2, false>(p, pj, spec);
 }
 
 }  // namespace mugpu

@@ -1,4 +1,4 @@
-// Last-axis passes of FP64 grids whose last axis has a run-time length: r2c
+// Last-axis passes of grids whose last axis has a run-time length: r2c
 // with the CG direction update and K : p in front, c2r with the p . Ap partial
 // sums behind.
 //
@@ -13,23 +13,24 @@ namespace mugpu {
 
 namespace {
 
+template <typename T>
 struct GLast {
-  const double* in;
-  const double* rvec;
-  double* pout;
+  const T* in;
+  const T* rvec;
+  T* pout;
   const double* scal;
-  const double* tan;
+  const T* tan;
   int tan_kind;
-  double2* spec;
-  double* out;
-  double* x;
-  double* ap;
-  const double* dotv;
+  c_t<T>* spec;
+  T* out;
+  T* x;
+  T* ap;
+  const T* dotv;
   double* partials;
   int64_t rows;
   int RB, L, P, LS;  // rows and lines per workgroup, threads per line, LDS line stride
   GenAxis ax;
-  const double2* tw;
+  const c_t<T>* tw;
   const int* active;  // FftPlan::active
   ScalarFold fold;
 };
@@ -38,16 +39,16 @@ struct GLast {
 // values per point].  The updated p of two rows is staged as it lies in memory
 // and read back a voxel per thread (a lane stride of NC doubles, odd in 3D: no
 // bank conflict), so that r, p are read and p is written in full cache lines.
-template <int CLS, int DIM, int IN, bool PK>
-__global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
+template <typename T, int CLS, int DIM, int IN, bool PK>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast<T> a) {
   constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x;
-  double2* s = reinterpret_cast<double2*>(smem);
-  double* sr = reinterpret_cast<double*>(smem);
+  c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
+  T* sr = reinterpret_cast<T*>(smem);
   __shared__ double red[16];
-  double2* tw = s + n * LS;
-  double* sp = reinterpret_cast<double*>(tw + n);
+  c_t<T>* tw = s + n * LS;
+  T* sp = reinterpret_cast<T*>(tw + n);
   // (the flag and the partial sums are read together)
   const int on = a.active ? a.active[0] : 1;
   const int64_t row0 = (int64_t)blockIdx.x * a.RB;
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
     constexpr int KB = 4;
     if (r0) __syncthreads();  // the staged rows before have been read
     for (int e0 = 0; e0 < tot; e0 += KB * NT) {
-      double pv[KB], rv[KB], xv[KB];
+      T pv[KB], rv[KB], xv[KB];
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
         const int e = e0 + i * NT + threadIdx.x;
@@ -76,12 +77,12 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
       for (int i = 0; i < KB; ++i) {
         const int e = e0 + i * NT + threadIdx.x;
         if (e < tot) {
-          double x = 0.0;
+          T x = T(0);
           if (base + e < lim) {
             x = pv[i];
-            if (XU) a.x[base + e] = xv[i] + al * x;
+            if (XU) a.x[base + e] = xv[i] + (T)al * x;
             if (PU) {
-              x = -rv[i] + beta * x;
+              x = -rv[i] + (T)beta * x;
               a.pout[base + e] = x;
             }
           }
@@ -89,27 +90,27 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
         }
       }
     }
-    if (r0 == 0) gen_twiddles<double>(tw, a.tw, n);
+    if (r0 == 0) gen_twiddles<T>(tw, a.tw, n);
     __syncthreads();
     // rows beyond the last one hold zeros, for which K : p is not evaluated
     auto voxels = [&](auto kind_c) {
       constexpr int KIND = decltype(kind_c)::value;
       for (int e = threadIdx.x; e < 2 * n; e += NT) {
         const int r = e >= n, m = e - r * n;
-        double p[NC], dp[NC];
+        T p[NC], dp[NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) p[c] = sp[e * NC + c];
         if (KIND >= 0 && row0 + r0 + r < a.rows) {
-          tangent_product<double, DIM>(KIND, a.tan, (row0 + r0 + r) * n + m, p, dp);
+          tangent_product<T, DIM>(KIND, a.tan, (row0 + r0 + r) * n + m, p, dp);
 #pragma unroll
-          for (int c = 0; c < NC; ++c) acc += p[c] * dp[c];
+          for (int c = 0; c < NC; ++c) acc += (double)p[c] * (double)dp[c];
         } else {
 #pragma unroll
           for (int c = 0; c < NC; ++c) dp[c] = p[c];
         }
-        double q[NL];
-        pack_lines<double, DIM, PK>(dp, q);
-        double* o = sr + 2 * (m * LS + (r0 >> 1) * NL) + r;
+        T q[NL];
+        pack_lines<T, DIM, PK>(dp, q);
+        T* o = sr + 2 * (m * LS + (r0 >> 1) * NL) + r;
 #pragma unroll
         for (int c = 0; c < NL; ++c) o[2 * c] = q[c];
       }
@@ -133,23 +134,23 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
   }
   __syncthreads();
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
-  auto none_ld = [](int) { return double2{}; };
-  auto none_st = [](int, double2) {};
-  gen_fft<double, CLS, -1, false, false>(a.ax, a.P, p, p < a.P, s + l, LS, tw, none_ld, none_st);
+  auto none_ld = [](int) { return c_t<T>{}; };
+  auto none_st = [](int, c_t<T>) {};
+  gen_fft<T, CLS, -1, false, false>(a.ax, a.P, p, p < a.P, s + l, LS, tw, none_ld, none_st);
   for (int r = 0; r < a.RB; ++r) {
     if (row0 + r >= a.rows) break;
-    double2* o = a.spec + (row0 + r) * nh * NL;
-    const double2* sl = s + (r >> 1) * NL;
+    c_t<T>* o = a.spec + (row0 + r) * nh * NL;
+    const c_t<T>* sl = s + (r >> 1) * NL;
     for (int e = threadIdx.x; e < nh * NL; e += NT) {
       const int k = e / NL, c = e - k * NL;
-      const double2 z = sl[k * LS + c], zc = sl[(k == 0 ? 0 : n - k) * LS + c];
-      double2 X;
+      const c_t<T> z = sl[k * LS + c], zc = sl[(k == 0 ? 0 : n - k) * LS + c];
+      c_t<T> X;
       if (!(r & 1)) {
-        X.x = 0.5 * (z.x + zc.x);
-        X.y = 0.5 * (z.y - zc.y);
+        X.x = T(0.5) * (z.x + zc.x);
+        X.y = T(0.5) * (z.y - zc.y);
       } else {
-        X.x = 0.5 * (z.y + zc.y);
-        X.y = -0.5 * (z.x - zc.x);
+        X.x = T(0.5) * (z.y + zc.y);
+        X.y = T(-0.5) * (z.x - zc.x);
       }
       o[e] = X;
     }
@@ -163,15 +164,15 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast a) {
 // LDS: [lines][twiddles]; the half lines of a workgroup are staged over the
 // lines, combined through registers (kGenVals values per thread at most, which
 // P guarantees) and transformed in place.
-template <int CLS, int DIM, int OUT, bool PK>
-__global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
+template <typename T, int CLS, int DIM, int OUT, bool PK>
+__global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast<T> a) {
   constexpr int NC = DIM * DIM, NL = nb_lines(DIM, PK);
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[16];
   const int n = a.ax.n, LS = a.LS, nh = n / 2 + 1, NT = blockDim.x, RB = a.RB;
-  double2* s = reinterpret_cast<double2*>(smem);
+  c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   const int stage = RB * nh * NL;  // staged values; the twiddles follow the larger of the two
-  double2* tw = s + (n * LS > stage ? n * LS : stage);
+  c_t<T>* tw = s + (n * LS > stage ? n * LS : stage);
   const int on = a.active ? a.active[0] : 1;
   const bool fold = OUT == OUT_RUPD && a.fold.pk;
   const double pk = fold ? fold_sum(a.fold.pk, a.fold.npk, red) : 0.0;
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
     const int64_t base = row0 * nh * NL, lim = a.rows * nh * NL;
     constexpr int KB = 4;
     for (int e0 = 0; e0 < stage; e0 += KB * NT) {
-      double2 t[KB];
+      c_t<T> t[KB];
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
         const int e = e0 + i * NT + threadIdx.x;
@@ -191,26 +192,26 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
         const int e = e0 + i * NT + threadIdx.x;
-        if (e < stage) s[e] = base + e < lim ? t[i] : double2{};
+        if (e < stage) s[e] = base + e < lim ? t[i] : c_t<T>{};
       }
     }
   }
-  gen_twiddles<double>(tw, a.tw, n);
+  gen_twiddles<T>(tw, a.tw, n);
   __syncthreads();
   const int p = threadIdx.x / a.L, l = threadIdx.x - p * a.L;
   const bool act = p < a.P;
   {
     const int rp = l / NL, c = l - rp * NL;
-    const double2* A0 = s + (2 * rp) * nh * NL + c;
-    const double2* B0 = A0 + nh * NL;
-    double2 v[kGenVals];
+    const c_t<T>* A0 = s + (2 * rp) * nh * NL + c;
+    const c_t<T>* B0 = A0 + nh * NL;
+    c_t<T> v[kGenVals];
 #pragma unroll
     for (int i = 0; i < kGenVals; ++i) {
       const int m = p + i * a.P;
       if (act && m < n) {
         const int kk = m < nh ? m : n - m;
-        double2 A = A0[kk * NL], B = B0[kk * NL];
-        if (kk == 0 || 2 * kk == n) A.y = B.y = 0.0;
+        c_t<T> A = A0[kk * NL], B = B0[kk * NL];
+        if (kk == 0 || 2 * kk == n) A.y = B.y = T(0);
         if (m >= nh) {
           A.y = -A.y;
           B.y = -B.y;
@@ -227,22 +228,22 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
     }
     __syncthreads();
   }
-  auto none_ld = [](int) { return double2{}; };
-  auto none_st = [](int, double2) {};
-  gen_fft<double, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
-  const double* sr = reinterpret_cast<const double*>(smem);
+  auto none_ld = [](int) { return c_t<T>{}; };
+  auto none_st = [](int, c_t<T>) {};
+  gen_fft<T, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
+  const T* sr = reinterpret_cast<const T*>(smem);
   const double al = OUT != OUT_RUPD ? 0.0 : fold ? alpha : a.scal[SC_ALPHA];
   double acc = 0.0;
   for (int r = 0; r < RB; ++r) {
     if (row0 + r >= a.rows) break;
     const int64_t base = (row0 + r) * n * NC;
-    const double* sl = sr + 2 * ((r >> 1) * NL) + (r & 1);
+    const T* sl = sr + 2 * ((r >> 1) * NL) + (r & 1);
     const int tot = n * NC;
     constexpr int KB = 4;
     for (int e0 = 0; e0 < tot; e0 += KB * NT) {
-      double dv[KB];
+      T dv[KB];
       if (OUT != OUT_PLAIN) {
-        const double* __restrict__ dsrc = OUT == OUT_RUPD ? a.out : a.dotv;
+        const T* __restrict__ dsrc = OUT == OUT_RUPD ? a.out : a.dotv;
 #pragma unroll
         for (int i = 0; i < KB; ++i) {
           const int e = e0 + i * NT + threadIdx.x;
@@ -254,15 +255,15 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
         const int e = e0 + i * NT + threadIdx.x;
         if (e < tot) {
           const int m = e / NC, c = e - m * NC;
-          const double val = sl[2 * (m * LS + line_of<DIM, PK>(c))];
+          const T val = sl[2 * (m * LS + line_of<DIM, PK>(c))];
           if (OUT == OUT_RUPD) {
-            const double rv = dv[i] + al * val;
+            const T rv = dv[i] + (T)al * val;
             a.out[base + e] = rv;
             if (a.ap) a.ap[base + e] = val;
-            acc += rv * rv;
+            acc += (double)rv * (double)rv;
           } else {
             a.out[base + e] = val;
-            if (OUT == OUT_DOT) acc += val * dv[i];
+            if (OUT == OUT_DOT) acc += (double)val * (double)dv[i];
           }
         }
       }
@@ -274,19 +275,20 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast a) {
   }
 }
 
-void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a) {
+template <typename T>
+void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast<T>& a) {
   const int d = p.dim - 1;
-  a.in = static_cast<const double*>(op.in);
-  a.rvec = static_cast<const double*>(op.rvec);
-  a.pout = static_cast<double*>(op.pout);
+  a.in = static_cast<const T*>(op.in);
+  a.rvec = static_cast<const T*>(op.rvec);
+  a.pout = static_cast<T*>(op.pout);
   a.scal = op.scal;
-  a.tan = static_cast<const double*>(op.tangent);
+  a.tan = static_cast<const T*>(op.tangent);
   a.tan_kind = op.tan_kind;
-  a.spec = static_cast<double2*>(spec);
-  a.out = static_cast<double*>(op.out);
-  a.dotv = static_cast<const double*>(op.dotv);
-  a.x = static_cast<double*>(op.xvec);
-  a.ap = static_cast<double*>(op.ap_out);
+  a.spec = static_cast<c_t<T>*>(spec);
+  a.out = static_cast<T*>(op.out);
+  a.dotv = static_cast<const T*>(op.dotv);
+  a.x = static_cast<T*>(op.xvec);
+  a.ap = static_cast<T*>(op.ap_out);
   a.partials = static_cast<double*>(p.partials);
   a.rows = p.N / p.res[d];
   a.RB = g.mult * 2;
@@ -294,69 +296,86 @@ void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast& a)
   a.P = g.P;
   a.LS = g.L | 1;
   a.ax = p.gen[d];
-  a.tw = static_cast<const double2*>(p.tw64[d]);
+  a.tw = static_cast<const c_t<T>*>(sizeof(T) == 8 ? p.tw64[d] : p.tw32[d]);
   a.active = p.active;
   a.fold = p.fold;
 }
 
-template <int CLS, int DIM, bool PK>
+template <typename T, int CLS, int DIM, bool PK>
 int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
   const GenShape& g = p.gen_last[PK ? 1 : 0];
-  GLast a{};
+  GLast<T> a{};
   fill(p, op, spec, g, a);
   if (!op.fin_alpha) a.partials = nullptr;
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT);
-  p.wg_r2c = grid.x;
-  if (a.fold.pk) a.partials = a.fold.pk;
-  if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
-  switch (op.in_mode) {
-    case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a); break;
-    case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN, PK>), grid, block, g.lds, stream(), a); break;
-    default:
-      if (op.xvec) hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE_X, PK>), grid, block, g.lds, stream(), a);
-      else hipLaunchKernelGGL((k_gen_r2c<CLS, DIM, IN_TAN_PUPDATE, PK>), grid, block, g.lds, stream(), a);
-      break;
+  if constexpr (sizeof(T) == 4) {
+    // FP32: the engine's transforms and the projections
+    if (op.in_mode != IN_PLAIN) return MUGPU_EARG;
+    hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a);
+  } else {
+    p.wg_r2c = grid.x;
+    if (a.fold.pk) a.partials = a.fold.pk;
+    if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
+    switch (op.in_mode) {
+      case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a); break;
+      case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_TAN, PK>), grid, block, g.lds, stream(), a); break;
+      default:
+        if (op.xvec)
+          hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_TAN_PUPDATE_X, PK>), grid, block, g.lds, stream(), a);
+        else
+          hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_TAN_PUPDATE, PK>), grid, block, g.lds, stream(), a);
+        break;
+    }
   }
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }
 
-template <int CLS, int DIM, bool PK>
+template <typename T, int CLS, int DIM, bool PK>
 int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
   const GenShape& g = p.gen_last[PK ? 1 : 0];
-  GLast a{};
+  GLast<T> a{};
   fill(p, op, spec, g, a);
   const dim3 grid((unsigned)((a.rows + a.RB - 1) / a.RB)), block((unsigned)g.NT_bwd);
-  p.wg_c2r = grid.x;
-  if (op.out_mode == OUT_RUPD)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds_bwd, stream(), a);
-  else if (op.out_mode == OUT_DOT)
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_DOT, PK>), grid, block, g.lds_bwd, stream(), a);
-  else
-    hipLaunchKernelGGL((k_gen_c2r<CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds_bwd, stream(), a);
+  if constexpr (sizeof(T) == 4) {
+    if (op.out_mode != OUT_PLAIN) return MUGPU_EARG;
+    hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds_bwd, stream(), a);
+  } else {
+    p.wg_c2r = grid.x;
+    if (op.out_mode == OUT_RUPD)
+      hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds_bwd, stream(), a);
+    else if (op.out_mode == OUT_DOT)
+      hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_DOT, PK>), grid, block, g.lds_bwd, stream(), a);
+    else
+      hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds_bwd, stream(), a);
+  }
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }
 
-template <int DIM, bool PK>
+template <typename T, int DIM, bool PK>
 int r2c_cls(FftPlan& p, const OpSpec& op, void* spec) {
-  return p.gen[DIM - 1].cls ? r2c_launch<1, DIM, PK>(p, op, spec) : r2c_launch<0, DIM, PK>(p, op, spec);
+  return p.gen[DIM - 1].cls ? r2c_launch<T, 1, DIM, PK>(p, op, spec) : r2c_launch<T, 0, DIM, PK>(p, op, spec);
 }
-template <int DIM, bool PK>
+template <typename T, int DIM, bool PK>
 int c2r_cls(FftPlan& p, const OpSpec& op, void* spec) {
-  return p.gen[DIM - 1].cls ? c2r_launch<1, DIM, PK>(p, op, spec) : c2r_launch<0, DIM, PK>(p, op, spec);
+  return p.gen[DIM - 1].cls ? c2r_launch<T, 1, DIM, PK>(p, op, spec) : c2r_launch<T, 0, DIM, PK>(p, op, spec);
 }
 
 }  // namespace
 
-int gen_r2c(FftPlan& p, const OpSpec& op, void* spec) {
-  if (p.packed) return p.dim == 3 ? r2c_cls<3, true>(p, op, spec) : r2c_cls<2, true>(p, op, spec);
-  return p.dim == 3 ? r2c_cls<3, false>(p, op, spec) : r2c_cls<2, false>(p, op, spec);
+int gen_r2c(FftPlan& p, int prec, const OpSpec& op, void* spec) {
+  if (prec != MUGPU_FP64)
+    return p.dim == 3 ? r2c_cls<float, 3, false>(p, op, spec) : r2c_cls<float, 2, false>(p, op, spec);
+  if (p.packed) return p.dim == 3 ? r2c_cls<double, 3, true>(p, op, spec) : r2c_cls<double, 2, true>(p, op, spec);
+  return p.dim == 3 ? r2c_cls<double, 3, false>(p, op, spec) : r2c_cls<double, 2, false>(p, op, spec);
 }
 
-int gen_c2r(FftPlan& p, const OpSpec& op, void* spec) {
-  if (p.packed) return p.dim == 3 ? c2r_cls<3, true>(p, op, spec) : c2r_cls<2, true>(p, op, spec);
-  return p.dim == 3 ? c2r_cls<3, false>(p, op, spec) : c2r_cls<2, false>(p, op, spec);
+int gen_c2r(FftPlan& p, int prec, const OpSpec& op, void* spec) {
+  if (prec != MUGPU_FP64)
+    return p.dim == 3 ? c2r_cls<float, 3, false>(p, op, spec) : c2r_cls<float, 2, false>(p, op, spec);
+  if (p.packed) return p.dim == 3 ? c2r_cls<double, 3, true>(p, op, spec) : c2r_cls<double, 2, true>(p, op, spec);
+  return p.dim == 3 ? c2r_cls<double, 3, false>(p, op, spec) : c2r_cls<double, 2, false>(p, op, spec);
 }
 
 }  // namespace mugpu

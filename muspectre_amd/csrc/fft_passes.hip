@@ -504,10 +504,11 @@ int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool genera
     }
   const int n = res[dim - 1];
   const int64_t rows = p.N / n;
-  // FP64 passes of run-time length (fft_gen.hpp) on every other axis whose
+  // passes of run-time length (fft_gen.hpp) on every other axis whose
   // workgroups fit: 2 to 6 times faster at 45^3 to 175x147x99, 1.3 times at 51^2;
-  // what is left to the passes below: FP32 and the cells of the FP32-refined
-  // solve, single points and the longest axes
+  // what is left to the passes below: the cells of the FP32-refined solve,
+  // single points and the longest axes.  On the compiled lengths they are
+  // slower (CG on 128^3 8.06 against 6.79 ms, on 256^2 and below within 10 %)
   for (int d = 0; d < dim; ++d) {
     if (!general || p.fastax[d] || !gen_radices(res[d], p.gen[d])) continue;
     int64_t inner = 1, outer = 1;
@@ -630,9 +631,9 @@ int launch_r2c(FftPlan& p, const OpSpec& op, c_t<T>* spec) {
     timing_end(MUGPU_K_LAST_R2C);
     return rc;
   }
-  if (sizeof(T) == 8 && p.genax[DIM - 1]) {
+  if (p.genax[DIM - 1]) {
     timing_begin(MUGPU_K_LAST_R2C);
-    const int rc = gen_r2c(p, op, spec);
+    const int rc = gen_r2c(p, prec_of<T>(), op, spec);
     timing_end(MUGPU_K_LAST_R2C);
     return rc;
   }
@@ -673,9 +674,9 @@ int launch_c2r(FftPlan& p, const OpSpec& op, c_t<T>* spec) {
     timing_end(MUGPU_K_LAST_C2R);
     return rc;
   }
-  if (sizeof(T) == 8 && p.genax[DIM - 1]) {
+  if (p.genax[DIM - 1]) {
     timing_begin(MUGPU_K_LAST_C2R);
-    const int rc = gen_c2r(p, op, spec);
+    const int rc = gen_c2r(p, prec_of<T>(), op, spec);
     timing_end(MUGPU_K_LAST_C2R);
     return rc;
   }
@@ -726,10 +727,10 @@ int launch_strided(FftPlan& p, int ax, int W, c_t<T>* spec, int sign) {
     timing_end(kc);
     return rc;
   }
-  if (sizeof(T) == 8 && p.genax[ax]) {
+  if (p.genax[ax]) {
     const int kc = ax == 0 ? MUGPU_K_AXIS0 : MUGPU_K_MIDDLE;
     timing_begin(kc);
-    const int rc = gen_strided(p, ax, spec, sign);
+    const int rc = gen_strided(p, prec_of<T>(), ax, spec, sign);
     timing_end(kc);
     return rc;
   }
@@ -758,9 +759,9 @@ int launch_project(FftPlan& p, const ProjParams& pj, c_t<T>* spec) {
     timing_end(MUGPU_K_AXIS0);
     return rc;
   }
-  if (sizeof(T) == 8 && p.genax[0]) {
+  if (p.genax[0]) {
     timing_begin(MUGPU_K_AXIS0);
-    const int rc = gen_axis0_project(p, pj, spec);
+    const int rc = gen_axis0_project(p, prec_of<T>(), pj, spec);
     timing_end(MUGPU_K_AXIS0);
     return rc;
   }
@@ -799,7 +800,7 @@ int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spec
   c_t<T>* spec = reinterpret_cast<c_t<T>*>(spectrum);
   // the fused x update and the early alpha are not carried by the passes of
   // this file
-  const bool carried = p.fastax[DIM - 1] || (sizeof(T) == 8 && p.genax[DIM - 1]);
+  const bool carried = p.fastax[DIM - 1] || p.genax[DIM - 1];
   if (op.xvec && !carried) return MUGPU_EARG;
   if ((op.fin_alpha || op.out_mode == OUT_RUPD) && (sizeof(T) != 8 || !carried)) return MUGPU_EARG;
   p.packed = sizeof(T) == 8 && p.can_pack && pj.kind == MUGPU_PROJ_SMALL_STRAIN &&

@@ -143,7 +143,7 @@ struct ScalarFold {
 };
 constexpr int kFoldMax = 1024;
 
-// ---- passes of run-time length (FP64; fft_gen.hpp) -------------------------------
+// ---- passes of run-time length (fft_gen.hpp) -------------------------------
 constexpr int kGenMaxPass = 12;
 constexpr int kGenQ = 4;          // output pairs of a prime radix formed at once
 constexpr int kGenTB = 2;         // such tasks held per thread
@@ -208,7 +208,7 @@ struct FftPlan {
   int64_t nzblocks = 0;      // z-pass workgroups, the largest of nzb
   int64_t nzb[2] = {0, 0};   // c2r workgroups (p.Ap partials) per precision (0 FP64, 1 FP32)
   bool fastax[3] = {false, false, false};  // compile-time-length passes (fft_fast.hip)
-  // run-time-length passes of FP64 grids, per axis (genax: the axis has them)
+  // run-time-length passes per axis (genax: the axis has them)
   GenAxis gen[3];
   bool genax[3] = {false, false, false};
   GenShape gen_last[2], gen_axis0[2], gen_str[3][2];  // one line per component; packed
@@ -242,7 +242,7 @@ void force_variant(int pass, int prec, int variant);
 // this length, dimension and precision
 bool fast_variant_valid(int pass, int n, int dim, int prec, int variant);
 
-// general: FP64 passes of run-time length where they fit, packed symmetric
+// general: passes of run-time length where they fit, packed symmetric
 // lines.  Cells of the
 // FP32-refined solve go without: their x carries the FP32 rounding of its
 // inner solves (1.5e-6 relative), so a last-bit change of the FP64 residuals
@@ -311,11 +311,11 @@ int fast_r2c(FftPlan& p, int prec, const OpSpec& op, void* spec);
 int fast_c2r(FftPlan& p, int prec, const OpSpec& op, void* spec);
 int fast_strided(FftPlan& p, int prec, int ax, void* spec, int sign);
 int fast_axis0_project(FftPlan& p, int prec, const ProjParams& pj, void* spec);
-// FP64 passes along axes of run-time length (fft_gen_last.hip, fft_gen_axis.hip)
-int gen_r2c(FftPlan& p, const OpSpec& op, void* spec);
-int gen_c2r(FftPlan& p, const OpSpec& op, void* spec);
-int gen_strided(FftPlan& p, int ax, void* spec, int sign);
-int gen_axis0_project(FftPlan& p, const ProjParams& pj, void* spec);
+// passes along axes of run-time length (fft_gen_last.hip, fft_gen_axis.hip)
+int gen_r2c(FftPlan& p, int prec, const OpSpec& op, void* spec);
+int gen_c2r(FftPlan& p, int prec, const OpSpec& op, void* spec);
+int gen_strided(FftPlan& p, int prec, int ax, void* spec, int sign);
+int gen_axis0_project(FftPlan& p, int prec, const ProjParams& pj, void* spec);
 // the HBM pattern of the first-axis pass alone (n rows of plane k-points of nc
 // complex components, tiles of kp k-points), in place (fft_fast.hip)
 int line_pattern(void* data, int prec, int n, int64_t plane, int nc, int kp);
