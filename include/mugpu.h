@@ -91,8 +91,11 @@ int mugpu_device_info(char *name, int name_len, int *cu_count,
  * map and unmap memory each time; the blocks are for work on the library
  * stream.  mugpu_free of a pointer mugpu_alloc did not return (or already
  * freed) fails with MUGPU_EARG.  mugpu_release_cached (no reference
- * counterpart) returns the cached blocks to the device after the library
- * stream's work; an allocation that fails does so by itself and retries. */
+ * counterpart) returns the cached blocks, the directions that idle cells keep
+ * (mugpu_cg_steps) and the pinned memory of large downloads (16 MiB, taken
+ * by the first mugpu_download of 2 MiB or more) after the library
+ * stream's work; an allocation that fails gives back device memory by
+ * itself and retries. */
 int mugpu_alloc(size_t bytes, void **d_ptr);
 /* Test hook for the failure paths of the library's own device allocations
  * (no reference counterpart; for tests of out-of-memory handling): from now
@@ -279,7 +282,13 @@ int mugpu_scale_copy(double a, const void *d_x, void *d_y, int64_t n);
  *   run (one whose r.r is NaN counts and stops the loop), *new_rdr the r.r
  *   of the last.  The host reads back once per call instead of once per
  *   iteration; the arithmetic is that of mugpu_cg_step.  Ap is work space
- *   of this call (A p is not stored where the last pass updates r).  Where the last
+ *   of this call (A p is not stored where the last pass updates r).  In a
+ *   solve whose b = G b on a large grid (from 4 MB of packed components in
+ *   3D small strain, else from 32 MB per vector) the cell keeps up to eight
+ *   directions p, in at most 1/16 of the device's memory, and adds them to
+ *   x together: x, r and p are complete when the call returns.  That
+ *   memory is given back with the cell, by mugpu_release_cached and when an
+ *   allocation of this library finds the device full.  Otherwise, where the last
  *   axis has compiled passes (lengths 16, 32, 48, 64, 96, 128, 256, 512),
  *   the x update of an iteration is applied by the next iteration's first
  *   pass (which reads p anyway), so the x update of the last iteration of a call is left

@@ -157,6 +157,12 @@ struct mugpu_cell_s {
   // alpha comes from p . K p and r is updated by the last pass of the operator
   bool early_alpha = false;
   void *x_pend = nullptr, *p_pend = nullptr;
+  // directions of a chunk of such a solve's iterations (RingFlush): ring_len fields
+  // of ring_nf components and, if those are packed, one for r; nothing in it outlives
+  // a call, so it is given back when device memory runs out (rings_release)
+  double* ring = nullptr;
+  int ring_len = 0, ring_nf = 0;
+  bool ring_busy = false;
   // captured chunks of mugpu_cg_steps (small cells), by vectors, chunk
   // length and form of the first iteration
   struct CgGraph {
@@ -197,6 +203,112 @@ void pending_clear(mugpu_cell c) {
 }  // namespace
 
 int flush_x(mugpu_cell c);
+
+// Cells with a ring.  A call that uses one holds it (RingHold); a ring not held
+// can be freed from any thread, together with the graphs that point into it.
+namespace {
+std::mutex g_ring_mu;
+std::vector<mugpu_cell> g_ring_cells;
+
+void ring_free_locked(mugpu_cell c) {
+  (void)hipFree(c->ring);
+  c->ring = nullptr;
+  for (auto& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
+  c->graphs.clear();
+}
+
+// gives back the rings not in use; true if there was one
+bool rings_release() {
+  std::lock_guard<std::mutex> lk(g_ring_mu);
+  bool any = false;
+  for (size_t i = 0; i < g_ring_cells.size();) {
+    if (g_ring_cells[i]->ring_busy) {
+      ++i;
+      continue;
+    }
+    ring_free_locked(g_ring_cells[i]);
+    g_ring_cells.erase(g_ring_cells.begin() + (std::ptrdiff_t)i);
+    any = true;
+  }
+  return any;
+}
+
+void ring_drop(mugpu_cell c) {
+  std::lock_guard<std::mutex> lk(g_ring_mu);
+  for (size_t i = 0; i < g_ring_cells.size(); ++i)
+    if (g_ring_cells[i] == c) {
+      ring_free_locked(c);
+      g_ring_cells.erase(g_ring_cells.begin() + (std::ptrdiff_t)i);
+      break;
+    }
+}
+
+// components per voxel of a cell's CG vectors inside a chunk of iterations: the
+// packed ones where the passes take them (operator_impl's rule)
+int ring_components(mugpu_cell c) {
+  const bool sym = c->plan.can_pack && c->pj.kind == MUGPU_PROJ_SMALL_STRAIN && c->tan_kind == TAN_ISO;
+  return sym ? c->dim * (c->dim + 1) / 2 : c->nc;
+}
+
+struct RingHold {
+  mugpu_cell c;
+  bool ok = false;  // the cell has a ring for its present vectors
+  explicit RingHold(mugpu_cell cell) : c(cell) {
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    c->ring_busy = true;
+    ok = c->early_alpha && c->ring && c->ring_nf == ring_components(c);
+  }
+  ~RingHold() {
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    c->ring_busy = false;
+  }
+  bool sym() const { return c->ring_nf < c->nc; }
+  int64_t field() const { return c->N * c->ring_nf; }
+  double* slot(int i) const { return c->ring + (int64_t)i * field(); }  // slot(ring_len): r
+};
+
+// A ring for the cell's next chunks: kRing directions, or half as many, within
+// 1/16 of the device's memory.  Without one (too small a field, none fits, or the
+// device is full) x is updated by the passes, as in solves without an early alpha.
+// It takes a sweep's worth of bytes out of an iteration (and with packed vectors
+// two thirds of one more), which counts where HBM sets the pace: CG on full fields
+// 256^3 finite strain 147.9 -> 139.1 ms, 175x147x99 18.0 -> 17.4, but 63^3 (18 MB
+// a field) 3.42 -> 3.45 and 405^2 the same; packed 128^3 12.8 -> 11.2 ms, 64^3
+// 2.56 -> 2.39, 48^3 (5 MB) 2.00 -> 1.92; packed 2D, a quarter less instead of a
+// third, 512^2 (6 MB) 1.46 -> 1.48 ms.  The last level of cache takes most of the
+// difference below the limits.
+constexpr size_t kRingField = (size_t)32 << 20, kRingFieldSym3 = (size_t)4 << 20;
+void ring_ensure(mugpu_cell c) {
+  const int nf = ring_components(c);
+  if (sizeof(double) * (size_t)c->N * nf < (nf == 6 ? kRingFieldSym3 : kRingField)) return ring_drop(c);
+  {
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    if (c->ring && c->ring_nf == nf) return;
+  }
+  ring_drop(c);
+  size_t fr = 0, tot = 0;
+  if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  const size_t field = sizeof(double) * (size_t)c->N * nf;
+  for (int len = kRing; len >= kRing / 2; len /= 2) {
+    const size_t bytes = field * (len + (nf < c->nc ? 1 : 0));
+    if (bytes > tot / 16 || bytes > fr / 2) continue;
+    void* q = nullptr;
+    if (hipMalloc(&q, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      continue;
+    }
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    c->ring = (double*)q;
+    c->ring_len = len;
+    c->ring_nf = nf;
+    g_ring_cells.push_back(c);
+    return;
+  }
+}
+}  // namespace
 
 namespace {
 
@@ -449,7 +561,8 @@ int mugpu::dev_alloc(void** p, size_t bytes, const char* what) {
     (void)hipGetLastError();
     *p = nullptr;
     std::lock_guard<std::mutex> lk(g_alloc_mu);
-    if (!g_cached.empty()) {
+    const bool rings = rings_release();
+    if (!g_cached.empty() || rings) {
       (void)hipStreamSynchronize(g_stream);
       release_cached_locked();
       e = hipMalloc(p, bytes ? bytes : 16);
@@ -501,10 +614,13 @@ extern "C" int mugpu_alloc(size_t bytes, void** d_ptr) {
     return MUGPU_OK;
   }
   hipError_t e = hipMalloc(d_ptr, sz);
-  if (e != hipSuccess && !g_cached.empty()) {
+  if (e != hipSuccess) {
     (void)hipGetLastError();
-    release_cached_locked();
-    e = hipMalloc(d_ptr, sz);
+    const bool rings = rings_release();
+    if (!g_cached.empty() || rings) {
+      release_cached_locked();
+      e = hipMalloc(d_ptr, sz);
+    }
   }
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -557,6 +673,7 @@ static void stage_release();
 
 extern "C" int mugpu_release_cached(void) {
   stage_release();
+  (void)rings_release();
   std::lock_guard<std::mutex> lk(g_alloc_mu);
   if (g_cached.empty()) return MUGPU_OK;
   MUGPU_HIP(hipStreamSynchronize(g_stream));
@@ -1098,7 +1215,7 @@ extern "C" int mugpu_cell_create(int dim, const int* res, const double* lengths,
   if (!rc) rc = dev_alloc(&c->P, fb, "the stress field");
   if (!rc) rc = dev_alloc(&c->tmp, fb, "the cell's work field");
   if (!rc) rc = dev_alloc(&c->spectrum, sb, "the cell's spectrum");
-  if (!rc) rc = dev_alloc(&c->scal, sizeof(double) * SC_COUNT, "the CG scalars");
+  if (!rc) rc = dev_alloc(&c->scal, sizeof(double) * (SC_COUNT + kRing), "the CG scalars");
   if (!rc) rc = dev_alloc(&c->partials, sizeof(double) * kRedBlocks, "the partial sums");
   if (!rc) rc = dev_alloc(&c->ctl, sizeof(int) * CTL_COUNT, "the CG control words");
   if (rc) {
@@ -1109,7 +1226,7 @@ extern "C" int mugpu_cell_create(int dim, const int* res, const double* lengths,
   }
   (void)hipMemsetAsync(c->F, 0, fb, g_stream);
   (void)hipMemsetAsync(c->P, 0, fb, g_stream);
-  (void)hipMemsetAsync(c->scal, 0, sizeof(double) * SC_COUNT, g_stream);
+  (void)hipMemsetAsync(c->scal, 0, sizeof(double) * (SC_COUNT + kRing), g_stream);
   *out = c;
   return MUGPU_OK;
 }
@@ -1117,6 +1234,7 @@ extern "C" int mugpu_cell_create(int dim, const int* res, const double* lengths,
 extern "C" int mugpu_cell_destroy(mugpu_cell c) {
   if (!c) return MUGPU_OK;
   pending_clear(c);  // a pending x update is dropped with the cell
+  ring_drop(c);
   (void)hipStreamSynchronize(g_stream);
   for (auto& m : c->mats) {
     free_dev(m.d_pix);
@@ -1623,8 +1741,63 @@ extern "C" int mugpu_cg_start(mugpu_cell c, const void* d_rhs, void* d_x, void* 
   *rdr = g_host_scal[SC_RDR];
   *rhs_norm2 = g_host_scal[SC_TMP0];
   c->early_alpha = carried && g_host_scal[SC_TMP1] <= kInRange * kInRange * g_host_scal[SC_TMP0];
+  if (c->early_alpha) ring_ensure(c);
   return MUGPU_OK;
 }
+
+namespace {
+// the vectors of iteration i of a chunk of n over a ring
+struct RingChunk {
+  const RingHold& ring;
+  bool update_p;  // of the first iteration
+  int n;
+  double *x, *r, *p;
+  // Full fields: the directions go to the ring, except a first one taken as it is
+  // (it stays in p) and the last one, which goes to p (unless the first one is
+  // still needed there).  Packed: all go to the ring.
+  double* slot(int i) const {
+    const int m = ring.c->ring_len;
+    if (!ring.sym()) {
+      if (i == 0 && !update_p) return p;
+      if (i == n - 1 && (update_p || n > m)) return p;
+    }
+    return ring.slot(i % m);
+  }
+  void vectors(int i, OpSpec& op) const {
+    op.in_mode = i > 0 || update_p ? IN_TAN_PUPDATE : IN_TAN;
+    op.in = i == 0 ? p : slot(i - 1);
+    op.pout = slot(i);
+    op.aring = ring.c->scal + SC_COUNT;
+    if (!ring.sym()) return;
+    double* rs = ring.slot(ring.c->ring_len);
+    op.sym = true;
+    op.sym_flags = (i == 0 ? SYM_SRC_FULL : 0) | (op.in_mode == IN_TAN_PUPDATE ? SYM_UPDATE : 0) |
+                   (i == n - 1 ? SYM_OUT_FULL : 0);
+    op.rvec = i == 0 ? r : rs;
+    op.out = i == n - 1 ? r : rs;
+  }
+  // after iteration i: the x update of a full ring or of the chunk's rest
+  int flush(int i, const int* ctl) const {
+    const int m = ring.c->ring_len;
+    if ((i + 1) % m != 0 && i + 1 != n) return MUGPU_OK;
+    RingFlush f{};
+    f.base = i / m * m;
+    f.len = i - f.base + 1;
+    f.total = n;
+    for (int j = 0; j < f.len; ++j) f.p[j] = slot(f.base + j);
+    f.before = f.base > 0 ? slot(f.base - 1) : nullptr;
+    f.x = x;
+    f.p_out = p;
+    f.r_out = r;
+    f.rs = ring.slot(m);
+    f.scal = ring.c->scal;
+    f.aring = ring.c->scal + SC_COUNT;
+    f.ctl = ctl;
+    f.n = ring.c->N * ring.c->nc;
+    return ring_flush(f, ring.c->dim, ring.sym());
+  }
+};
+}  // namespace
 
 // the x update left by mugpu_cg_steps: x += alpha p (alpha of its last iteration)
 int flush_x(mugpu_cell c) {
@@ -1651,10 +1824,14 @@ extern "C" int mugpu_cg_step(mugpu_cell c, int update_p, void* d_x, void* d_r, v
   op.scal = c->scal;
   op.tan_kind = c->tan_kind;
   op.tangent = c->tan64;
+  const RingHold ring(c);
   if (c->early_alpha) {
+    const RingChunk ch{ring, update_p != 0, 1, (double*)d_x, (double*)d_r, (double*)d_p};
+    const bool sym = ring.ok && ring.sym();  // (as the iterations of mugpu_cg_steps)
     op.fin_alpha = c->scal;
     op.out_mode = OUT_RUPD;
     op.out = d_r;
+    if (sym) ch.vectors(0, op);
     op.ap_out = d_Ap;
     if (c->plan.fold_ok) op.fold_pk = c->partials;
     MUGPU_TRY(run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum));
@@ -1662,7 +1839,7 @@ extern "C" int mugpu_cg_step(mugpu_cell c, int update_p, void* d_x, void* d_r, v
       MUGPU_TRY(fold_beta((const double*)c->plan.partials, (int)c->plan.wg_c2r, c->scal, nullptr, 1));
     else
       MUGPU_TRY(finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA));
-    MUGPU_TRY(axpy_alpha(MUGPU_FP64, d_x, d_p, c->scal, n));
+    MUGPU_TRY(sym ? ch.flush(0, nullptr) : axpy_alpha(MUGPU_FP64, d_x, d_p, c->scal, n));
   } else {
     op.out_mode = OUT_DOT;
     op.out = d_Ap;
@@ -1709,8 +1886,10 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
   // a solve with an early alpha; the last one is left pending for the next call
   // or mugpu_cg_finish where the passes are compiled, else applied below
   const bool pends = c->plan.fastax[c->dim - 1];
-  const bool fuse = pends || early;
-  const bool pend_here = c->x_pending && c->x_pend == d_x && c->p_pend == d_p && update_p;
+  const RingHold ring(c);
+  const RingChunk ch{ring, update_p != 0, max_steps, (double*)d_x, (double*)d_r, (double*)d_p};
+  const bool fuse = !ring.ok && (pends || early);
+  const bool pend_here = fuse && c->x_pending && c->x_pend == d_x && c->p_pend == d_p && update_p;
   if (c->x_pending && !pend_here) MUGPU_TRY(flush_x(c));
   // the first r2c applies the pending update with scal[SC_ALPHA]
   if (pend_here) MUGPU_TRY(scal_copy(c->scal, SC_XALPHA, SC_ALPHA));
@@ -1720,15 +1899,15 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
     op.in_mode = (i > 0 || update_p) ? IN_TAN_PUPDATE : IN_TAN;
     op.xvec = fuse && (i > 0 || pend_here) ? d_x : nullptr;
     op.fold_iter = i;
+    if (ring.ok) ch.vectors(i, op);
     int e = run_operator(c->plan, MUGPU_FP64, op, c->pj, c->spectrum);
-    if (op.fold_pk)
-      return e != MUGPU_OK || i + 1 < max_steps
-                 ? e
-                 : fold_beta((const double*)c->plan.partials, (int)c->plan.wg_c2r, c->scal, c->ctl, max_steps);
-    if (early)
-      return e != MUGPU_OK ? e
-                           : finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA,
-                                      c->ctl);
+    if (early) {
+      if (e == MUGPU_OK && !op.fold_pk)
+        e = finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_BETA, c->ctl);
+      else if (e == MUGPU_OK && i + 1 == max_steps)
+        e = fold_beta((const double*)c->plan.partials, (int)c->plan.wg_c2r, c->scal, c->ctl, max_steps);
+      return e == MUGPU_OK && ring.ok ? ch.flush(i, c->ctl) : e;
+    }
     if (e == MUGPU_OK)
       e = finalize((const double*)c->plan.partials, c->plan.wg_c2r, c->scal, FIN_ALPHA, c->ctl);
     if (e == MUGPU_OK)
@@ -1744,10 +1923,10 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
   const bool graph = g_cg_graphs && n <= kCgGraphMaxValues && g_timing_class < 0;
   if (graph) {
     hipGraphExec_t ex = nullptr;
-    const int fu = update_p ? 1 : 0, fx = pend_here ? 1 : 0;
+    const int fu = update_p ? 1 : 0, fx = pend_here ? 1 : 0, el = (early ? 1 : 0) + (ring.ok ? 2 : 0);
     for (auto& g : c->graphs)
       if (g.x == d_x && g.r == d_r && g.p == d_p && g.Ap == d_Ap && g.steps == max_steps &&
-          g.first_update_p == fu && g.first_x == fx && g.early == (early ? 1 : 0))
+          g.first_update_p == fu && g.first_x == fx && g.early == el)
         ex = g.exec;
     if (!ex) {
       hipGraph_t gr = nullptr;
@@ -1767,7 +1946,7 @@ extern "C" int mugpu_cg_steps(mugpu_cell c, int update_p, void* d_x, void* d_r, 
           (void)hipGraphExecDestroy(c->graphs.front().exec);
           c->graphs.erase(c->graphs.begin());
         }
-        c->graphs.push_back({d_x, d_r, d_p, d_Ap, max_steps, fu, fx, early ? 1 : 0, ex});
+        c->graphs.push_back({d_x, d_r, d_p, d_Ap, max_steps, fu, fx, el, ex});
       }
     }
     if (rc == MUGPU_OK && hipGraphLaunch(ex, g_stream) != hipSuccess)

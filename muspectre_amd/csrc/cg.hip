@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kRT) void k_dot(const A* __restrict__ a, const B* _
 
 __global__ __launch_bounds__(1024) void k_finalize(const double* __restrict__ partials,
                                                    int64_t count, double* scal, int mode,
-                                                   int* ctl) {
+                                                   int* ctl, double* aring) {
   if (ctl && !ctl[CTL_ACTIVE]) return;
   __shared__ double red[1024];
   double acc = 0.0;
@@ -49,6 +49,7 @@ __global__ __launch_bounds__(1024) void k_finalize(const double* __restrict__ pa
       case FIN_ALPHA:
         scal[SC_PAP] = s;
         scal[SC_ALPHA] = scal[SC_RDR] / s;
+        if (aring) aring[ctl ? ctl[CTL_ITER] & (kRing - 1) : 0] = scal[SC_ALPHA];
         break;
       case FIN_BETA:
         scal[SC_NEWRDR] = s;
@@ -143,6 +144,57 @@ __global__ __launch_bounds__(1024) void k_cg_start_final(const double* __restric
     scal[SC_RDR] = t;
     scal[SC_TMP0] = t;
     scal[SC_TMP1] = u;
+  }
+}
+
+// The x update of up to kRing CG iterations at once: per iteration x then costs
+// one read of p and 1 / kRing of a sweep of x instead of a whole sweep (read and
+// write).  In the order of the iterations, with the arithmetic of k_axpy_alpha.
+template <int DIM, bool SYM>
+__global__ __launch_bounds__(kRT) void k_ring_flush(RingFlush a) {
+  constexpr int NC = DIM * DIM, NL = nb_lines(DIM, SYM);
+  int cnt = a.len;
+  bool fin = a.base + a.len == a.total;
+  if (a.ctl && !a.ctl[CTL_ACTIVE]) {
+    // (an iteration whose r . r is NaN ended the loop without being counted)
+    const double s = a.scal[SC_NEWRDR];
+    const int left = a.ctl[CTL_ITER] + (s == s ? 0 : 1) - a.base;
+    // (with folded scalars the test after the last iteration of a full ring comes
+    // with the next iteration: the loop then turns out to have stopped here, with
+    // left = 0, and p and r are still to be copied)
+    if (left < 0 || (left == 0 && !a.before)) return;
+    if (left <= cnt) {
+      cnt = left;
+      fin = true;
+    }
+  }
+  const double* const pk = cnt > 0 ? a.p[cnt - 1] : a.before;
+  const bool all = a.base + cnt == a.total;
+  double al[kRing];
+#pragma unroll
+  for (int j = 0; j < kRing; ++j) al[j] = a.aring[(a.base + j) & (kRing - 1)];
+  const int64_t stride = (int64_t)gridDim.x * kRT;
+  for (int64_t e = (int64_t)blockIdx.x * kRT + threadIdx.x; e < a.n; e += stride) {
+    int64_t g = e;
+    if (SYM) {
+      const int64_t v = e / NC;
+      g = v * NL + line_of<DIM, SYM>((int)(e - v * NC));
+    }
+    double x = a.x[e], pj[kRing], last = cnt > 0 ? 0.0 : pk[g];
+#pragma unroll
+    for (int j = 0; j < kRing; ++j)
+      if (j < cnt) pj[j] = a.p[j][g];
+#pragma unroll
+    for (int j = 0; j < kRing; ++j)
+      if (j < cnt) {
+        x += al[j] * pj[j];
+        last = pj[j];
+      }
+    a.x[e] = x;
+    if (fin) {
+      if (pk != a.p_out) a.p_out[e] = last;
+      if (SYM && !all) a.r_out[e] = a.rs[g];
+    }
   }
 }
 
@@ -487,9 +539,9 @@ int set_ctl(int* ctl, int maxit, double* d_scal, double tol2) {
   return MUGPU_OK;
 }
 
-int finalize(const double* d_partials, int64_t count, double* d_scal, int mode, int* ctl) {
+int finalize(const double* d_partials, int64_t count, double* d_scal, int mode, int* ctl, double* aring) {
   hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, stream(), d_partials, count, d_scal, mode,
-                     ctl);
+                     ctl, aring);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }
@@ -517,6 +569,22 @@ int axpy_alpha(int prec, void* x, const void* p, const double* d_scal, int64_t n
   else
     hipLaunchKernelGGL((k_axpy_alpha<float>), dim3(g), dim3(kRT), 0, stream(), (float*)x,
                        (const float*)p, d_scal, n, slot);
+  MUGPU_HIP(hipGetLastError());
+  return MUGPU_OK;
+}
+
+int ring_flush(const RingFlush& a, int dim, bool sym) {
+  if (a.len < 1 || a.len > kRing) return MUGPU_EARG;
+  const dim3 g(grid_for(a.n, kRedBlocks)), b(kRT);
+  timing_begin(MUGPU_K_CG_UPDATE);
+  if (dim == 3) {
+    if (sym) hipLaunchKernelGGL((k_ring_flush<3, true>), g, b, 0, stream(), a);
+    else hipLaunchKernelGGL((k_ring_flush<3, false>), g, b, 0, stream(), a);
+  } else {
+    if (sym) hipLaunchKernelGGL((k_ring_flush<2, true>), g, b, 0, stream(), a);
+    else hipLaunchKernelGGL((k_ring_flush<2, false>), g, b, 0, stream(), a);
+  }
+  timing_end(MUGPU_K_CG_UPDATE);
   MUGPU_HIP(hipGetLastError());
   return MUGPU_OK;
 }

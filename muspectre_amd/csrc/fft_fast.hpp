@@ -195,6 +195,14 @@ constexpr size_t lds_lines() {
   constexpr size_t stage = PK ? (size_t)z_rows(N, DIM, H) * N * DIM * DIM * sizeof(T) : 0;
   return lines > stage ? lines : stage;
 }
+// of the r2c pass in an input mode
+template <typename T, int N, int DIM, int IN, int H, bool PK>
+constexpr size_t lds_r2c() {
+  if (IN != IN_TAN_S) return lds_lines<T, N, DIM, H, PK>();
+  constexpr size_t lines = (size_t)N * lstride(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK)) * sizeof(c_t<T>);
+  constexpr size_t stage = (size_t)z_rows(N, DIM, H) * N * nb_lines(DIM, PK) * sizeof(T);
+  return lines > stage ? lines : stage;
+}
 template <typename T, int N, int E, int DIM, int H, bool PK>
 constexpr size_t lds_c2r() {
   constexpr int NL = nb_lines(DIM, PK);
@@ -429,6 +437,7 @@ struct LArgs {
   T* x;               // OpSpec::xvec (IN_TAN_PUPDATE_X kernels only)
   T* ap;              // OpSpec::ap_out (OUT_RUPD kernels only)
   ScalarFold fold;    // (FP64)
+  int sym;            // SymFlags (IN_TAN_S and OUT_RUPD_S kernels)
 };
 
 // ISO: the tangent is known to be isotropic (TAN_ISO), which the compiler
@@ -446,7 +455,8 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
     // packed K : p (or the symmetric part of the field) of its voxels in
     // registers, and the lines take the place of the staged rows
     static_assert(IN == IN_PLAIN || ISO, "packed lines need a symmetric K : p");
-    constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
+    constexpr bool S = IN == IN_TAN_S, XU = IN == IN_TAN_PUPDATE_X, PU = IN == IN_TAN_PUPDATE || XU || S;
+    constexpr int NF = S ? NL : NC;  // components of the staged field
     T beta = PU ? (T)a.scal[SC_BETA] : T(0);
     if constexpr (sizeof(T) == 8 && PU) {
       if (a.fold.rr) {
@@ -456,9 +466,11 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
       }
     }
     const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
-    constexpr int TOT = RB * N * NC, kBatch = 8;
-    const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
-    for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
+    constexpr int TOT = RB * N * NF, kBatch = 8;
+    const int64_t base = row0 * N * NF, lim = a.rows * N * NF;
+    if constexpr (S) {
+      sym_stage<T, DIM, kBatch>(a.in, a.rvec, a.pout, a.sym, beta, base, lim, TOT, NT, sr);
+    } else for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
       T pv[kBatch], rv[kBatch], xv[kBatch];
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
@@ -493,8 +505,12 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
       const int e = threadIdx.x + i * NT;
       if (e < RB * N) {
         T pv[NC], dp[NC];
+        if constexpr (S) {
+          unpack_lines<T, DIM>(sr + e * NF, pv);
+        } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) pv[c] = sr[e * NC + c];
+          for (int c = 0; c < NC; ++c) pv[c] = sr[e * NC + c];
+        }
         if (IN != IN_PLAIN) {
           // (rows beyond the last one: p is zero and the tangent read is the
           // last voxel's, so K : p is zero)
@@ -673,11 +689,11 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
 
 template <typename T, int N, int E, int DIM, int IN, bool ISO, int H, bool PK>
 __global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E))
-MUGPU_WPE(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), (lds_lines<T, N, DIM, H, PK>())) void k_r2c_fast(LArgs<T> a) {
+MUGPU_WPE(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), (lds_r2c<T, N, DIM, IN, H, PK>())) void k_r2c_fast(LArgs<T> a) {
   if (a.active && !a.active[0]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   LArgs<T> b = a;
-  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), lds_lines<T, N, DIM, H, PK>()>(a.tw, smem);
+  b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), lds_r2c<T, N, DIM, IN, H, PK>()>(a.tw, smem);
   r2c_body<T, N, E, DIM, IN, ISO, H, PK>(b, smem, blockIdx.x);
 }
 
@@ -718,8 +734,9 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   constexpr int NT = L * (N / E), NH = N / 2 + 1;
   c_t<T>* s = reinterpret_cast<c_t<T>*>(smem);
   const int64_t row0 = bx * RB;
+  constexpr bool S = OUT == OUT_RUPD_S, RU = OUT == OUT_RUPD || S;
   T alpha = T(0);
-  if constexpr (sizeof(T) == 8 && OUT == OUT_RUPD) {
+  if constexpr (sizeof(T) == 8 && RU) {
     if (a.fold.pk) {
       alpha = fold_alpha(a.fold, fold_sum(a.fold.pk, a.fold.npk, reinterpret_cast<double*>(smem)));
       __syncthreads();
@@ -782,8 +799,16 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
   const T* sr = reinterpret_cast<const T*>(smem);
   const int64_t base = row0 * N * NC, lim = a.rows * N * NC;
   double acc = 0.0;
-  const T al = OUT != OUT_RUPD ? T(0) : a.fold.pk ? alpha : (T)a.scal[SC_ALPHA];
-  {
+  const T al = !RU ? T(0) : a.fold.pk ? alpha : (T)a.scal[SC_ALPHA];
+  if constexpr (S) {
+    const int64_t left = (a.rows - row0) * N * NL;
+    constexpr int TOT = RB * N * NL;
+    acc = sym_rupd<T, DIM, 8>(a.rvec, a.out, a.ap, a.sym, al, row0 * N * NL, left < TOT ? (int)left : TOT, NT,
+                              [&](int v, int c) {
+                                const int r = v / N, m = v - r * N;
+                                return sr[2 * (m * LS + (r >> 1) * NL + c) + (r & 1)];
+                              });
+  } else {
     constexpr int TOT = RB * N * NC, kBatch = 8;
     for (int e0 = 0; e0 < TOT; e0 += kBatch * NT) {
       T dv[kBatch];
@@ -816,7 +841,7 @@ __device__ __forceinline__ void c2r_body(const LArgs<T>& a, unsigned char* smem,
       }
     }
   }
-  if constexpr (OUT == OUT_RUPD) {
+  if constexpr (RU) {
     __syncthreads();
     const double t = block_sum_waves(acc, reinterpret_cast<double*>(smem), NT);
     if (threadIdx.x == 0) a.partials[bx] = t;

@@ -31,8 +31,11 @@ int c2r_n(FftPlan& p, const OpSpec& op, void* spec) {
     a.scal = op.scal;
     a.ap = reinterpret_cast<T*>(op.ap_out);
     a.fold = p.fold;
+    a.rvec = reinterpret_cast<const T*>(op.rvec);
+    a.sym = op.sym_flags;
     if (p.packed) {
-      if (op.out_mode == OUT_RUPD) c2r_go<T, N, E, DIM, OUT_RUPD, H, true>(p, a);
+      if (op.sym) c2r_go<T, N, E, DIM, OUT_RUPD_S, H, true>(p, a);
+      else if (op.out_mode == OUT_RUPD) c2r_go<T, N, E, DIM, OUT_RUPD, H, true>(p, a);
       else if (op.out_mode == OUT_DOT) c2r_go<T, N, E, DIM, OUT_DOT, H, true>(p, a);
       else c2r_go<T, N, E, DIM, OUT_PLAIN, H, true>(p, a);
       MUGPU_HIP(hipGetLastError());

@@ -11,7 +11,7 @@ namespace {
 template <typename T, int N, int E, int DIM, int IN, bool ISO, int H, bool PK>
 void r2c_go(FftPlan& p, const LArgs<T>& a) {
   constexpr int RB = z_rows(N, DIM, H), NT = RB / 2 * nb_lines(DIM, PK) * (N / E);
-  constexpr size_t lds = TwLds<T, N>::total(lds_lines<T, N, DIM, H, PK>());
+  constexpr size_t lds = TwLds<T, N>::total(lds_r2c<T, N, DIM, IN, H, PK>());
   const dim3 grid((unsigned)((a.rows + RB - 1) / RB));
   if (sizeof(T) == 8) p.wg_r2c = grid.x;
   hipLaunchKernelGGL((k_r2c_fast<T, N, E, DIM, IN, ISO, H, PK>), grid, dim3(NT), lds, stream(), a);
@@ -39,10 +39,12 @@ int r2c_n(FftPlan& p, const OpSpec& op, void* spec) {
   const bool iso = op.tan_kind == TAN_ISO;
   // the fused x update goes with the p update only
   const bool xu = op.xvec != nullptr;
-  if (xu && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
+  if (xu && (op.in_mode != IN_TAN_PUPDATE || op.sym)) return MUGPU_EARG;
   if constexpr (sizeof(T) == 8) {
+    a.sym = op.sym_flags;
     if (p.packed) {
-      if (op.in_mode == IN_PLAIN) r2c_go<T, N, E, DIM, IN_PLAIN, false, H, true>(p, a);
+      if (op.sym) r2c_go<T, N, E, DIM, IN_TAN_S, true, H, true>(p, a);
+      else if (op.in_mode == IN_PLAIN) r2c_go<T, N, E, DIM, IN_PLAIN, false, H, true>(p, a);
       else if (op.in_mode == IN_TAN) r2c_go<T, N, E, DIM, IN_TAN, true, H, true>(p, a);
       else if (xu) r2c_go<T, N, E, DIM, IN_TAN_PUPDATE_X, true, H, true>(p, a);
       else r2c_go<T, N, E, DIM, IN_TAN_PUPDATE, true, H, true>(p, a);

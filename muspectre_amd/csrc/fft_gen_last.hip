@@ -33,6 +33,7 @@ struct GLast {
   const c_t<T>* tw;
   const int* active;  // FftPlan::active
   ScalarFold fold;
+  int sym;  // SymFlags
 };
 
 // LDS: [lines: n * LS complex][twiddles: n complex][staging: 2 rows of NC
@@ -52,18 +53,22 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast<T> a) {
   // (the flag and the partial sums are read together)
   const int on = a.active ? a.active[0] : 1;
   const int64_t row0 = (int64_t)blockIdx.x * a.RB;
-  constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X, XU = IN == IN_TAN_PUPDATE_X;
+  constexpr bool S = IN == IN_TAN_S, XU = IN == IN_TAN_PUPDATE_X;
+  constexpr bool PU = IN == IN_TAN_PUPDATE || XU || S;
+  constexpr int NF = S ? NL : NC;  // components of the staged field
   double beta = PU ? a.scal[SC_BETA] : 0.0;
   const double rr = PU && a.fold.rr ? fold_sum(a.fold.rr, a.fold.nrr, red) : 0.0;
   if (!on || (PU && a.fold.rr && !fold_beta_test(a.fold, rr, beta))) return;
   const double al = XU ? a.scal[SC_ALPHA] : 0.0;
   double acc = 0.0;  // p . K p
   for (int r0 = 0; r0 < a.RB; r0 += 2) {
-    const int64_t base = (row0 + r0) * n * NC, lim = a.rows * n * NC;
-    const int tot = 2 * n * NC;
+    const int64_t base = (row0 + r0) * n * NF, lim = a.rows * n * NF;
+    const int tot = 2 * n * NF;
     constexpr int KB = 4;
     if (r0) __syncthreads();  // the staged rows before have been read
-    for (int e0 = 0; e0 < tot; e0 += KB * NT) {
+    if constexpr (S) {
+      sym_stage<T, DIM, KB>(a.in, a.rvec, a.pout, a.sym, (T)beta, base, lim, tot, NT, sp);
+    } else for (int e0 = 0; e0 < tot; e0 += KB * NT) {
       T pv[KB], rv[KB], xv[KB];
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
@@ -98,8 +103,12 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_r2c(GLast<T> a) {
       for (int e = threadIdx.x; e < 2 * n; e += NT) {
         const int r = e >= n, m = e - r * n;
         T p[NC], dp[NC];
+        if constexpr (S) {
+          unpack_lines<T, DIM>(sp + e * NF, p);
+        } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) p[c] = sp[e * NC + c];
+          for (int c = 0; c < NC; ++c) p[c] = sp[e * NC + c];
+        }
         if (KIND >= 0 && row0 + r0 + r < a.rows) {
           tangent_product<T, DIM>(KIND, a.tan, (row0 + r0 + r) * n + m, p, dp);
 #pragma unroll
@@ -174,7 +183,8 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast<T> a) {
   const int stage = RB * nh * NL;  // staged values; the twiddles follow the larger of the two
   c_t<T>* tw = s + (n * LS > stage ? n * LS : stage);
   const int on = a.active ? a.active[0] : 1;
-  const bool fold = OUT == OUT_RUPD && a.fold.pk;
+  constexpr bool S = OUT == OUT_RUPD_S, RU = OUT == OUT_RUPD || S;
+  const bool fold = RU && a.fold.pk;
   const double pk = fold ? fold_sum(a.fold.pk, a.fold.npk, red) : 0.0;
   if (!on) return;
   const double alpha = fold ? fold_alpha(a.fold, pk) : 0.0;
@@ -232,9 +242,15 @@ __global__ __launch_bounds__(kGenMaxNT) void k_gen_c2r(GLast<T> a) {
   auto none_st = [](int, c_t<T>) {};
   gen_fft<T, CLS, +1, false, false>(a.ax, a.P, p, act, s + l, LS, tw, none_ld, none_st);
   const T* sr = reinterpret_cast<const T*>(smem);
-  const double al = OUT != OUT_RUPD ? 0.0 : fold ? alpha : a.scal[SC_ALPHA];
+  const double al = !RU ? 0.0 : fold ? alpha : a.scal[SC_ALPHA];
   double acc = 0.0;
-  for (int r = 0; r < RB; ++r) {
+  if constexpr (S) {
+    for (int r = 0; r < RB && row0 + r < a.rows; ++r) {
+      const T* sl = sr + 2 * ((r >> 1) * NL) + (r & 1);
+      acc += sym_rupd<T, DIM, 4>(a.rvec, a.out, a.ap, a.sym, (T)al, (row0 + r) * n * NL, n * NL, NT,
+                                 [&](int m, int c) { return sl[2 * (m * LS + c)]; });
+    }
+  } else for (int r = 0; r < RB; ++r) {
     if (row0 + r >= a.rows) break;
     const int64_t base = (row0 + r) * n * NC;
     const T* sl = sr + 2 * ((r >> 1) * NL) + (r & 1);
@@ -289,6 +305,7 @@ void fill(FftPlan& p, const OpSpec& op, void* spec, const GenShape& g, GLast<T>&
   a.dotv = static_cast<const T*>(op.dotv);
   a.x = static_cast<T*>(op.xvec);
   a.ap = static_cast<T*>(op.ap_out);
+  a.sym = op.sym_flags;
   a.partials = static_cast<double*>(p.partials);
   a.rows = p.N / p.res[d];
   a.RB = g.mult * 2;
@@ -315,7 +332,15 @@ int r2c_launch(FftPlan& p, const OpSpec& op, void* spec) {
   } else {
     p.wg_r2c = grid.x;
     if (a.fold.pk) a.partials = a.fold.pk;
-    if (op.xvec && op.in_mode != IN_TAN_PUPDATE) return MUGPU_EARG;
+    if (op.xvec && (op.in_mode != IN_TAN_PUPDATE || op.sym)) return MUGPU_EARG;
+    if constexpr (PK) {
+      if (op.sym) {
+        const size_t less = (size_t)2 * a.ax.n * (DIM * DIM - nb_lines(DIM, PK)) * sizeof(T);
+        hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_TAN_S, PK>), grid, block, g.lds - less, stream(), a);
+        MUGPU_HIP(hipGetLastError());
+        return MUGPU_OK;
+      }
+    }
     switch (op.in_mode) {
       case IN_PLAIN: hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_PLAIN, PK>), grid, block, g.lds, stream(), a); break;
       case IN_TAN: hipLaunchKernelGGL((k_gen_r2c<T, CLS, DIM, IN_TAN, PK>), grid, block, g.lds, stream(), a); break;
@@ -342,6 +367,13 @@ int c2r_launch(FftPlan& p, const OpSpec& op, void* spec) {
     hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_PLAIN, PK>), grid, block, g.lds_bwd, stream(), a);
   } else {
     p.wg_c2r = grid.x;
+    if constexpr (PK) {
+      if (op.sym) {
+        hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_RUPD_S, PK>), grid, block, g.lds_bwd, stream(), a);
+        MUGPU_HIP(hipGetLastError());
+        return MUGPU_OK;
+      }
+    }
     if (op.out_mode == OUT_RUPD)
       hipLaunchKernelGGL((k_gen_c2r<T, CLS, DIM, OUT_RUPD, PK>), grid, block, g.lds_bwd, stream(), a);
     else if (op.out_mode == OUT_DOT)

@@ -806,8 +806,10 @@ int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spec
   p.packed = sizeof(T) == 8 && p.can_pack && pj.kind == MUGPU_PROJ_SMALL_STRAIN &&
              (op.in_mode == IN_PLAIN || op.tan_kind == TAN_ISO) &&
              (p.general || op.out_mode != OUT_PLAIN);
+  if (op.sym && !(p.packed && op.fin_alpha && op.rvec && op.pout)) return MUGPU_EARG;
   p.fold = ScalarFold{};
   if (op.fin_alpha && op.fold_pk) {
+    p.fold.aring = op.aring;
     p.fold.pk = op.fold_pk;
     p.fold.iter = op.fold_iter;
     p.fold.ctl = const_cast<int*>(p.active);
@@ -822,7 +824,7 @@ int operator_impl(FftPlan& p, const OpSpec& op, const ProjParams& pj, void* spec
   p.fold.npk = (int)p.wg_r2c;
   if (op.fin_alpha && !op.fold_pk)
     MUGPU_TRY(finalize((const double*)p.partials, p.wg_r2c, op.fin_alpha, FIN_ALPHA,
-                       const_cast<int*>(p.active)));
+                       const_cast<int*>(p.active), op.aring));
   if (DIM == 3) MUGPU_TRY(launch_strided<T>(p, 1, p.yW, spec, -1));
   if (pj.kind >= 0) {
     MUGPU_TRY((launch_project<T, DIM>(p, pj, spec)));

@@ -140,8 +140,12 @@ struct ScalarFold {
   int iter = 0;                // iterations of the chunk already run
   int* ctl = nullptr;          // CTL_* words (r2c with rr)
   double* scal = nullptr;
+  double* aring = nullptr;     // OpSpec::aring
 };
 constexpr int kFoldMax = 1024;
+// directions of a chunk of CG iterations kept before they are added to x
+// (ring_flush); alpha of iteration i in aring[i % kRing]
+constexpr int kRing = 8;
 
 // ---- passes of run-time length (fft_gen.hpp) -------------------------------
 constexpr int kGenMaxPass = 12;
@@ -261,11 +265,20 @@ struct ProjParams {
 // input stage of the last-axis r2c pass
 // IN_TAN_PUPDATE_X: kernel form of IN_TAN_PUPDATE that also applies x +=
 // alpha p_old (chosen by the launcher when OpSpec::xvec is set)
-enum InMode { IN_PLAIN = 0, IN_TAN = 1, IN_TAN_PUPDATE = 2, IN_TAN_PUPDATE_X = 3 };
+// IN_TAN_S: kernel form of IN_TAN and IN_TAN_PUPDATE for packed symmetric CG
+// vectors (OpSpec::sym)
+enum InMode { IN_PLAIN = 0, IN_TAN = 1, IN_TAN_PUPDATE = 2, IN_TAN_PUPDATE_X = 3, IN_TAN_S = 4 };
 // output stage of the last-axis c2r pass
 // OUT_RUPD: r += alpha A p with the partials of r . r, for solves whose alpha is
 // known before the inverse transform (OpSpec::fin_alpha)
-enum OutMode { OUT_PLAIN = 0, OUT_DOT = 1, OUT_RUPD = 2 };
+// OUT_RUPD_S: kernel form of OUT_RUPD for packed symmetric CG vectors
+enum OutMode { OUT_PLAIN = 0, OUT_DOT = 1, OUT_RUPD = 2, OUT_RUPD_S = 3 };
+// forms of a pass over packed symmetric CG vectors
+enum SymFlags {
+  SYM_SRC_FULL = 1,  // p and r come from fields of dim^2 components
+  SYM_UPDATE = 2,    // p = -r + beta p (else p is taken as it is)
+  SYM_OUT_FULL = 4   // r goes to a field of dim^2 components
+};
 
 struct OpSpec {
   int in_mode = IN_PLAIN;
@@ -292,6 +305,12 @@ struct OpSpec {
   // partials of p . K p, where the scalars may be folded into the passes
   double* fold_pk = nullptr;
   int fold_iter = 0;             // iterations of the chunk already run; > 0: beta is folded too
+  // packed runs with an early alpha: pout holds the packed components of p
+  // (always written), in and rvec (the r that is read) too unless
+  // SYM_SRC_FULL, out (the r that is written) unless SYM_OUT_FULL
+  bool sym = false;
+  int sym_flags = 0;
+  double* aring = nullptr;       // also store alpha in aring[iteration % kRing]
 };
 
 // full operator: r2c (with input stage) -> [axis passes] -> projection ->
@@ -360,8 +379,9 @@ int dot_device(int prec, const void* a, const void* b, int64_t n, double* d_part
 // ctl (optional, CTL_* words): skip when ctl[CTL_ACTIVE] == 0; FIN_BETA then
 // also applies SolverCG's loop test (ctl[CTL_ITER] + 1 < ctl[CTL_MAXIT] and
 // r.r > scal[SC_TOL2]) and clears CTL_ACTIVE when it fails
+// aring (FIN_ALPHA): OpSpec::aring
 int finalize(const double* d_partials, int64_t count, double* d_scal, int mode,
-             int* ctl = nullptr);
+             int* ctl = nullptr, double* aring = nullptr);
 // ctl = {active, 0 iterations, maxit}, scal[SC_TOL2] = tol2 (on the stream)
 int set_ctl(int* ctl, int maxit, double* d_scal, double tol2);
 enum FinalizeMode { FIN_ALPHA = 0, FIN_BETA = 1, FIN_STORE_TMP0 = 2, FIN_STORE_TMP1 = 3,
@@ -378,6 +398,22 @@ int scal_copy(double* d_scal, int from, int to);
 // beta after the last iteration of a folded chunk (ctl != null: where the chunk
 // still ran; `iters` iterations of it were queued) or after a single step
 int fold_beta(const double* rr, int count, double* d_scal, int* ctl, int iters);
+// x += sum alpha_i p_i over the iterations [base, base + len) of a chunk that were
+// run, then, after the last one run, p and (sym) r in their full fields
+struct RingFlush {
+  const double* p[kRing];  // directions, packed symmetric with `sym`
+  const double* before;    // direction of iteration base - 1, null for base = 0
+  double* x;
+  double* p_out;
+  double* r_out;
+  const double* rs;      // sym: packed r, copied to r_out if the last iteration has not run
+  const double* scal;
+  const double* aring;
+  const int* ctl;        // CTL_* words, null: every iteration was run
+  int64_t n;             // values of x
+  int base, len, total;  // total: iterations of the chunk
+};
+int ring_flush(const RingFlush& a, int dim, bool sym);
 // start of an FP64 solve: x = 0, r = -b, p = b; b.b into scal[SC_RDR] and
 // scal[SC_TMP0], |b - g|^2 into scal[SC_TMP1]
 int cg_start_vectors(const double* b, const double* g, double* x, double* r, double* p, int64_t n,

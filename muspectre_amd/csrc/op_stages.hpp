@@ -29,6 +29,17 @@ template <int DIM, bool PK>
 __host__ __device__ constexpr int line_of(int c) {
   return PK ? sym_line<DIM>(c % DIM, c / DIM) : c;
 }
+// components i + DIM j and j + DIM i of line c
+template <int DIM>
+__device__ __forceinline__ void sym_pair(int c, int& a, int& b) {
+  a = DIM == 3 ? (0x367840 >> (4 * c)) & 15 : (0x230 >> (4 * c)) & 15;
+  b = DIM == 3 ? (0x125840 >> (4 * c)) & 15 : (0x130 >> (4 * c)) & 15;
+}
+template <typename T, int DIM>
+__device__ __forceinline__ void unpack_lines(const T* q, T* f) {
+#pragma unroll
+  for (int c = 0; c < DIM * DIM; ++c) f[c] = q[line_of<DIM, true>(c)];
+}
 template <typename T, int DIM, bool PK>
 __device__ __forceinline__ void pack_lines(const T* f, T* q) {
   if constexpr (PK) {
@@ -412,6 +423,129 @@ __device__ __forceinline__ double fold_sum(const double* __restrict__ part, int 
   return red[0];
 }
 
+// ---- packed symmetric CG vectors ----------------------------------------------------
+// In a packed run p and r of a chunk of iterations hold the dim (dim + 1) / 2
+// components too (48 instead of 72 B per voxel in 3D, five sweeps per iteration);
+// the chunk's first iteration reads them from the full fields (the mean of two
+// mirrored components) and its last one writes r back to them.
+
+// p (packed) of `tot` values from `base` on, at most KB per thread in flight,
+// stored and staged in sp; with SYM_UPDATE p = -r + beta p.  Values at and beyond
+// `lim` are staged as zeros.
+template <typename T, int DIM, int KB>
+__device__ __forceinline__ void sym_stage(const T* in, const T* rvec, T* pout, int flags, T beta,
+                                          int64_t base, int64_t lim, int tot, int NT, T* sp) {
+  constexpr int NC = DIM * DIM, NL = sym_lines(DIM);
+  const bool upd = flags & SYM_UPDATE, full = flags & SYM_SRC_FULL;
+  const int last = lim - base < tot ? (int)(lim - base) - 1 : tot - 1;  // (>= 0: row 0 exists)
+  const int64_t vox0 = base / NL;
+  for (int e0 = 0; e0 < tot; e0 += KB * NT) {
+    T pv[KB], rv[KB];
+    if (full) {
+      T pw[KB], rw[KB];
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        int e = e0 + i * NT + (int)threadIdx.x;
+        if (e > last) e = last;
+        const int m = e / NL;
+        int ca, cb;
+        sym_pair<DIM>(e - m * NL, ca, cb);
+        const int64_t g = (vox0 + m) * NC;
+        pv[i] = in[g + ca];
+        pw[i] = in[g + cb];
+        rv[i] = rvec[g + ca];
+        rw[i] = rvec[g + cb];
+      }
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        pv[i] = T(0.5) * (pv[i] + pw[i]);
+        rv[i] = T(0.5) * (rv[i] + rw[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        int e = e0 + i * NT + (int)threadIdx.x;
+        if (e > last) e = last;
+        pv[i] = in[base + e];
+        rv[i] = rvec[base + e];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+      const int e = e0 + i * NT + (int)threadIdx.x;
+      if (e < tot) {
+        T x = T(0);
+        if (e <= last) {
+          x = upd ? -rv[i] + beta * pv[i] : pv[i];
+          pout[base + e] = x;
+        }
+        sp[e] = x;
+      }
+    }
+  }
+}
+
+// r += alpha A p over `tot` packed values from `base` on (A p of value e from
+// get(voxel, line)); returns this thread's part of r . r over all dim^2
+// components
+template <typename T, int DIM, int KB, typename G>
+__device__ __forceinline__ double sym_rupd(const T* rin, T* out, T* ap, int flags, T al, int64_t base,
+                                           int tot, int NT, const G& get) {
+  constexpr int NC = DIM * DIM, NL = sym_lines(DIM);
+  const bool sfull = flags & SYM_SRC_FULL, ofull = flags & SYM_OUT_FULL;
+  const int64_t vox0 = base / NL;
+  double acc = 0.0;
+  for (int e0 = 0; e0 < tot; e0 += KB * NT) {
+    T dv[KB];
+    if (sfull) {
+      T dw[KB];
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        int e = e0 + i * NT + (int)threadIdx.x;
+        if (e >= tot) e = tot - 1;
+        const int m = e / NL;
+        int ca, cb;
+        sym_pair<DIM>(e - m * NL, ca, cb);
+        const int64_t g = (vox0 + m) * NC;
+        dv[i] = rin[g + ca];
+        dw[i] = rin[g + cb];
+      }
+#pragma unroll
+      for (int i = 0; i < KB; ++i) dv[i] = T(0.5) * (dv[i] + dw[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < KB; ++i) {
+        const int e = e0 + i * NT + (int)threadIdx.x;
+        dv[i] = rin[base + (e < tot ? e : tot - 1)];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+      const int e = e0 + i * NT + (int)threadIdx.x;
+      if (e < tot) {
+        const int m = e / NL, c = e - m * NL;
+        const T val = get(m, c);
+        const T rv = dv[i] + al * val;
+        int ca, cb;
+        sym_pair<DIM>(c, ca, cb);
+        const int64_t g = (vox0 + m) * NC;
+        if (ofull) {
+          out[g + ca] = rv;
+          out[g + cb] = rv;
+        } else {
+          out[base + e] = rv;
+        }
+        if (ap) {
+          ap[g + ca] = val;
+          ap[g + cb] = val;
+        }
+        acc += (c < DIM ? 1.0 : 2.0) * ((double)rv * (double)rv);
+      }
+    }
+  }
+  return acc;
+}
+
 // r2c: beta and SolverCG's loop test after the previous iteration, from the sum s
 // of its r . r partials; false: the loop has stopped (workgroup 0 says so to the
 // later kernels)
@@ -435,6 +569,7 @@ __device__ __forceinline__ double fold_alpha(const ScalarFold& f, double s) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     f.scal[SC_PAP] = s;
     f.scal[SC_ALPHA] = al;
+    if (f.aring) f.aring[f.iter & (kRing - 1)] = al;
   }
   return al;
 }
