@@ -12,7 +12,8 @@ rows or k-points per workgroup (bit 1): half the LDS, more workgroups per CU
 also exists with an occupancy hint on its register allocation (bit 2),
 which changes its instruction schedule.  Which one
 is fastest depends on the pass, the length, the dimension and the
-precision.  This script times every variant of every pass on the GPU
+precision; the FP64 passes that also run on packed symmetric lines (small
+strain, isotropic tangent) are timed in that form too.  This script times every variant of every pass on the GPU
 (mugpu_fft_tune_pass, zeroed scratch buffers of a grid large enough to fill
 the device) and writes the table the library is compiled with
 (csrc/fft_tuned.inc).  A variant replaces the default only when it is
@@ -72,7 +73,7 @@ def main():
             for pass_ in (0, 1, 2, 3, 4):
                 if pass_ == 1 and dim == 2:
                     continue
-                for iso in ((0, 1) if pass_ == 0 else (0,)):
+                for iso in ((0, 1) if pass_ == 0 or (pass_ in (2, 3) and prec == _capi.FP64) else (0,)):
                     for n in LENGTHS:
                         res = grid(pass_, n, dim)
                         t = {}
@@ -95,7 +96,8 @@ def main():
                         if best:
                             entries.append((pass_, n, dim, prec, iso, best))
     lines = ["// Variants of the compile-time-length FFT passes: {pass, axis length, dim,",
-             "// precision (0 FP64, 1 FP32), isotropic tangent (r2c pass only), variant}.",
+             "// precision (0 FP64, 1 FP32), isotropic tangent (r2c pass; FP64: packed lines),",
+             "// variant}.",
              "// Written by muspectre_amd/autotune.py; entries absent here take variant 0.",
              "static const FastTuned kFastTuned[] = {",
              "    {-1, 0, 0, 0, 0, 0},"]

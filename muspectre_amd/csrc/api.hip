@@ -897,8 +897,9 @@ extern "C" int mugpu_fft_tune_pass(int dim, const int* res, int precision, int p
   for (int i = 0; i < 2; ++i) plan.fvar[pr][pass][i] = (unsigned char)variant;
   // (the plan's partials buffer holds the c2r partials of every variant)
   const size_t s = precision == MUGPU_FP64 ? 8 : 4;
-  // (the FP64 isotropic r2c runs with packed lines, as in a CG iteration)
-  plan.packed = pass == FV_R2C && precision == MUGPU_FP64 && iso != 0;
+  // (the FP64 passes of isotropic tangents run with packed lines, as in a CG
+  // iteration; the last-axis ones with packed vectors, as inside a chunk)
+  plan.packed = (pass == FV_R2C || pass == FV_C2R || pass == FV_AXIS0) && precision == MUGPU_FP64 && iso != 0;
   const int tk = iso ? TAN_ISO : (dim == 3 ? TAN_SYM : TAN_FULL);
   const size_t nd = (size_t)plan.N * nc;
   void *spec = nullptr, *a = nullptr, *b = nullptr, *c = nullptr, *tan = nullptr;
@@ -931,7 +932,12 @@ extern "C" int mugpu_fft_tune_pass(int dim, const int* res, int precision, int p
         op.in = a;
         op.rvec = b;
         op.pout = a;
-        op.xvec = c;
+        if (plan.packed) {
+          op.sym = true;
+          op.sym_flags = SYM_UPDATE;
+        } else {
+          op.xvec = c;
+        }
         op.scal = scal;
         op.tan_kind = tk;
         op.tangent = tan;
@@ -939,9 +945,14 @@ extern "C" int mugpu_fft_tune_pass(int dim, const int* res, int precision, int p
       }
       case FV_C2R: {
         OpSpec op;
-        op.out_mode = OUT_DOT;
+        op.out_mode = plan.packed ? OUT_RUPD : OUT_DOT;
         op.out = c;
         op.dotv = a;
+        if (plan.packed) {
+          op.sym = true;
+          op.rvec = c;
+          op.scal = scal;
+        }
         return fast_c2r(plan, precision, op, spec);
       }
       case FV_AXIS0: {
