@@ -50,6 +50,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+HBM_BYTES = 288 << 30
 
 
 def parse():
@@ -128,9 +129,9 @@ class Workload:
             self.prefix_note = ("load step 1, the first 3 Newton iterations (the increment "
                                 "falls 2.2e-3, 1.1e-3, 5.0e-4; from the 4th it grows, the 6th "
                                 "CG fails): no load step of the ramp converges at 256^3")
-            # 9*(6*8 + 9*8) + 360: the tangent is major-symmetric, stored as
-            # its 45-entry upper triangle
-            self.T = 360
+            # the FP64 operator keeps the consistent tangent as 26 factors, the
+            # FP32 one as the 45-entry upper triangle of the symmetric matrix
+            self.T = 208 if self.prec == "fp64" else 360
         elif w == "c2":
             self.n = args.size or 128
             self.res = [self.n] * 3
@@ -176,14 +177,14 @@ class Workload:
             self.equil_tol = 2.0
             self.T = 16
         self.N = int(np.prod(self.res))
-        # algorithmic bytes per voxel per CG iteration: nc (6 s_f + 9 s_v) + T,
-        # six sweeps of operator-precision fields (K:p input, two spectrum
-        # round trips, Ap) and nine of CG vectors, plus the tangent; the FP32
-        # form keeps operator fields, CG vectors and the tangent copy in FP32
-        nc = len(self.res) ** 2
         s = 8 if self.prec == "fp64" else 4
         self.T_prec = self.T * s // 8
-        self.B_alg = nc * (6 * s + 9 * s) + self.T_prec
+        # bytes per voxel per CG iteration: what its kernels read and write once
+        # (kernel_bytes); the x update of up to eight FP64 iterations is one launch
+        self.B_alg = round((kernel_bytes(self, 0, self.prec) + (2 if len(self.res) == 3 else 0) *
+                            kernel_bytes(self, 1, self.prec) + kernel_bytes(self, 2, self.prec) +
+                            kernel_bytes(self, 3, self.prec) +
+                            (kernel_bytes(self, 5, self.prec) or 0) / updates_every(self)) / self.N, 1)
         if not hasattr(self, "newton_maxiter"):
             self.newton_maxiter = 0
         self.converged = None
@@ -239,44 +240,94 @@ FAST = (16, 32, 48, 64, 96, 128, 256, 512)
 
 
 def kernel_name(wl, k):
-    """Symbol of the kernel behind a timing class for this grid: axis
-    lengths 16..512 run the compile-time-length passes."""
+    """Symbol of the kernel behind a timing class for this grid: axis lengths
+    16..512 run the compile-time-length passes, the other axes of FP64 cells
+    the run-time-length ones (fft_gen*.hip)."""
     last, first = wl.res[-1], wl.res[0]
     mid = wl.res[1] if len(wl.res) == 3 else None
-    return {0: "k_r2c_fast" if last in FAST else "k_last_r2c",
-            1: "k_strided_fast (middle axis)" if mid in FAST else "k_strided (middle axis)",
-            2: "k_axis0_fast" if first in FAST else "k_axis0_project",
-            3: "k_c2r_fast" if last in FAST else "k_last_c2r",
-            4: "material", 5: "k_cg_update"}[k]
+    gen = wl.prec == "fp64"
+    return {0: "k_r2c_fast" if last in FAST else "k_gen_r2c" if gen else "k_last_r2c",
+            1: "k_strided_fast (middle axis)" if mid in FAST
+               else "k_gen_strided (middle axis)" if gen else "k_strided (middle axis)",
+            2: "k_axis0_fast" if first in FAST else "k_gen_axis0" if gen else "k_axis0_project",
+            3: "k_c2r_fast" if last in FAST else "k_gen_c2r" if gen else "k_last_c2r",
+            4: "material", 5: "k_ring_flush" if gen else "k_cg_update"}[k]
 
 
-def kernel_bytes(wl, kclass, prec):
-    """Algorithmic HBM bytes of one launch: each input read once and each
-    output written once.  For the spectrum passes this is a read and a write
-    of the Hermitian half spectrum, Kpts x nc complex values."""
+def cg_shape(wl):
+    """(components of a spectrum line, components of p and r inside a chunk of
+    iterations, directions kept until x is updated, 0: none) of an FP64 solve:
+    small-strain workloads have isotropic tangents, so their spectra are packed;
+    on large grids (ring_ensure, csrc/api.hip) p and r are too, and x is updated
+    once per eight or four iterations."""
+    dim = len(wl.res)
+    nc = dim * dim
+    nl = dim * (dim + 1) // 2 if wl.form == "small" else nc
+    field = 8 * wl.N * nl
+    if field < (4 << 20 if nl == 6 else 32 << 20):
+        return nl, nc, 0
+    for m in (8, 4):
+        if field * (m + (1 if nl < nc else 0)) <= HBM_BYTES // 16:
+            return nl, nl, m
+    return nl, nc, 0
+
+
+def updates_every(wl):
+    """CG iterations per launch of the update kernel."""
+    return (cg_shape(wl)[2] or 1) if wl.prec == "fp64" else 1
+
+
+def kernel_read_write_bytes(wl, kclass, prec):
+    """(read, written) HBM bytes of one launch: each input read once and each
+    output written once.  For the spectrum passes this is the Hermitian half
+    spectrum, Kpts x components complex values."""
     dim = len(wl.res)
     nc = dim * dim
     s = 8 if prec == "fp64" else 4
-    herm = list(wl.res[:-1]) + [wl.res[-1] // 2 + 1]
-    kpts = int(np.prod(herm))
-    if kclass in (1, 2):
-        return 2 * kpts * nc * 2 * s
+    kpts = int(np.prod(list(wl.res[:-1]) + [wl.res[-1] // 2 + 1]))
+    field = wl.N * nc * s
+    if prec == "fp64":
+        nl, nf, ring = cg_shape(wl)
+        spec, vec = kpts * nl * 2 * s, wl.N * nf * s
+        if kclass in (1, 2):
+            return spec, spec
+        if kclass == 0:
+            # r, p and the tangent read, p and the spectrum written; without
+            # kept directions x += alpha p_old rides here
+            x = 0 if ring else field
+            return 2 * vec + x + wl.N * wl.T_prec, vec + x + spec
+        if kclass == 3:
+            # r += alpha A p
+            return spec + vec, vec
+        if kclass == 5 and ring:
+            # x += sum alpha_i p_i; packed directions also leave p in its full field
+            return ring * vec + field, field + (field if nf < nc else 0)
+        return None
+    spec = kpts * nc * 2 * s
     # with compile-time-length passes on the last axis the x update of a CG
     # iteration rides on the next iteration's r2c (x += alpha p_old where p
     # is read anyway), so the r2c moves x twice more and the update kernel
     # reads neither x nor p
     fused = wl.res[-1] in FAST
+    if kclass in (1, 2):
+        return spec, spec
     if kclass == 0:
         # r and p read, p written (p = -r + beta p), [x read and written],
         # tangent read, half spectrum written
-        return (5 if fused else 3) * wl.N * nc * s + wl.N * wl.T_prec + kpts * nc * 2 * s
+        return (3 if fused else 2) * field + wl.N * wl.T_prec, (2 if fused else 1) * field + spec
     if kclass == 3:
         # half spectrum read, Ap written, p read for the dot product
-        return kpts * nc * 2 * s + 2 * wl.N * nc * s
+        return spec + field, field
     if kclass == 5:
         # [x, p read, x written,] r and Ap read, r written
-        return (3 if fused else 6) * wl.N * nc * s
+        return (2 if fused else 4) * field, (1 if fused else 2) * field
     return None
+
+
+def kernel_bytes(wl, kclass, prec):
+    """HBM bytes of one launch (kernel_read_write_bytes)."""
+    rw = kernel_read_write_bytes(wl, kclass, prec)
+    return None if rw is None else rw[0] + rw[1]
 
 
 # ------------------------------------------------------------- CPU baseline
@@ -421,27 +472,6 @@ def line_bandwidth(capi, wl, reps=3):
         capi.check(lib.mugpu_line_bandwidth(prec, n, plane, nc, kp, reps, ctypes.byref(g)))
         out["kpts_per_tile_{}".format(kp)] = round(g.value, 1)
     return out
-
-
-def kernel_read_write_bytes(wl, kclass, prec):
-    """(read, written) algorithmic bytes of one launch (their sum is
-    kernel_bytes)."""
-    dim = len(wl.res)
-    nc = dim * dim
-    s = 8 if prec == "fp64" else 4
-    herm = list(wl.res[:-1]) + [wl.res[-1] // 2 + 1]
-    spec = int(np.prod(herm)) * nc * 2 * s
-    field = wl.N * nc * s
-    fused = wl.res[-1] in FAST
-    if kclass in (1, 2):
-        return spec, spec
-    if kclass == 0:
-        return (3 if fused else 2) * field + wl.N * wl.T_prec, (2 if fused else 1) * field + spec
-    if kclass == 3:
-        return spec + field, field
-    if kclass == 5:
-        return (2 if fused else 4) * field, (1 if fused else 2) * field
-    return None
 
 
 def achievable_time(rw, copy_gbs):
