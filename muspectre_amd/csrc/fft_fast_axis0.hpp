@@ -56,7 +56,7 @@ int axis0_hb(FftPlan& p, const ProjParams& pj, void* spec, int v) {
 }
 template <typename T, int DIM>
 int axis0_any(FftPlan& p, const ProjParams& pj, void* spec) {
-  const int v = p.fvar[pi_of<T>()][FV_AXIS0][p.packed ? 1 : 0];
+  const int v = p.fvar[pi_of<T>()][FV_AXIS0][p.packed ? 2 : 0];
 #define C_(n, e) axis0_hb<T, n, e, DIM>(p, pj, spec, v)
   MUGPU_FAST_SWITCH(p.res[0], v & 1, C_)
 #undef C_

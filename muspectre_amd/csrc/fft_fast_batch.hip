@@ -89,7 +89,7 @@ int b_axis0_h(FftPlan& p, const BatchSlot* slots, int ns, int h) {
 template <int DIM>
 int batch_operator_dim(FftPlan& p, const BatchSlot* slots, int ns) {
   int rc = MUGPU_EARG;
-  const unsigned char(&fv)[FV_COUNT][2] = p.fvar[1];
+  const unsigned char(&fv)[FV_COUNT][3] = p.fvar[1];
   timing_begin(MUGPU_K_LAST_R2C);
 #define C_(n, e) b_r2c_h<n, e, DIM>(p, slots, ns, (fv[FV_R2C][1] >> 1) & 1)
   rc = [&]() -> int { MUGPU_FAST_SWITCH(p.res[DIM - 1], fv[FV_R2C][1] & 1, C_) return MUGPU_EARG; }();

@@ -64,7 +64,7 @@ int c2r_h(FftPlan& p, const OpSpec& op, void* spec, int h) {
 }
 template <typename T, int DIM>
 int c2r_any(FftPlan& p, const OpSpec& op, void* spec) {
-  const int v = p.fvar[pi_of<T>()][FV_C2R][p.packed ? 1 : 0];
+  const int v = p.fvar[pi_of<T>()][FV_C2R][p.packed ? 2 : 0];
 #define C_(n, e) c2r_h<T, n, e, DIM>(p, op, spec, v >> 1)
   MUGPU_FAST_SWITCH(p.res[DIM - 1], v & 1, C_)
 #undef C_

@@ -77,7 +77,7 @@ int r2c_h(FftPlan& p, const OpSpec& op, void* spec, int h) {
 }
 template <typename T, int DIM>
 int r2c_any(FftPlan& p, const OpSpec& op, void* spec) {
-  const int v = p.fvar[pi_of<T>()][FV_R2C][p.packed || op.tan_kind == TAN_ISO ? 1 : 0];
+  const int v = p.fvar[pi_of<T>()][FV_R2C][p.packed ? 2 : op.tan_kind == TAN_ISO ? 1 : 0];
 #define C_(n, e) r2c_h<T, n, e, DIM>(p, op, spec, v >> 1)
   MUGPU_FAST_SWITCH(p.res[DIM - 1], v & 1, C_)
 #undef C_

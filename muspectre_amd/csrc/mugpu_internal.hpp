@@ -225,11 +225,11 @@ struct FftPlan {
   // variant of each compile-time-length pass (bit 0: 8 values per thread
   // instead of 16 or 12; bit 1: half the rows or k-points per workgroup, for
   // the last-axis and first-axis projection passes), per precision (0 FP64,
-  // 1 FP32), per pass and, for the r2c pass, per tangent (0 full matrices,
-  // 1 isotropic); for the FP64 c2r and projection passes 1 is the packed form,
-  // whose tiles are two thirds as wide (first axis at 256^3: the variant best for
+  // 1 FP32), per pass and per form: 0 one line per component, 1 the same with an
+  // isotropic tangent (r2c pass), 2 packed lines (FP64 last-axis and projection
+  // passes), whose tiles are two thirds as wide (first axis at 256^3: the variant best for
   // nine lines takes 687 us on six, the best one 415; at 128^3 52.6 and 43.7)
-  unsigned char fvar[2][5][2] = {};
+  unsigned char fvar[2][5][3] = {};
   ScalarFold fold;  // of the run in hand (operator_impl)
   bool fold_ok = false;  // no last-axis pass of this plan has more than kFoldMax workgroups
   // while set: every pass kernel returns at once when active[0] == 0 (CG
@@ -240,7 +240,7 @@ struct FftPlan {
 enum FastVariantPass { FV_R2C = 0, FV_STRIDED1 = 1, FV_AXIS0 = 2, FV_C2R = 3, FV_STRIDED0 = 4, FV_COUNT = 5 };
 // variant of a pass for an axis length, dimension, precision and tangent
 // class, from the tuned table (fft_tuned.inc)
-int fast_variant(int pass, int n, int dim, int prec, int iso);
+int fast_variant(int pass, int n, int dim, int prec, int form);
 // make fast_variant return `variant` for a pass and precision wherever that
 // variant exists (-1: the tuned table again); plans read it when created
 void force_variant(int pass, int prec, int variant);

@@ -14,7 +14,8 @@ namespace mugpu {
 // yz, xz, xy) instead of dim^2, 2/3 (3D) or 3/4 (2D) of the bytes and of the
 // transforms.  The projection of a field is that of its symmetric part, which
 // is taken when a field enters.  Measured per launch at 128^3 FP64: middle axis
-// 56 + 46 -> 38 + 32 us, first axis 62 -> 53, c2r 98 -> 76.
+// 56 + 46 -> 38 + 32 us, first axis 62 -> 44 (in the variant best for six lines),
+// c2r 98 -> 76.
 __host__ __device__ constexpr int sym_lines(int dim) { return dim * (dim + 1) / 2; }
 // lines per row or k-point: packed or one per component
 __host__ __device__ constexpr int nb_lines(int dim, bool packed) {
@@ -427,7 +428,9 @@ __device__ __forceinline__ double fold_sum(const double* __restrict__ part, int 
 // In a packed run p and r of a chunk of iterations hold the dim (dim + 1) / 2
 // components too (48 instead of 72 B per voxel in 3D, five sweeps per iteration);
 // the chunk's first iteration reads them from the full fields (the mean of two
-// mirrored components) and its last one writes r back to them.
+// mirrored components) and its last one writes r back to them.  Per launch at
+// 128^3, with x no longer in the r2c pass: r2c 168 -> 94 us, c2r 76 -> 69; at
+// 125^3 128 -> 96 and 102 -> 78.
 
 // p (packed) of `tot` values from `base` on, at most KB per thread in flight,
 // stored and staged in sp; with SYM_UPDATE p = -r + beta p.  Values at and beyond
