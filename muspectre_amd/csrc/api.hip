@@ -1362,7 +1362,11 @@ extern "C" int mugpu_material_add_pixels(mugpu_cell c, int mat, int64_t count,
   for (int64_t i = 0; i < count; ++i) {
     m.h_pix.push_back(pixels[i]);
     if (m.family == MUGPU_LE2) {
-      for (int k = 0; k < c->nc; ++k) m.h_params.push_back(params[i * c->nc + k]);
+      const double* e = params + i * c->nc;
+      for (int k = 0; k < c->nc; ++k) m.h_params.push_back(e[k]);
+      for (int a = 0; a < c->dim; ++a)
+        for (int b = 0; b < a; ++b)
+          if (!(e[a + c->dim * b] == e[b + c->dim * a])) m.major_sym = false;
     } else if (m.family == MUGPU_LE3 || m.family == MUGPU_LE4) {
       const double E = params[2 * i], nu = params[2 * i + 1];
       m.h_params.push_back(lame_lambda(E, nu));
@@ -1400,11 +1404,12 @@ extern "C" int mugpu_cell_initialise(mugpu_cell c) {
   // consistent HEP1 tangent; 3D) -> upper triangle; otherwise the full matrix
   // FP64 cells of LE1-4 alone, or in 3D of the consistent HEP1 alone, keep the
   // factors of the tangent (the FP32-refined solve reads an FP32 copy of the
-  // matrix)
+  // matrix).  LE2 with a nonsymmetric eigenstrain has a nonsymmetric S, which
+  // the six numbers of LEF do not hold
   bool all_hep = !c->mats.empty(), all_sym = c->dim == 3 && !c->mats.empty(), any_gen = false;
   bool all_le = !c->mats.empty() && c->prec == MUGPU_FP64, all_ct = all_le && c->dim == 3;
   for (auto& m : c->mats) {
-    all_le = all_le && m.family >= MUGPU_LE1 && m.family <= MUGPU_LE4;
+    all_le = all_le && m.family >= MUGPU_LE1 && m.family <= MUGPU_LE4 && m.major_sym;
     all_ct = all_ct && m.family == MUGPU_HEP1_CT;
     all_hep = all_hep && m.family == MUGPU_HEP1;
     all_sym = all_sym && m.family != MUGPU_HEP1 && (m.family != MUGPU_LEG || m.major_sym);

@@ -78,8 +78,8 @@ void timing_void(int64_t from);
 // SYM : the upper triangle r <= c of a major-symmetric K (finite-strain
 //       hyperelastic laws and the consistent elasto-plastic tangent),
 //       nc (nc + 1) / 2 entries, row by row
-// LEF : FP64 finite-strain cells of linear elastic laws (LE1-4): F, the PK2
-//       stress S (Voigt order) and (lambda, mu), from which dP = dF S +
+// LEF : FP64 finite-strain cells of linear elastic laws (LE1-4; eigenstrains
+//       symmetric, else S is not): F, the PK2 stress S (Voigt order) and (lambda, mu), from which dP = dF S +
 //       F (C : sym(F^T dF)) is formed; dim^2 + dim (dim + 1) / 2 + 2 numbers, 17
 //       in 3D where the matrix has 45
 // HCT : FP64 3D cells of HyperElastoPlastic1 with the consistent tangent alone:
@@ -445,7 +445,7 @@ struct MaterialDev {
   int ppn = 0;
   std::vector<double> h_C;       // MUGPU_LEG: C_ijkl at (i + d j) + d^2 (k + d l)
   double* d_C = nullptr;
-  bool major_sym = true;         // MUGPU_LEG: C_ijkl == C_klij
+  bool major_sym = true;         // MUGPU_LEG: C_ijkl == C_klij; MUGPU_LE2: symmetric eigenstrains
   int* d_pix = nullptr;
   double* d_params = nullptr;
   double* Fp[2] = {nullptr, nullptr};
