@@ -1400,19 +1400,20 @@ extern "C" int mugpu_cell_initialise(mugpu_cell c) {
   // small strain: isotropic Hooke per voxel -> (lambda, mu), unless a
   // generic material brings a general C; finite strain: the coded HEP1
   // tangent alone -> its dim^3 form; laws whose tangent is major-symmetric
-  // (LE1-4 and a major-symmetric generic C pushed forward from PK2, the
-  // consistent HEP1 tangent; 3D) -> upper triangle; otherwise the full matrix
+  // (LE1-4 with symmetric eigenstrains and a major-symmetric generic C pushed
+  // forward from PK2, the consistent HEP1 tangent; 3D) -> upper triangle;
+  // otherwise the full matrix
   // FP64 cells of LE1-4 alone, or in 3D of the consistent HEP1 alone, keep the
   // factors of the tangent (the FP32-refined solve reads an FP32 copy of the
   // matrix).  LE2 with a nonsymmetric eigenstrain has a nonsymmetric S, which
-  // the six numbers of LEF do not hold
+  // neither the six numbers of LEF nor a triangle of the matrix holds
   bool all_hep = !c->mats.empty(), all_sym = c->dim == 3 && !c->mats.empty(), any_gen = false;
   bool all_le = !c->mats.empty() && c->prec == MUGPU_FP64, all_ct = all_le && c->dim == 3;
   for (auto& m : c->mats) {
     all_le = all_le && m.family >= MUGPU_LE1 && m.family <= MUGPU_LE4 && m.major_sym;
     all_ct = all_ct && m.family == MUGPU_HEP1_CT;
     all_hep = all_hep && m.family == MUGPU_HEP1;
-    all_sym = all_sym && m.family != MUGPU_HEP1 && (m.family != MUGPU_LEG || m.major_sym);
+    all_sym = all_sym && m.family != MUGPU_HEP1 && m.major_sym;
     any_gen = any_gen || m.family == MUGPU_LEG;
   }
   c->tan_kind = c->form == MUGPU_SMALL_STRAIN && !any_gen ? TAN_ISO

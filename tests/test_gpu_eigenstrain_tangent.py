@@ -41,3 +41,11 @@ def _cells(capi, oracle, res, prec=0):
 def test_nonsymmetric_eigenstrain_2d(capi, oracle, res):
     oc, gc, F = _cells(capi, oracle, res)
     _check(capi, oc, gc, F, 1)
+
+
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("res", [[5, 3, 7], [3, 5, 16]], ids=lambda r: "x".join(map(str, r)))
+def test_nonsymmetric_eigenstrain_3d(capi, oracle, res, prec):
+    """(an FP32 cell's material stage, tangent and FP64 operator)"""
+    oc, gc, F = _cells(capi, oracle, res, prec)
+    _check(capi, oc, gc, F, 1)
