@@ -463,6 +463,14 @@ int mugpu_fft_tune_pass(int dim, const int *resolutions, int precision, int pass
  * `pass` (MUGPU_PASS_*) in `precision` on every axis length where that
  * variant exists, in place of the tuned one; variant < 0 restores the table. */
 int mugpu_debug_force_variant(int pass, int precision, int variant);
+/* Test hook for the bounds of the r2c pass over packed small-strain CG vectors
+ * (no reference counterpart; needs no device): the lowest and the highest
+ * element of p and r (fields of dim^2 components on the grid `resolutions`)
+ * that the pass's last workgroup, the only one with rows missing, reads in a
+ * chunk's first iteration, from the index functions of the kernel, and the rows
+ * of a workgroup. */
+int mugpu_debug_stage_reads(int dim, const int *resolutions, int64_t *lowest,
+                            int64_t *highest, int *rows_per_workgroup);
 /* streaming device copy of `bytes` (multiple of 16), the bandwidth
  * reference for the roofline and for the HBM counter calibration */
 int mugpu_copy(void *d_dst, const void *d_src, size_t bytes);

@@ -108,6 +108,7 @@ SIGNATURES = [
     ("mugpu_line_bandwidth", _int, [_int, _int, ctypes.c_int64, _int, _int, _int, _dp]),
     ("mugpu_debug_fail_allocations", _int, [_int]),
     ("mugpu_debug_force_variant", _int, [_int, _int, _int]),
+    ("mugpu_debug_stage_reads", _int, [_int, _ip, _i64p, _i64p, _ip]),
 ]
 NOALLOC_MAX_VALUES = 2796000  # MUGPU_NOALLOC_MAX_VALUES
 K_LAST_R2C, K_MIDDLE, K_AXIS0, K_LAST_C2R, K_MATERIAL, K_CG_UPDATE = range(6)

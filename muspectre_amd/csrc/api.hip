@@ -590,6 +590,46 @@ extern "C" int mugpu_debug_force_variant(int pass, int precision, int variant) {
   return MUGPU_OK;
 }
 
+extern "C" int mugpu_debug_stage_reads(int dim, const int* res, int64_t* lowest, int64_t* highest,
+                                       int* rows_per_workgroup) {
+  if ((dim != 2 && dim != 3) || !res || !lowest || !highest || !rows_per_workgroup) return MUGPU_EARG;
+  const int n = res[dim - 1], nl = sym_lines(dim);
+  int64_t rows = 1;
+  for (int d = 0; d < dim; ++d)
+    if (res[d] < 1) return MUGPU_EARG;
+  for (int d = 0; d + 1 < dim; ++d) rows *= res[d];
+  int rb, stage;  // rows of a workgroup, and of them staged at once
+  if (fast_size(n)) {
+    rb = stage = fast_rows_per_block(n, dim, fast_variant(FV_R2C, n, dim, MUGPU_FP64, 2));
+  } else {
+    GenAxis ax;
+    const GenShape g = gen_radices(n, ax) ? gen_last_shape(ax, dim * dim, nl, rows) : GenShape{};
+    if (!g.NT) {
+      set_error("no pass of run-time length for a last axis of %d", n);
+      return MUGPU_EARG;
+    }
+    rb = 2 * g.mult;
+    stage = 2;
+  }
+  *rows_per_workgroup = rb;
+  *lowest = INT64_MAX;
+  *highest = INT64_MIN;
+  // (only the last workgroup can have rows missing)
+  const int64_t row0 = (rows - 1) / rb * rb, lim = rows * n * nl;
+  for (int r0 = 0; r0 < rb; r0 += stage) {
+    const int64_t base = (row0 + r0) * n * nl;
+    const int left = sym_left(base, lim, stage * n * nl);
+    for (int e = 0; e < left; ++e) {
+      int64_t a, b;
+      if (dim == 3) sym_entries<3>(base, e, a, b);
+      else sym_entries<2>(base, e, a, b);
+      *lowest = std::min(*lowest, std::min(a, b));
+      *highest = std::max(*highest, std::max(a, b));
+    }
+  }
+  return MUGPU_OK;
+}
+
 extern "C" int mugpu_debug_fail_allocations(int after) {
   g_fail_alloc_after.store(after < 0 ? -1 : after);
   return MUGPU_OK;

@@ -32,7 +32,7 @@ __host__ __device__ constexpr int line_of(int c) {
 }
 // components i + DIM j and j + DIM i of line c
 template <int DIM>
-__device__ __forceinline__ void sym_pair(int c, int& a, int& b) {
+__host__ __device__ __forceinline__ void sym_pair(int c, int& a, int& b) {
   a = DIM == 3 ? (0x367840 >> (4 * c)) & 15 : (0x230 >> (4 * c)) & 15;
   b = DIM == 3 ? (0x125840 >> (4 * c)) & 15 : (0x130 >> (4 * c)) & 15;
 }
@@ -432,16 +432,36 @@ __device__ __forceinline__ double fold_sum(const double* __restrict__ part, int 
 // 128^3, with x no longer in the r2c pass: r2c 168 -> 94 us, c2r 76 -> 69; at
 // 125^3 128 -> 96 and 102 -> 78.
 
+// of `tot` packed values from `base` on, those that lie before `lim`; <= 0 where
+// the rows are all beyond the last one (the later row pairs of a last workgroup)
+__host__ __device__ __forceinline__ int sym_left(int64_t base, int64_t lim, int tot) {
+  return lim - base < tot ? (int)(lim - base) : tot;
+}
+// the two entries of a field of dim^2 components that hold packed value base + e
+// (base: a multiple of dim (dim + 1) / 2)
+template <int DIM>
+__host__ __device__ __forceinline__ void sym_entries(int64_t base, int e, int64_t& a, int64_t& b) {
+  constexpr int NC = DIM * DIM, NL = sym_lines(DIM);
+  const int m = e / NL;
+  int ca, cb;
+  sym_pair<DIM>(e - m * NL, ca, cb);
+  const int64_t g = (base / NL + m) * NC;
+  a = g + ca;
+  b = g + cb;
+}
+
 // p (packed) of `tot` values from `base` on, at most KB per thread in flight,
 // stored and staged in sp; with SYM_UPDATE p = -r + beta p.  Values at and beyond
-// `lim` are staged as zeros.
+// `lim` are staged as zeros; nothing is read there.
 template <typename T, int DIM, int KB>
 __device__ __forceinline__ void sym_stage(const T* in, const T* rvec, T* pout, int flags, T beta,
                                           int64_t base, int64_t lim, int tot, int NT, T* sp) {
-  constexpr int NC = DIM * DIM, NL = sym_lines(DIM);
   const bool upd = flags & SYM_UPDATE, full = flags & SYM_SRC_FULL;
-  const int last = lim - base < tot ? (int)(lim - base) - 1 : tot - 1;  // (>= 0: row 0 exists)
-  const int64_t vox0 = base / NL;
+  const int last = sym_left(base, lim, tot) - 1;
+  if (last < 0) {
+    for (int e = threadIdx.x; e < tot; e += NT) sp[e] = T(0);
+    return;
+  }
   for (int e0 = 0; e0 < tot; e0 += KB * NT) {
     T pv[KB], rv[KB];
     if (full) {
@@ -450,14 +470,12 @@ __device__ __forceinline__ void sym_stage(const T* in, const T* rvec, T* pout, i
       for (int i = 0; i < KB; ++i) {
         int e = e0 + i * NT + (int)threadIdx.x;
         if (e > last) e = last;
-        const int m = e / NL;
-        int ca, cb;
-        sym_pair<DIM>(e - m * NL, ca, cb);
-        const int64_t g = (vox0 + m) * NC;
-        pv[i] = in[g + ca];
-        pw[i] = in[g + cb];
-        rv[i] = rvec[g + ca];
-        rw[i] = rvec[g + cb];
+        int64_t a, b;
+        sym_entries<DIM>(base, e, a, b);
+        pv[i] = in[a];
+        pw[i] = in[b];
+        rv[i] = rvec[a];
+        rw[i] = rvec[b];
       }
 #pragma unroll
       for (int i = 0; i < KB; ++i) {
