@@ -459,11 +459,7 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
     constexpr int NF = S ? NL : NC;  // components of the staged field
     T beta = PU ? (T)a.scal[SC_BETA] : T(0);
     if constexpr (sizeof(T) == 8 && PU) {
-      if (a.fold.rr) {
-        const double rr = fold_sum(a.fold.rr, a.fold.nrr, reinterpret_cast<double*>(smem));
-        if (!fold_beta_test(a.fold, rr, beta)) return;
-        __syncthreads();
-      }
+      if (a.fold.rr && !fold_goes_on(a.fold, a.active, reinterpret_cast<double*>(smem), beta)) return;
     }
     const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
     constexpr int TOT = RB * N * NF, kBatch = 8;
@@ -567,11 +563,7 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
     constexpr bool XU = IN == IN_TAN_PUPDATE_X;
     T beta = PU ? (T)a.scal[SC_BETA] : T(0);
     if constexpr (sizeof(T) == 8 && PU) {
-      if (a.fold.rr) {
-        const double rr = fold_sum(a.fold.rr, a.fold.nrr, reinterpret_cast<double*>(smem));
-        if (!fold_beta_test(a.fold, rr, beta)) return;
-        __syncthreads();
-      }
+      if (a.fold.rr && !fold_goes_on(a.fold, a.active, reinterpret_cast<double*>(smem), beta)) return;
     }
     const T al = XU ? (T)a.scal[SC_ALPHA] : T(0);
     {
@@ -690,7 +682,9 @@ __device__ __forceinline__ void r2c_body(const LArgs<T>& a, unsigned char* smem,
 template <typename T, int N, int E, int DIM, int IN, bool ISO, int H, bool PK>
 __global__ __launch_bounds__(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E))
 MUGPU_WPE(z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), (lds_r2c<T, N, DIM, IN, H, PK>())) void k_r2c_fast(LArgs<T> a) {
-  if (a.active && !a.active[0]) return;
+  // (with folded scalars this launch writes the flag: fold_goes_on reads it)
+  constexpr bool PU = IN == IN_TAN_PUPDATE || IN == IN_TAN_PUPDATE_X || IN == IN_TAN_S;
+  if (!(sizeof(T) == 8 && PU && a.fold.rr) && a.active && !a.active[0]) return;
   extern __shared__ __align__(16) unsigned char smem[];
   LArgs<T> b = a;
   b.tw = twiddles_for<T, N, z_rows(N, DIM, H) / 2 * nb_lines(DIM, PK) * (N / E), lds_r2c<T, N, DIM, IN, H, PK>()>(a.tw, smem);

@@ -584,6 +584,20 @@ __device__ __forceinline__ bool fold_beta_test(const ScalarFold& f, double s, do
   }
   return go;
 }
+// The whole of it: whether the iteration runs, with its beta.  Workgroup 0 of this
+// very launch clears the flag, so the wavefronts of another workgroup may read
+// different values of it: none returns before all have summed the partials,
+// and where the flag was cleared by this launch the test fails for everyone.
+// Every thread must call it (barriers inside); red holds one double and is free
+// again on return
+__device__ __forceinline__ bool fold_goes_on(const ScalarFold& f, const int* active, double* red,
+                                             double& beta) {
+  const int on = active ? active[0] : 1;
+  const double s = fold_sum(f.rr, f.nrr, red);
+  if (!on || !fold_beta_test(f, s, beta)) return false;
+  __syncthreads();
+  return true;
+}
 // c2r: alpha from the sum s of the p . K p partials
 __device__ __forceinline__ double fold_alpha(const ScalarFold& f, double s) {
   const double al = f.scal[f.iter & 1 ? SC_RDR1 : SC_RDR] / s;
