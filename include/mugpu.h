@@ -309,6 +309,10 @@ int mugpu_cg_steps(mugpu_cell cell, int update_p, void *d_x, void *d_r,
                    void *d_p, void *d_Ap, double tol2, int max_steps,
                    int *steps, double *new_rdr);
 int mugpu_cg_finish(mugpu_cell cell);
+/* The directions that the cell keeps at present (eight, four or none) and the
+ * components per voxel in which p and r are held inside a chunk (no reference
+ * counterpart): what one iteration moves depends on them. */
+int mugpu_cell_kept_directions(mugpu_cell cell, int *directions, int *components);
 /* mugpu_cg_steps on cells of at most 2^20 values (nb_pixels x nb_components)
  * replays each chunk from a captured hipGraph (kept on the cell per set of
  * vectors, chunk length and form of the first iteration; the arithmetic is
@@ -463,6 +467,10 @@ int mugpu_fft_tune_pass(int dim, const int *resolutions, int precision, int pass
  * `pass` (MUGPU_PASS_*) in `precision` on every axis length where that
  * variant exists, in place of the tuned one; variant < 0 restores the table. */
 int mugpu_debug_force_variant(int pass, int precision, int variant);
+/* Test hook for the kept directions of mugpu_cg_steps (no reference
+ * counterpart): gives back those of idle cells; from then on cells keep at most
+ * `most` (8 again: the default; 4; below 4: none). */
+int mugpu_debug_kept_directions(int most);
 /* Test hook for the bounds of the r2c pass over packed small-strain CG vectors
  * (no reference counterpart; needs no device): the lowest and the highest
  * element of p and r (fields of dim^2 components on the grid `resolutions`)

@@ -87,6 +87,7 @@ SIGNATURES = [
     ("mugpu_cg_step", _int, [_vp, _int, _vp, _vp, _vp, _vp, _dp]),
     ("mugpu_cg_steps", _int, [_vp, _int, _vp, _vp, _vp, _vp, _dbl, _int, _ip, _dp]),
     ("mugpu_cg_finish", _int, [_vp]),
+    ("mugpu_cell_kept_directions", _int, [_vp, _ip, _ip]),
     ("mugpu_cg_graphs", _int, [_int]),
     ("mugpu_cg_solve_mixed", _int, [_vp, _vp, _vp, _dbl, _int, _dbl, _i64p, _ip, _dp]),
     ("mugpu_cg_solve_mixed_noalloc", _int, [_vp, _vp, _vp, _dbl, _int, _dbl, _i64p, _ip, _dp]),
@@ -108,6 +109,7 @@ SIGNATURES = [
     ("mugpu_line_bandwidth", _int, [_int, _int, ctypes.c_int64, _int, _int, _int, _dp]),
     ("mugpu_debug_fail_allocations", _int, [_int]),
     ("mugpu_debug_force_variant", _int, [_int, _int, _int]),
+    ("mugpu_debug_kept_directions", _int, [_int]),
     ("mugpu_debug_stage_reads", _int, [_int, _ip, _i64p, _i64p, _ip]),
 ]
 NOALLOC_MAX_VALUES = 2796000  # MUGPU_NOALLOC_MAX_VALUES

@@ -209,6 +209,7 @@ int flush_x(mugpu_cell c);
 namespace {
 std::mutex g_ring_mu;
 std::vector<mugpu_cell> g_ring_cells;
+int g_ring_max = kRing;  // mugpu_debug_kept_directions
 
 void ring_free_locked(mugpu_cell c) {
   (void)hipFree(c->ring);
@@ -293,6 +294,7 @@ void ring_ensure(mugpu_cell c) {
   }
   const size_t field = sizeof(double) * (size_t)c->N * nf;
   for (int len = kRing; len >= kRing / 2; len /= 2) {
+    if (len > g_ring_max) continue;
     const size_t bytes = field * (len + (nf < c->nc ? 1 : 0));
     if (bytes > tot / 16 || bytes > fr / 2) continue;
     void* q = nullptr;
@@ -587,6 +589,20 @@ extern "C" int mugpu_debug_force_variant(int pass, int precision, int variant) {
     return MUGPU_EARG;
   }
   force_variant(pass, precision, variant < 0 ? -1 : variant);
+  return MUGPU_OK;
+}
+
+extern "C" int mugpu_debug_kept_directions(int most) {
+  (void)rings_release();
+  g_ring_max = most;
+  return MUGPU_OK;
+}
+
+extern "C" int mugpu_cell_kept_directions(mugpu_cell c, int* directions, int* components) {
+  if (!c || !directions || !components) return MUGPU_EARG;
+  std::lock_guard<std::mutex> lk(g_ring_mu);
+  *directions = c->ring ? c->ring_len : 0;
+  *components = c->ring ? c->ring_nf : c->nc;
   return MUGPU_OK;
 }
 
