@@ -285,10 +285,12 @@ int mugpu_scale_copy(double a, const void *d_x, void *d_y, int64_t n);
  *   of this call (A p is not stored where the last pass updates r).  In a
  *   solve whose b = G b on a large grid (from 4 MB of packed components in
  *   3D small strain, else from 32 MB per vector) the cell keeps up to eight
- *   directions p, in at most 1/16 of the device's memory, and adds them to
- *   x together: x, r and p are complete when the call returns.  That
- *   memory is given back with the cell, by mugpu_release_cached and when an
- *   allocation of this library finds the device full.  Otherwise, where the last
+ *   directions p, in at most 1/16 of the device's memory (1/8 for all cells
+ *   together; beyond that the ones idle longest give theirs back), and adds
+ *   them to x together: x, r and p are complete when the call returns.  That
+ *   memory is also given back with the cell, by mugpu_release_cached and when
+ *   an allocation of this library finds the device full; a program that takes
+ *   device memory from another allocator too calls mugpu_release_cached.  Otherwise, where the last
  *   axis has compiled passes (lengths 16, 32, 48, 64, 96, 128, 256, 512),
  *   the x update of an iteration is applied by the next iteration's first
  *   pass (which reads p anyway), so the x update of the last iteration of a call is left
@@ -471,6 +473,9 @@ int mugpu_debug_force_variant(int pass, int precision, int variant);
  * counterpart): gives back those of idle cells; from then on cells keep at most
  * `most` (8 again: the default; 4; below 4: none). */
 int mugpu_debug_kept_directions(int most);
+/* The same for the bytes that all cells together keep (0: the default, 1/8 of
+ * the device's memory). */
+int mugpu_debug_kept_bytes(size_t total);
 /* Test hook for the bounds of the r2c pass over packed small-strain CG vectors
  * (no reference counterpart; needs no device): the lowest and the highest
  * element of p and r (fields of dim^2 components on the grid `resolutions`)

@@ -110,6 +110,7 @@ SIGNATURES = [
     ("mugpu_debug_fail_allocations", _int, [_int]),
     ("mugpu_debug_force_variant", _int, [_int, _int, _int]),
     ("mugpu_debug_kept_directions", _int, [_int]),
+    ("mugpu_debug_kept_bytes", _int, [ctypes.c_size_t]),
     ("mugpu_debug_stage_reads", _int, [_int, _ip, _i64p, _i64p, _ip]),
 ]
 NOALLOC_MAX_VALUES = 2796000  # MUGPU_NOALLOC_MAX_VALUES

@@ -1,6 +1,7 @@
 // C-ABI of libmugpu.so (declared in include/mugpu.h).  Handles wrap device
 // buffers; every function reports errors through return codes and
 // mugpu_last_error().  Work runs on one library stream.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -161,6 +162,7 @@ struct mugpu_cell_s {
   // of ring_nf components and, if those are packed, one for r; nothing in it outlives
   // a call, so it is given back when device memory runs out (rings_release)
   double* ring = nullptr;
+  size_t ring_bytes = 0;
   int ring_len = 0, ring_nf = 0;
   bool ring_busy = false;
   // captured chunks of mugpu_cg_steps (small cells), by vectors, chunk
@@ -209,13 +211,33 @@ int flush_x(mugpu_cell c);
 namespace {
 std::mutex g_ring_mu;
 std::vector<mugpu_cell> g_ring_cells;
-int g_ring_max = kRing;  // mugpu_debug_kept_directions
+int g_ring_max = kRing;     // mugpu_debug_kept_directions
+size_t g_ring_total = 0;    // mugpu_debug_kept_bytes, 0: 1/8 of the device
 
 void ring_free_locked(mugpu_cell c) {
   (void)hipFree(c->ring);
   c->ring = nullptr;
   for (auto& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
   c->graphs.clear();
+}
+
+// whether a ring of so many bytes keeps all of them within `most`, after the ones
+// not in use have been given back as far as needed, the first ones first
+bool ring_room(size_t bytes, size_t most) {
+  if (bytes > most) return false;
+  size_t sum = bytes;
+  for (mugpu_cell o : g_ring_cells) sum += o->ring_bytes;
+  for (size_t i = 0; sum > most && i < g_ring_cells.size();) {
+    mugpu_cell o = g_ring_cells[i];
+    if (o->ring_busy) {
+      ++i;
+      continue;
+    }
+    sum -= o->ring_bytes;
+    ring_free_locked(o);
+    g_ring_cells.erase(g_ring_cells.begin() + (std::ptrdiff_t)i);
+  }
+  return sum <= most;
 }
 
 // gives back the rings not in use; true if there was one
@@ -269,7 +291,7 @@ struct RingHold {
 };
 
 // A ring for the cell's next chunks: kRing directions, or half as many, within
-// 1/16 of the device's memory.  Without one (too small a field, none fits, or the
+// 1/16 of the device's memory and half of what is free.  Without one (too small a field, none fits, or the
 // device is full) x is updated by the passes, as in solves without an early alpha.
 // It takes a sweep's worth of bytes out of an iteration (and with packed vectors
 // two thirds of one more), which counts where HBM sets the pace: CG on full fields
@@ -279,12 +301,20 @@ struct RingHold {
 // third, 512^2 (6 MB) 1.46 -> 1.48 ms.  The last level of cache takes most of the
 // difference below the limits.
 constexpr size_t kRingField = (size_t)32 << 20, kRingFieldSym3 = (size_t)4 << 20;
+// All cells together keep at most 1/8 of the device: beyond that the ones whose
+// latest solve began first give theirs back, so programs with many large cells
+// (or another allocator on the device) do not lose more to idle ones.  Taking
+// one anew costs a map and an unmap per solve.
 void ring_ensure(mugpu_cell c) {
   const int nf = ring_components(c);
   if (sizeof(double) * (size_t)c->N * nf < (nf == 6 ? kRingFieldSym3 : kRingField)) return ring_drop(c);
   {
     std::lock_guard<std::mutex> lk(g_ring_mu);
-    if (c->ring && c->ring_nf == nf) return;
+    if (c->ring && c->ring_nf == nf) {
+      const auto it = std::find(g_ring_cells.begin(), g_ring_cells.end(), c);
+      std::rotate(it, it + 1, g_ring_cells.end());
+      return;
+    }
   }
   ring_drop(c);
   size_t fr = 0, tot = 0;
@@ -296,14 +326,20 @@ void ring_ensure(mugpu_cell c) {
   for (int len = kRing; len >= kRing / 2; len /= 2) {
     if (len > g_ring_max) continue;
     const size_t bytes = field * (len + (nf < c->nc ? 1 : 0));
-    if (bytes > tot / 16 || bytes > fr / 2) continue;
+    if (bytes > tot / 16) continue;
+    std::lock_guard<std::mutex> lk(g_ring_mu);
+    if (!ring_room(bytes, g_ring_total ? g_ring_total : tot / 8)) continue;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > fr / 2) {
+      (void)hipGetLastError();
+      continue;
+    }
     void* q = nullptr;
     if (hipMalloc(&q, bytes) != hipSuccess) {
       (void)hipGetLastError();
       continue;
     }
-    std::lock_guard<std::mutex> lk(g_ring_mu);
     c->ring = (double*)q;
+    c->ring_bytes = bytes;
     c->ring_len = len;
     c->ring_nf = nf;
     g_ring_cells.push_back(c);
@@ -595,6 +631,12 @@ extern "C" int mugpu_debug_force_variant(int pass, int precision, int variant) {
 extern "C" int mugpu_debug_kept_directions(int most) {
   (void)rings_release();
   g_ring_max = most;
+  return MUGPU_OK;
+}
+
+extern "C" int mugpu_debug_kept_bytes(size_t total) {
+  (void)rings_release();
+  g_ring_total = total;
   return MUGPU_OK;
 }
 
