@@ -61,6 +61,7 @@ void DeviceVector::set_zero() { check(mugpu_memset_zero(ptr_, sizeof(Real) * n_)
 void ResultField::capture(const void* d_src, int64_t n) {
   dev_ = std::make_shared<DeviceVector>(n);
   check(mugpu_scale_copy(1.0, d_src, dev_->data(), n));
+  read_ = false;
   host_.clear();
   host_valid_ = false;
 }
@@ -73,8 +74,13 @@ const std::vector<Real>& ResultField::host() const {
   return host_;
 }
 void ResultField::copy_to(Real* dst) const {
-  if (host_valid_) std::copy(host_.begin(), host_.end(), dst);
-  else if (dev_) dev_->download(dst);
+  if (!host_valid_ && dev_ && !read_ && dev_->size() >= kDirect) {
+    read_ = true;
+    dev_->download(dst);
+    return;
+  }
+  const std::vector<Real>& h = host();
+  std::copy(h.begin(), h.end(), dst);
 }
 void ResultField::assign(const Real* h, int64_t n) {
   dev_.reset();

@@ -92,7 +92,10 @@ class DeviceVector {
 };
 
 // A field of a result record: a device copy taken when the record is made
-// (one HBM-speed copy), downloaded to the host on first access and kept.
+// (one HBM-speed copy), downloaded to the host on first access and kept.  A
+// large field's first read goes straight into the caller's array (18 MB: 5.9 ms
+// by way of the kept copy, 0.7 ms) and the copy is made by the second one;
+// further reads cost a copy in host memory (83 KB: 0.9 us, a download 43 us).
 class ResultField {
  public:
   ResultField() = default;
@@ -102,12 +105,14 @@ class ResultField {
   const std::vector<Real>& host() const;
   // the values into dst (size() of them)
   void copy_to(Real* dst) const;
+  static constexpr int64_t kDirect = (int64_t)(2 << 20) / sizeof(Real);
   void assign(const Real* h, int64_t n);
 
  private:
   std::shared_ptr<DeviceVector> dev_;
   mutable std::vector<Real> host_;
   mutable bool host_valid_{false};
+  mutable bool read_{false};
 };
 
 // src/solver/solver_common.hh:50-67
