@@ -50,7 +50,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-HBM_BYTES = 288 << 30
 
 
 def parse():
@@ -179,15 +178,19 @@ class Workload:
         self.N = int(np.prod(self.res))
         s = 8 if self.prec == "fp64" else 4
         self.T_prec = self.T * s // 8
-        # bytes per voxel per CG iteration: what its kernels read and write once
-        # (kernel_bytes); the x update of up to eight FP64 iterations is one launch
-        self.B_alg = round((kernel_bytes(self, 0, self.prec) + (2 if len(self.res) == 3 else 0) *
-                            kernel_bytes(self, 1, self.prec) + kernel_bytes(self, 2, self.prec) +
-                            kernel_bytes(self, 3, self.prec) +
-                            (kernel_bytes(self, 5, self.prec) or 0) / updates_every(self)) / self.N, 1)
         if not hasattr(self, "newton_maxiter"):
             self.newton_maxiter = 0
         self.converged = None
+        self.kept = None  # (directions kept, components of p and r) of the solves
+
+    @property
+    def B_alg(self):
+        """Bytes per voxel per CG iteration: what its kernels read and write once
+        (kernel_bytes); the x update of up to eight FP64 iterations is one launch."""
+        mid = 2 if len(self.res) == 3 else 0
+        return round((kernel_bytes(self, 0, self.prec) + mid * kernel_bytes(self, 1, self.prec) +
+                      kernel_bytes(self, 2, self.prec) + kernel_bytes(self, 3, self.prec) +
+                      (kernel_bytes(self, 5, self.prec) or 0) / updates_every(self)) / self.N, 1)
 
     def make_cell(self, mu):
         dim = len(self.res)
@@ -231,6 +234,10 @@ class Workload:
             self.last = res
             its += sum(r.nb_it for r in res)
             cg += res[-1].nb_fev
+        if self.kept not in (None, cell.kept_directions):
+            print("bench: kept directions {} -> {}: another schedule than in the last step".format(
+                self.kept, cell.kept_directions), file=sys.stderr, flush=True)
+        self.kept = cell.kept_directions
         return its, cg
 
 
@@ -258,18 +265,11 @@ def cg_shape(wl):
     """(components of a spectrum line, components of p and r inside a chunk of
     iterations, directions kept until x is updated, 0: none) of an FP64 solve:
     small-strain workloads have isotropic tangents, so their spectra are packed;
-    on large grids (ring_ensure, csrc/api.hip) p and r are too, and x is updated
-    once per eight or four iterations."""
+    the rest is what the cell of the latest solve kept."""
     dim = len(wl.res)
-    nc = dim * dim
-    nl = dim * (dim + 1) // 2 if wl.form == "small" else nc
-    field = 8 * wl.N * nl
-    if field < (4 << 20 if nl == 6 else 32 << 20):
-        return nl, nc, 0
-    for m in (8, 4):
-        if field * (m + (1 if nl < nc else 0)) <= HBM_BYTES // 16:
-            return nl, nl, m
-    return nl, nc, 0
+    nl = dim * (dim + 1) // 2 if wl.form == "small" else dim * dim
+    ring, nf = wl.kept
+    return nl, nf, ring
 
 
 def updates_every(wl):

@@ -455,6 +455,14 @@ void bind_cell(py::module& m) {
       .def("get_stress", [nc](Sys& s) { return field_to(s.get_stress(), nc, s.size()); })
       .def("get_tangent", [nc](Sys& s) { return field_to(s.get_tangent(), nc * nc, s.size()); })
       .def_property_readonly("size", [](Sys& s) { return s.size(); })
+      .def_property_readonly(
+          "kept_directions",
+          [](Sys& s) {
+            int directions = 0, components = 0;
+            check(mugpu_cell_kept_directions(s.handle(), &directions, &components));
+            return std::make_pair(directions, components);
+          },
+          "CG directions the cell keeps for its next solve, and components per pixel of p and r in a chunk")
       .def(
           "evaluate_stress_tangent",
           [nc](Sys& s, farr v) {
