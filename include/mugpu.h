@@ -290,7 +290,11 @@ int mugpu_scale_copy(double a, const void *d_x, void *d_y, int64_t n);
  *   them to x together: x, r and p are complete when the call returns.  That
  *   memory is also given back with the cell, by mugpu_release_cached and when
  *   an allocation of this library finds the device full; a program that takes
- *   device memory from another allocator too calls mugpu_release_cached.  Otherwise, where the last
+ *   device memory from another allocator too calls mugpu_release_cached.
+ *   Whether a cell keeps directions, and how many, thus depends on free
+ *   memory.  In full fields the results are the same bits either way; small
+ *   strain sums r.r over the packed components with kept directions and over
+ *   all of them without, so the last bits may differ.  Otherwise, where the last
  *   axis has compiled passes (lengths 16, 32, 48, 64, 96, 128, 256, 512),
  *   the x update of an iteration is applied by the next iteration's first
  *   pass (which reads p anyway), so the x update of the last iteration of a call is left

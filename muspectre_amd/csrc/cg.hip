@@ -1,8 +1,10 @@
 // Vector kernels of SolverCG (src/solver/solver_cg.cc:62-96) and of the
 // Newton drivers (src/solver/solvers.cc:142-187).  Reductions are
 // deterministic: a fixed grid writes per-workgroup partial sums, and one
-// workgroup adds them in a fixed order, so a result does not depend on
-// what else runs on the device.
+// workgroup adds them in a fixed order.  The schedule that a solve takes can
+// depend on free device memory (kept directions, ring_ensure in api.hip): x, r
+// and p are the same bits either way in full fields, while packed small-strain
+// vectors sum r . r in another order than full ones.
 #include "mugpu_internal.hpp"
 #include "op_stages.hpp"
 

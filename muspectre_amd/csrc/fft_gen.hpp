@@ -13,8 +13,9 @@
 // and is a kernel of its own), and a pass for any other prime.  A thread holds
 // the inputs of up to gen_held(R) butterflies in registers between the reads
 // and the writes of a pass, so one LDS buffer serves.  No integer division by
-// a run-time value is left inside a pass: j / NS is a multiplication by a
-// reciprocal made with the plan.
+// a run-time value is left inside a pass of a compiled radix: j / NS is a
+// multiplication by a reciprocal made with the plan.  The pass for other primes
+// divides once per task, which forms (R - 1) / 2 products for each output pair.
 //
 // Bound by HBM from about 64^3 on, by latency below.  Measured per launch on a
 // 125^3 small-strain CG iteration, against the passes of fft_passes.hip that

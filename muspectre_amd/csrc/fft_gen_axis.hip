@@ -84,7 +84,9 @@ bool gen_radices(int n, GenAxis& ax) {
 
 GenShape gen_last_shape(const GenAxis& ax, int nc, int nl, int64_t rows) {
   // pairs of rows per workgroup: more while the grid keeps 1024 workgroups
-  // and the LDS leaves room for four of them per CU
+  // and the LDS leaves room for four of them per CU.  The staging area counted is
+  // that of full fields; packed CG vectors stage two thirds of it (2D: three
+  // quarters) and are launched with as much less LDS, but in the same shape
   GenShape best{};
   const int n = ax.n;
   for (int mult = 1; mult <= 8; ++mult) {

@@ -248,11 +248,12 @@ void force_variant(int pass, int prec, int variant);
 // this length, dimension and precision
 bool fast_variant_valid(int pass, int n, int dim, int prec, int variant);
 
-// general: passes of run-time length where they fit, packed symmetric
-// lines.  Cells of the
-// FP32-refined solve go without: their x carries the FP32 rounding of its
-// inner solves (1.5e-6 relative), so a last-bit change of the FP64 residuals
-// would move their results by that much
+// general: passes of run-time length where they fit, packed symmetric lines in
+// every operator.  Cells of the FP32-refined solve and the served ones have not
+// been moved to them (their FP32 loop keeps the plain schedule on nine
+// components), so they give the bits they always gave.  Nothing in their
+// accuracy asks for it: x carries the FP32 rounding of the inner solves, 1.5e-6
+// relative, far above a last-bit change of any pass
 int plan_init(FftPlan& p, int dim, const int* res, int nc, int prec, bool general = true);
 void plan_free(FftPlan& p);
 
