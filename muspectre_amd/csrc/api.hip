@@ -1460,15 +1460,18 @@ extern "C" int mugpu_material_add_pixels(mugpu_cell c, int mat, int64_t count,
   for (int64_t i = 0; i < count; ++i) {
     m.h_pix.push_back(pixels[i]);
     if (m.family == MUGPU_LE2) {
-      const double* e = params + i * c->nc;
-      for (int k = 0; k < c->nc; ++k) m.h_params.push_back(e[k]);
-      for (int a = 0; a < c->dim; ++a)
-        for (int b = 0; b < a; ++b)
-          if (!(e[a + c->dim * b] == e[b + c->dim * a])) m.major_sym = false;
+      for (int k = 0; k < c->nc; ++k) m.h_params.push_back(params[i * c->nc + k]);
     } else if (m.family == MUGPU_LE3 || m.family == MUGPU_LE4) {
       const double E = params[2 * i], nu = params[2 * i + 1];
       m.h_params.push_back(lame_lambda(E, nu));
       m.h_params.push_back(lame_mu(E, nu));
+    }
+  }
+  if (m.family == MUGPU_LE2) {
+    for (int64_t i = 0; i < count && m.major_sym; ++i) {
+      const double* e = params + i * c->nc;
+      for (int a = 0; a < c->dim; ++a)
+        for (int b = 0; b < a; ++b) m.major_sym = m.major_sym && e[a + c->dim * b] == e[b + c->dim * a];
     }
   }
   return MUGPU_OK;
